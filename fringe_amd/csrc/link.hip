@@ -139,10 +139,16 @@ static void launch_reg32(const SolveArgs& a, hipStream_t s) {
         hipLaunchKernelGGL((solve_reg_kernel<T, Tg, MODE_EVD, 32, false, NC>), dim3(blocks), dim3(64), 0, s, a);
 }
 
-// n <= 64: register-resident solver, two pixels per wave (n <= 32) or one
+// n <= 64: the matrix-core solver (FP32, n <= 32), or the register-resident
+// one with two pixels per wave (n <= 32) or one
 template <typename T, typename Tg>
 static void dispatch_reg(const SolveArgs& a, hipStream_t s) {
-    if (a.n <= 16) {
+    if constexpr (sizeof(T) == 4) {
+        if (a.n <= 32) {
+            launch_solve_mfma(a, s);
+            return;
+        }
+    } else if (a.n <= 16) {
         launch_reg32<T, Tg, 16>(a, s);
     } else if (a.n <= 24) {
         launch_reg32<T, Tg, 24>(a, s);
@@ -152,7 +158,8 @@ static void dispatch_reg(const SolveArgs& a, hipStream_t s) {
         launch_reg32<T, Tg, 30>(a, s);
     } else if (a.n <= 32) {
         launch_reg32<T, Tg, 32>(a, s);
-    } else {
+    }
+    if (a.n > 32) {
         const unsigned blocks = (unsigned)a.slots;
         if (a.module == FRINGE_MODULE_PHASE_LINK)
             hipLaunchKernelGGL((solve_reg_kernel<T, Tg, MODE_EMI, 64, false>), dim3(blocks), dim3(64), 0, s, a);
@@ -416,8 +423,14 @@ template <typename K> static int occupancy_blocks(K kernel, int threads, size_t 
 // One persistent launch over the jobs of pa (all of class cls).  sched: 0
 // = default (one full residency of the kernel, grab 4), else
 // (waves_per_cu << 8 | grab).
+static SolveArgs solve_args_of(const PJob& J, int module, int method);
+
 template <typename T, typename Tg>
 static void launch_persistent(PersistArgs pa, int cls, int mode, int sched, hipStream_t s) {
+    if (cls == 0 && sizeof(T) == 4) {   // the matrix-core solver has grid launches only
+        for (int j = 0; j < pa.njobs; ++j) launch_solve_mfma(solve_args_of(pa.job[j], pa.module, pa.method), s);
+        return;
+    }
     int grab = 4, waves_cu = 0;
     if (sched) {
         waves_cu = sched >> 8;
@@ -460,9 +473,11 @@ static void launch_persistent(PersistArgs pa, int cls, int mode, int sched, hipS
         hipLaunchKernelGGL(k, grid_for(k, 64, 0), dim3(64), 0, s, pa);              \
     } while (0)
         if (cls == 0) {
-            if (mode == 0) FRINGE_PERSIST(MODE_EMI, 32);
-            else if (mode == 2) FRINGE_PERSIST(MODE_MLE, 32);
-            else FRINGE_PERSIST(MODE_EVD, 32);
+            if constexpr (sizeof(T) == 8) {   // FP32: the matrix-core solver above
+                if (mode == 0) FRINGE_PERSIST(MODE_EMI, 32);
+                else if (mode == 2) FRINGE_PERSIST(MODE_MLE, 32);
+                else FRINGE_PERSIST(MODE_EVD, 32);
+            }
         } else {
             if (mode == 0) FRINGE_PERSIST(MODE_EMI, 64);
             else if (mode == 2) FRINGE_PERSIST(MODE_MLE, 64);

@@ -43,6 +43,10 @@ struct SolveArgs {
     // keeps its FP64 coherence there, at the start of each workgroup's area.
     void* awork;
     size_t awork_stride;
+    // matrix-core solver: 1/n, 1/pairs of the temporal coherence, 1/(n - ref)
+    // (set by its launcher)
+    float inv_n;
+    double inv_pairs, inv_comp;
 };
 
 // Certification of an FP32 eigenpair.  The FP32 chain's backward error is
@@ -61,6 +65,9 @@ struct SolveArgs {
 constexpr float kCertScale = 1.0e4f;
 constexpr float kCertThrMargin = 256.0f;
 constexpr double kCertPivotMin = 1.0e-4;
+
+// FP32 solver of the mixed precisions up to 32 dates (solve_mfma.hpp).
+void launch_solve_mfma(const SolveArgs& a, hipStream_t s);
 
 // ---- persistent solve launch over a queue of jobs -------------------------
 // A job is one round segment of one tile: slots [0, slots) of its coherence

@@ -1,7 +1,8 @@
 // solve32.hpp -- register-resident per-pixel estimator for n <= 64 dates.
 //
-// NR = 32 (n <= 32): a wave holds two pixels and lane r of a 32-lane half
-// owns row r of every matrix of its pixel in registers.  NR = 64
+// NR = 32 (n <= 32, FP64 only: solve_mfma.hpp serves FP32): a wave holds two
+// pixels and lane r of a 32-lane half owns row r of every matrix of its
+// pixel in registers.  NR = 64
 // (32 < n <= 64): one pixel per wave, lane r owns row r.  LDS (about 3.5 KB per pixel) is used only
 // to publish one row or one vector to the other lanes, so many waves fit on
 // a CU and the arithmetic is not serialised behind LDS round trips.
@@ -754,9 +755,7 @@ __device__ __forceinline__ void solve_reg_pixel(const SolveArgs& a, LdsR<T, NR>&
 // FP64 Gram into LDS and solves it there, looping over the list.  NC: the
 // columns the tridiagonal reductions process (n <= NC; same results).
 template <typename T, typename Tg, int MODE, int NR, bool LIST, int NC = NR>
-__global__ __launch_bounds__(64)
-__attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && NR == 32 && MODE == MODE_MLE ? 4 : 1)))
-void solve_reg_kernel(SolveArgs a) {
+__global__ __launch_bounds__(64) void solve_reg_kernel(SolveArgs a) {
     __shared__ LdsR<T, NR> sm[64 / NR];
     const int grp = threadIdx.x / NR, r = threadIdx.x % NR;
     LdsR<T, NR>& L = sm[grp];
@@ -795,8 +794,7 @@ void solve_reg_kernel(SolveArgs a) {
 // Persistent launch up to 64 dates: each wave takes units (two pixels for
 // NR = 32, one for NR = 64) of the queued jobs until the queue is drained.
 template <typename T, typename Tg, int MODE, int NR>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && NR == 32 ? 4 : 1)))
-void solve_reg_persistent(PersistArgs pa) {
+__global__ __launch_bounds__(64) void solve_reg_persistent(PersistArgs pa) {
     __shared__ LdsR<T, NR> sm[64 / NR];
     __shared__ int s_u;
     const int total = pa.unit_end[pa.njobs - 1];
