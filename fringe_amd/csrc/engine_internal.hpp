@@ -124,11 +124,11 @@ size_t resolve_generic_lds_bytes(int n, int Nx, int Ny);
 inline size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 // Value of a schedule key (fringe_schedule_set), or fallback when unset.
 int schedule_lookup(int kind, int k0, int k1, int k2, int fallback);
-// FRINGE_SCHED_GENERIC_A when unset: the register-row solver (2) at
-// 33..128 dates (FP32: 33..48 and 65..128), otherwise the one-row-per-lane
-// solver up to 64 dates and the LDS work matrix above (0).
+// FRINGE_SCHED_GENERIC_A when unset: rows in registers (2) at 33..128 dates
+// in both precisions (the other layouts measured 2.9-9 times slower in
+// FP32, 1.2-13 in FP64), otherwise a work matrix (0).
 constexpr int kGenericARowsDefault = 2;
-int generic_a_default(int n, int precision_key);
+int generic_a_default(int n);
 // 33..128 dates under FRINGE_SCHED_GENERIC_A = 2 (either precision; the
 // FP64 re-solve follows the FP64 choice, whose outputs it must equal).
 bool rows_solver_selected(int n, int precision);

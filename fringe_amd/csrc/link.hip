@@ -61,21 +61,20 @@ static void launch_solve_generic(SolveArgs a, hipStream_t s) {
                        a);
 }
 
-// 32 < n <= 128: the register-row solver (FP32 with two threads per row,
-// four up to 48 dates, in the mixed precisions; FP64 with four in the plain
-// path and the re-solve) where the schedule FRINGE_SCHED_GENERIC_A (or its
-// default) selects it;
-// otherwise the one-row-per-lane solver up to 64 dates and a work matrix
+// 32 < n <= 128: the matrix-core solver in the mixed precisions, the
+// register-row solver (four threads per row) in the plain FP64 path and the
+// re-solve, where the schedule FRINGE_SCHED_GENERIC_A (or its default) asks
+// for rows in registers; otherwise the one-row-per-lane solver up to 64 dates and a work matrix
 // above.
 bool rows_solver_selected(int n, int precision) {
     if (n <= 32 || n > kMaxBandsMfma) return false;
     const int pk = precision == FRINGE_PREC_FP64 ? 0 : 1;
-    return schedule_lookup(FRINGE_SCHED_GENERIC_A, n, pk, 0, generic_a_default(n, pk)) == 2;
+    return schedule_lookup(FRINGE_SCHED_GENERIC_A, n, pk, 0, generic_a_default(n)) == 2;
 }
 
 static void launch_rows_solver(const SolveArgs& a, bool fp64, hipStream_t s) {
     if (fp64) launch_rows_solver_f64(a, s);
-    else launch_rows_solver_f32(a, s);
+    else launch_solve_mfma(a, s);
 }
 
 template <typename T, typename Tg>

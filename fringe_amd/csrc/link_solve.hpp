@@ -43,8 +43,8 @@ struct SolveArgs {
     // keeps its FP64 coherence there, at the start of each workgroup's area.
     void* awork;
     size_t awork_stride;
-    // matrix-core solver: 1/n, 1/pairs of the temporal coherence, 1/(n - ref)
-    // (set by its launcher)
+    // matrix-core solvers: 1/n, 1/pairs of the temporal coherence, 1/(n - ref)
+    // (set_solve_counts)
     float inv_n;
     double inv_pairs, inv_comp;
 };
@@ -66,8 +66,29 @@ constexpr float kCertScale = 1.0e4f;
 constexpr float kCertThrMargin = 256.0f;
 constexpr double kCertPivotMin = 1.0e-4;
 
-// FP32 solver of the mixed precisions up to 32 dates (solve_mfma.hpp).
+// FP32 solver of the mixed precisions up to 128 dates (solve_mfma.hpp,
+// solve_mfma_wg.hpp).
 void launch_solve_mfma(const SolveArgs& a, hipStream_t s);
+// FP64 solver up to 128 dates (solve_mfma64.hpp): the plain path, and the
+// re-solve of a pixel list (a.awork / a.awork_stride: the workgroups' areas,
+// at least n^2 complex doubles each, `blocks` of them; a.g64, a.list*: the
+// FP64 Gram and the list).
+void launch_solve_mfma64(const SolveArgs& a, hipStream_t s);
+void launch_resolve_mfma64(const SolveArgs& a, unsigned blocks, hipStream_t s);
+// LDS of the re-solve's workgroup (static chain state plus one FP64 Gram
+// scratch per wave), for the launch checks.
+size_t resolve_mfma64_lds_bytes(int n, int Nx, int Ny);
+// Fills inv_n, inv_pairs and inv_comp.
+inline void set_solve_counts(SolveArgs& a) {
+    long long pairs = (long long)a.n * (a.n - 1) / 2;
+    if (a.module == FRINGE_MODULE_EVD && a.method == FRINGE_METHOD_STBAS) {
+        pairs = 0;
+        for (int i = 0; i < a.n; ++i) pairs += (i + a.bw + 1 < a.n ? i + a.bw + 1 : a.n) - i - 1;
+    }
+    a.inv_n = 1.0f / (float)a.n;
+    a.inv_pairs = 1.0 / (double)pairs;
+    a.inv_comp = 1.0 / (double)(a.n - a.ref);
+}
 
 // ---- persistent solve launch over a queue of jobs -------------------------
 // A job is one round segment of one tile: slots [0, slots) of its coherence

@@ -1,21 +1,11 @@
 // solve_mfma.hip -- launcher of the matrix-core estimator chain (mixed
-// precisions, up to 32 dates).
-#include <algorithm>
-
-#include "solve_mfma.hpp"
+// precisions, up to 128 dates): one wave per pixel up to 32 dates, one
+// workgroup of a wave per 32 dates above.
+#include "solve_mfma_wg.hpp"
 
 namespace fringe {
 
-void launch_solve_mfma(const SolveArgs& args, hipStream_t s) {
-    SolveArgs a = args;
-    long long pairs = (long long)a.n * (a.n - 1) / 2;
-    if (a.module == FRINGE_MODULE_EVD && a.method == FRINGE_METHOD_STBAS) {
-        pairs = 0;
-        for (int i = 0; i < a.n; ++i) pairs += std::min(a.n, i + a.bw + 1) - i - 1;
-    }
-    a.inv_n = 1.0f / (float)a.n;
-    a.inv_pairs = 1.0 / (double)pairs;
-    a.inv_comp = 1.0 / (double)(a.n - a.ref);
+static void launch_wave(const SolveArgs& a, hipStream_t s) {
     constexpr int WPB = 4;
     const dim3 grid((unsigned)((a.slots + WPB - 1) / WPB)), block(64 * WPB);
     if (a.module == FRINGE_MODULE_PHASE_LINK)
@@ -24,6 +14,25 @@ void launch_solve_mfma(const SolveArgs& args, hipStream_t s) {
         hipLaunchKernelGGL((solve_mfma_kernel<MODE_MLE, WPB>), grid, block, 0, s, a);
     else
         hipLaunchKernelGGL((solve_mfma_kernel<MODE_EVD, WPB>), grid, block, 0, s, a);
+}
+
+template <int NT> static void launch_wg(const SolveArgs& a, hipStream_t s) {
+    const dim3 grid((unsigned)a.slots), block(64 * NT);
+    if (a.module == FRINGE_MODULE_PHASE_LINK)
+        hipLaunchKernelGGL((solve_mfma_wg_kernel<MODE_EMI, NT>), grid, block, 0, s, a);
+    else if (a.method == FRINGE_METHOD_MLE)
+        hipLaunchKernelGGL((solve_mfma_wg_kernel<MODE_MLE, NT>), grid, block, 0, s, a);
+    else
+        hipLaunchKernelGGL((solve_mfma_wg_kernel<MODE_EVD, NT>), grid, block, 0, s, a);
+}
+
+void launch_solve_mfma(const SolveArgs& args, hipStream_t s) {
+    SolveArgs a = args;
+    set_solve_counts(a);
+    if (a.n > 96) launch_wg<4>(a, s);
+    else if (a.n > 64) launch_wg<3>(a, s);
+    else if (a.n > 32) launch_wg<2>(a, s);
+    else launch_wave(a, s);
 }
 
 }  // namespace fringe

@@ -43,15 +43,15 @@ namespace fringe {
 typedef float mf32x16 __attribute__((ext_vector_type(16)));
 typedef double mf64x4 __attribute__((ext_vector_type(4)));
 
-// Certification distance of this solver: no eigenvalue may lie within
-// kCertScaleMfma eps |A| / min_t |v_t| of the selected one, as for kCertScale.
-// Its eigenvectors carry smaller errors than the tridiagonalising solvers'
-// (rms against the FP64 path 2-7 times smaller on the same pixels, the
-// constant C of kCertScale's criterion at most 0.4), and |A| is bounded by
-// the eigenvalues' mean and deviation (1.2-1.6 times the norm): a quarter of
-// the scale keeps the phase estimate below 5e-4 rad with C = 1.25, and the
-// certified pixels' errors below the former solver's.
-constexpr float kCertScaleMfma = 2.5e3f;
+// Certification distance of this solver, as kCertScale: no eigenvalue may lie
+// within scale eps |A| / min_t |v_t| of the selected one, with |A| bounded by
+// the eigenvalues' mean and deviation (1.2-1.6 times the norm).  Against the
+// FP64 path, on tiles of 30 to 96 dates whose windows hold few more samples
+// than dates, the phase errors of certified pixels are C eps |A| / (gap
+// min|v|) with C at most 0.07 for H (the former solver: 0.61) and 0.91 for
+// Gamma (the former: 1.4): the scales keep the estimate below 5e-4 rad, half
+// the tolerance, with C = 0.5 and C = 1.25.
+constexpr float kCertScaleEmi = 1.0e3f, kCertScaleEvd = 2.5e3f;
 
 struct LdsMfma32 {
     static constexpr int S = 36;   // row stride of T: 16-byte rows of four, spread over the banks
@@ -84,6 +84,10 @@ __device__ __forceinline__ float both32(float x) {   // x.lo + x.hi in both halv
 // they are instead of being hoisted into (spilled) scalar registers
 __device__ __forceinline__ int fresh(int x) {
     asm volatile("" : "+s"(x));
+    return x;
+}
+__device__ __forceinline__ int fresh_lane(int x) {   // the same for a lane value
+    asm volatile("" : "+v"(x));
     return x;
 }
 // a uniform value as a scalar (control flow and scalar operands)
@@ -170,10 +174,11 @@ struct GammaBuf {
 
 // Gamma in the accumulator layout; rows and columns >= n read as zero
 __device__ __forceinline__ void load_gamma32(const GammaBuf& gam, int n, int col, int h, mf32x16& R, mf32x16& I) {
-    const int o = gam.offset(4 * h, col);
+    int o = fresh_lane(gam.offset(4 * h, col));   // (offsets are not worth registers from one load to the next)
 #pragma unroll
     for (int v = 0; v < 16; ++v) {
-        const cx<float> g = gam.at(o + (8 * (v / 4) + v % 4) * n * 8);
+        const cx<float> g = gam.at(o);
+        o += (v % 4 == 3 ? 5 : 1) * n * 8;
         R[v] = g.re;
         I[v] = g.im;
     }
@@ -183,6 +188,7 @@ struct EigState {
     cx<float> x;     // unit vector, component col
     float theta;     // Rayleigh quotient of B^-1
     float dn, q;     // last step's change and contraction
+    float dq;        // the change that q was measured with
     bool done;
 };
 
@@ -191,16 +197,20 @@ struct EigState {
 // or until the contraction proves worse than kSlow (moving the shift then
 // costs less than going on).
 constexpr float kSlow = 0.35f;
-__device__ __forceinline__ void iterate32(LdsMfma32& L, const mf32x16& R, const mf32x16& I, int col, int h,
+constexpr int kNearInside = 1600000;   // |pivot| >= 0.1
+// qb > 0: polishing instead, until the error predicted from the contraction
+// qb that the spectrum allows is below 4e-7.
+__device__ __forceinline__ void iterate32(LdsMfma32& L, const mf32x16& R, const mf32x16& I, int col, int h, float qb,
                                           EigState& E) {
     float dp = 0.0f;
-    E.done = false;
-    E.q = 1.0f;
-    for (int k = 0; k < 2; ++k) E.x = csub(E.x, apply32(L, R, I, E.x, col, h));
-    const float nr = __builtin_amdgcn_rsqf(uni(red32<OpAdd>(cabs2(E.x))));
-    E.x = cscale(E.x, nr);
-    for (int k = 0; k < 24; ++k) {
+    if (!(qb > 0.0f)) E.q = E.dq = 0.0f;
+    for (int k = qb > 0.0f ? 0 : -2; k < 24; ++k) {
         const cx<float> y = csub(E.x, apply32(L, R, I, E.x, col, h));
+        if (k < 0) {
+            const float nr = k < -1 ? 1.0f : __builtin_amdgcn_rsqf(uni(red32<OpAdd>(cabs2(y))));
+            E.x = cscale(y, nr);
+            continue;
+        }
         const float th = uni(red32<OpAdd>(y.re * E.x.re + y.im * E.x.im));
         const float it = __builtin_amdgcn_rcpf(th);
         const cx<float> d = {fmaf(y.re, it, -E.x.re), fmaf(y.im, it, -E.x.im)};
@@ -210,10 +220,17 @@ __device__ __forceinline__ void iterate32(LdsMfma32& L, const mf32x16& R, const 
         E.x = cx<float>{(E.x.re + d.re) * s, (E.x.im + d.im) * s};
         E.theta = th;
         E.dn = dn;
+        E.done = false;
         if (!(dn < 3.0e38f)) return;   // not finite
+        if (qb > 0.0f) {
+            E.done = dn * qb < 4.0e-7f * (1.0f - qb);
+            if (E.done) return;
+            continue;
+        }
         if (dn < 4.0e-7f) E.done = true;
         if (k > 0) {
             E.q = dn * __builtin_amdgcn_rcpf(dp);
+            E.dq = dn;
             const float q = fminf(E.q, 0.99f);
             if (dn * q < 4.0e-7f * (1.0f - q)) E.done = true;
             if (k > 1 && E.q > kSlow && dn > 2.0e-5f && !E.done) return;
@@ -333,12 +350,11 @@ __device__ __forceinline__ void solve_mfma_pixel(const SolveArgs& a, LdsMfma32& 
                                                  const GammaBuf& gam, long long pix) {
     const int n = a.n, col = lane & 31, h = lane >> 5;
     const bool in = col < n;
-    const int vd = ((col >> 2) & 1) == h ? 4 * (col >> 3) + (col & 3) : -1;   // register of this lane's diagonal entry
+    const int vd0 = ((col >> 2) & 1) == h ? 4 * (col >> 3) + (col & 3) : -1;   // register of this lane's diagonal entry
     const bool stbas = a.method == FRINGE_METHOD_STBAS && MODE == MODE_EVD;
     float code = 0.0f;
     bool unc = false;
     bool inv = MODE != MODE_EVD;   // matrix: H (smallest eigenvalue), else Gamma (largest)
-    mf32x16 R, I;
     EigState E;
     E.x = cx<float>{0.0f, 0.0f};
 
@@ -347,13 +363,14 @@ __device__ __forceinline__ void solve_mfma_pixel(const SolveArgs& a, LdsMfma32& 
         if constexpr (MODE == MODE_MLE) {
             // smallest eigenvalue of Gamma at least 1e-6, by a margin
             // (Gamma has unit diagonal: its norm is at most n)
+            mf32x16 R, I;
             load_gamma32(gam, n, col, h, R, I);
             const float s = 1.0e-6f + kCertThrMargin * Lim<float>::eps() * (float)n;
             float sum = 0.0f;
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
                 sum += fabsf(R[v]) + fabsf(I[v]);
-                if (v == vd) R[v] = -s;   // 1 - s, stored minus 1
+                if (v == vd0) R[v] = -s;   // 1 - s, stored minus 1
             }
             if (!__all(sum < 3.0e38f)) {
                 code = -1.0f;
@@ -402,11 +419,12 @@ __device__ __forceinline__ void solve_mfma_pixel(const SolveArgs& a, LdsMfma32& 
         const float dg = inv ? (in ? L.T[col * LdsMfma32::S + col] : 0.0f) : 1.0f;
         if (!inv) {
             sg = -1.0f;
+            mf32x16 R, I;
             load_gamma32(gam, n, col, h, R, I);
             float f2 = 0.0f, sum = 0.0f;
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
-                if (stbas && abs(8 * (v / 4) + 4 * h + v % 4 - col) > a.bw) {
+                if (stbas && abs(8 * (v / 4) + v % 4 - fresh_lane(col - 4 * h)) > a.bw) {
                     R[v] = 0.0f;
                     I[v] = 0.0f;
                 }
@@ -429,18 +447,20 @@ __device__ __forceinline__ void solve_mfma_pixel(const SolveArgs& a, LdsMfma32& 
                 }
                 // the residual of the last vector but one bounds the distance
                 // to an eigenvalue; the largest lies above the quotient
-                sigma = rho + rho * fmaxf(0.5f * __builtin_amdgcn_sqrtf(dn), 0.02f);
+                sigma = rho + rho * fmaxf(__builtin_amdgcn_sqrtf(dn), 0.02f);
                 const float m2 = sum * a.inv_n - 1.0f;
                 tn = 1.0f + __builtin_amdgcn_sqrtf(fmaxf(m2, 0.0f) * (float)(n - 1));
             }
         }
-        bool certified = false, checking = false;
+        bool certified = false, checking = false, close = false;
         float lam = 0.0f, delta = 0.0f;
         if (code == 0.0f)
-            for (int att = 0; att < 5; ++att) {
+            for (int att = 0; att < 6; ++att) {
+                const int vd = fresh_lane(vd0);
                 // ---- B = +-(A - sigma I), diagonal minus 1 ----
                 const float off = sg * (dg - sigma) - 1.0f;
-                if (inv || att > 0) load_gamma32(gam, n, col, h, R, I);
+                mf32x16 R, I;
+                load_gamma32(gam, n, col, h, R, I);
                 float f2 = 0.0f;
                 if (inv) {
 #pragma unroll
@@ -467,7 +487,7 @@ __device__ __forceinline__ void solve_mfma_pixel(const SolveArgs& a, LdsMfma32& 
                 } else {
 #pragma unroll
                     for (int v = 0; v < 16; ++v) {
-                        const bool out = stbas && abs(8 * (v / 4) + 4 * h + v % 4 - col) > a.bw;
+                        const bool out = stbas && abs(8 * (v / 4) + v % 4 - fresh_lane(col - 4 * h)) > a.bw;
                         R[v] = out ? 0.0f : -R[v];
                         I[v] = out ? 0.0f : -I[v];
                         if (v == vd) R[v] = in ? off : 0.0f;
@@ -485,14 +505,14 @@ __device__ __forceinline__ void solve_mfma_pixel(const SolveArgs& a, LdsMfma32& 
                     else sigma = sigma * 1.15f;
                     continue;
                 }
-                iterate32(L, R, I, col, h, E);
+                iterate32(L, R, I, col, h, 0.0f, E);
                 const float mu = __builtin_amdgcn_rcpf(E.theta);
                 lam = sigma + sg * mu;
                 if (!(fabsf(lam) < 3.0e38f)) break;
                 if (!E.done) {
                     // eigenvalues of B: mu, and the next one at |mu| / q on the
                     // far side; move the shift next to the first
-                    const float q = fminf(fmaxf(E.q, 1.0e-3f), 0.98f);
+                    const float q = E.q > 0.0f ? fminf(fmaxf(E.q, 1.0e-3f), 0.98f) : 0.98f;
                     const float gap = fabsf(mu) / q - mu;
                     const float e = fminf(E.dn * q / (1.0f - q), 1.0f);
                     sigma += sg * (mu - (e * e + 0.15f) * gap);
@@ -500,7 +520,7 @@ __device__ __forceinline__ void solve_mfma_pixel(const SolveArgs& a, LdsMfma32& 
                 }
                 // ---- certification ----
                 const float m2 = red32<OpMin>(in ? cabs2(E.x) : 3.0e38f);
-                delta = kCertScaleMfma * Lim<float>::eps() * tn * __builtin_amdgcn_rsqf(uni(m2));
+                delta = (inv ? kCertScaleEmi : kCertScaleEvd) * Lim<float>::eps() * tn * __builtin_amdgcn_rsqf(uni(m2));
                 if (!(delta <= tn)) break;
                 // Frobenius norm of the inverse: its other eigenvalues'
                 // squares sum to S2, so none of them exceeds sqrt(S2)
@@ -515,11 +535,29 @@ __device__ __forceinline__ void solve_mfma_pixel(const SolveArgs& a, LdsMfma32& 
                 const float s2 = fmaxf(f - E.theta * E.theta, 0.0f) + 4.0e-6f * f;
                 const float t = mu + delta;
                 const bool side = neg == 0 ? E.theta > 0.0f : E.theta < 0.0f;
-                if (side && (t <= 0.0f || s2 * t * t < 1.0f)) {
+                if (!side) break;
+                // the contraction is at most qb: the error left by the last step
+                const float qb = __builtin_amdgcn_sqrtf(s2) * fabsf(mu);
+                bool conv = qb < 0.8f;
+                if (conv && E.dn * qb > 4.0e-7f * (1.0f - qb)) {
+                    iterate32(L, R, I, col, h, qb, E);
+                    conv = E.done;
+                }
+                // a shift inside the spectrum: small pivots would have cost accuracy
+                if (neg != 0 && near < kNearInside && !close) conv = false;
+                if (conv && (t <= 0.0f || s2 * t * t < 1.0f)) {
                     certified = true;
                     break;
                 }
-                if (!side) break;
+                // the next eigenvalue as the measured contraction places it is
+                // too close for any certificate: the FP64 path's pixel
+                if (E.q > 0.02f && E.dq > 4.0e-6f && fabsf(mu) * __builtin_amdgcn_rcpf(E.q) - mu < 0.7f * delta) break;
+                if (!close) {   // once more from a quarter of the distance away
+                    close = true;
+                    sigma = lam - sg * 0.25f * delta;
+                    continue;
+                }
+                if (!conv) break;
                 checking = true;
                 sigma = lam + sg * delta;
             }
@@ -577,6 +615,7 @@ __device__ __forceinline__ void solve_mfma_pixel(const SolveArgs& a, LdsMfma32& 
     wsync();
     float xr[16], xi[16];
     row_values(L, h, xr, xi);
+    mf32x16 R, I;
     load_gamma32(gam, n, col, h, R, I);
     float tr = 0.0f, ti = 0.0f;
     const int rb = stbas ? col - a.bw : 0;

@@ -50,6 +50,25 @@ def test_tile_edges(n, module, method):
     assert res.size < 0.5 * rows * cols
 
 
+@pytest.mark.parametrize("module,method", EST)
+@pytest.mark.parametrize("n", [34, 63, 65, 95, 98, 127])
+def test_workgroup_tile_edges(n, module, method):
+    """33 to 128 dates, a wave per 32: partial last tiles (one, two and 31
+    columns) and a reference date in the last tile."""
+    rows, cols, Nx, Ny = 16, 20, 7, 5
+    print(f"case n={n} {module}/{method}", flush=True)
+    slc = synthetic.stack(n, rows, cols, seed=950 + n, ramp=0.05)
+    wts = synthetic.full_mask(rows, cols, Nx, Ny)
+    bw = n // 4 if method == "STBAS" else -1
+    g, res = _run(slc, wts, Nx, Ny, module, method, ref=n - 1, bw=bw)
+    r = oracle.link(slc, wts, Nx, Ny, module=module, method=method, mini_stack_count=n, bandwidth=bw, want_gap=True)
+    st = compare_link(g, r, r["gap"], stack=slc, ref_index=n - 1)
+    print(st, "re-solved", res.size)
+    assert st["untouched_equal"] and st["codes_equal"]
+    assert st["n_well"] >= (0 if method == "MLE" and module == "evd" else 36)
+    assert st["phase_max"] <= PHASE_TOL and st["tcorr_max"] <= TCORR_TOL and st["comp_err"] <= PHASE_TOL
+
+
 @pytest.mark.parametrize("module,method", EST[:2])
 def test_rank_one_phases(module, method):
     """One phase per date and unit-modulus noise in amplitude only: Gamma =
