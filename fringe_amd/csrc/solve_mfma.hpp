@@ -90,6 +90,19 @@ __device__ __forceinline__ int fresh_lane(int x) {   // the same for a lane valu
     asm volatile("" : "+v"(x));
     return x;
 }
+__device__ __forceinline__ int lane_now() {   // the lane's number, held in no register until here
+    int x;
+    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(x));
+    return x;
+}
+__device__ __forceinline__ float scal(float x) {   // a value alike in all lanes, in a scalar register
+    asm volatile("" : "+v"(x));   // (else the arithmetic is moved behind the read and stays in a vector register)
+    return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(x)));
+}
+__device__ __forceinline__ double lit(double x) {   // a constant, likewise
+    asm volatile("" : "+s"(x));
+    return x;
+}
 // a uniform value as a scalar (control flow and scalar operands)
 __device__ __forceinline__ float uni(float x) { return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(x))); }
 

@@ -12,8 +12,8 @@
 // Bound by the matrix instructions and the vector unit together (65-95 % of
 // the kernel's cycles; the rest is the latency of a pivot's chain).  Solve
 // stage against the register-row and one-row-per-lane solvers it replaced:
-// 48 dates (208 x 224, EMI) 4.8 -> 2.8 ms, 64 dates (131 k pixels, EVD) 15.1
-// -> 3.8 ms, 96 dates (256 x 256, EMI) 37.4 -> 22.5 ms, with the pixels left
+// 48 dates (208 x 224, EMI) 4.8 -> 2.7 ms, 64 dates (131 k pixels, EVD) 15.1
+// -> 3.6 ms, 96 dates (256 x 256, EMI) 37.4 -> 21.0 ms, with the pixels left
 // to the FP64 re-solve down from 10.9 k, 0 and 38.5 k to 1.1 k, 0 and 14.7 k.
 #pragma once
 #include "solve_mfma.hpp"
@@ -41,7 +41,7 @@ template <int NT, bool INV> struct LdsMfmaWg {
 template <int NT, bool INV>
 __device__ __forceinline__ float wg_sum(LdsMfmaWg<NT, INV>& L, int w, int& turn, float x) {
     turn ^= 1;
-    if ((threadIdx.x & 63) == 0) L.red[turn][w][0] = (double)x;
+    if (lane_now() == 0) L.red[turn][w][0] = (double)x;
     __syncthreads();
     float s = 0.0f;
 #pragma unroll
@@ -113,26 +113,29 @@ __device__ __forceinline__ void apply_wg(LdsMfmaWg<NT, INV>& L, const Tiles<NT>&
             L.xi[w][col] = x[J].im;
         }
     wsync();
-    float xr[16], xi[16];
-#pragma unroll
-    for (int a = 0; a < 4; ++a) {
-        const float4 p = *(const float4*)&L.xr[w][8 * a + 4 * h];
-        const float4 q = *(const float4*)&L.xi[w][8 * a + 4 * h];
-        xr[4 * a] = p.x; xr[4 * a + 1] = p.y; xr[4 * a + 2] = p.z; xr[4 * a + 3] = p.w;
-        xi[4 * a] = q.x; xi[4 * a + 1] = q.y; xi[4 * a + 2] = q.z; xi[4 * a + 3] = q.w;
-    }
     turn ^= 1;
+    float re[NT], im[NT];
+#pragma unroll
+    for (int J = 0; J < NT; ++J) re[J] = im[J] = 0.0f;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {   // four rows at a time
+        const float4 p = *(const float4*)&L.xr[w][8 * q + 4 * h];
+        const float4 s = *(const float4*)&L.xi[w][8 * q + 4 * h];
+        const float xr[4] = {p.x, p.y, p.z, p.w}, xi[4] = {s.x, s.y, s.z, s.w};
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+#pragma unroll
+            for (int J = 0; J < NT; ++J) {   // conj(M_rc) x_r
+                const int v = 4 * q + k;
+                re[J] = fmaf(R[J][v], xr[k], re[J]);
+                im[J] = fmaf(R[J][v], xi[k], im[J]);
+                re[J] = fmaf(I[J][v], xi[k], re[J]);
+                im[J] = fmaf(-I[J][v], xr[k], im[J]);
+            }
+    }
 #pragma unroll
     for (int J = 0; J < NT; ++J) {
-        float re[2] = {0.0f, 0.0f}, im[2] = {0.0f, 0.0f};
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-            re[v & 1] = fmaf(R[J][v], xr[v], re[v & 1]);
-            im[v & 1] = fmaf(R[J][v], xi[v], im[v & 1]);
-            re[v & 1] = fmaf(I[J][v], xi[v], re[v & 1]);
-            im[v & 1] = fmaf(-I[J][v], xr[v], im[v & 1]);
-        }
-        const cx<float> s = {both32(re[0] + re[1]), both32(im[0] + im[1])};
+        const cx<float> s = {both32(re[J]), both32(im[J])};
         if (h == 0) L.part[turn][w][32 * J + col] = s;
     }
     __syncthreads();
@@ -181,6 +184,7 @@ template <int NT, bool INV>
 __device__ __forceinline__ void iterate_wg(LdsMfmaWg<NT, INV>& L, const Tiles<NT>& R, const Tiles<NT>& I, int w,
                                            int col, int h, int& turn, float qb, EigStateWg<NT>& E) {
     float dp = 0.0f;
+    const float left = scal(4.0e-7f * (1.0f - qb));
     if (!(qb > 0.0f)) E.q = E.dq = 0.0f;
     cx<float> y[NT];
     for (int k = qb > 0.0f ? 0 : -2; k < 24; ++k) {
@@ -198,7 +202,7 @@ __device__ __forceinline__ void iterate_wg(LdsMfmaWg<NT, INV>& L, const Tiles<NT
         E.done = false;
         if (!(dn < 3.0e38f)) return;   // not finite
         if (qb > 0.0f) {
-            E.done = dn * qb < 4.0e-7f * (1.0f - qb);
+            E.done = dn * qb < left;
             if (E.done) return;
             continue;
         }
@@ -294,29 +298,45 @@ __device__ __forceinline__ bool sweep64_wg(LdsMfmaWg<NT, INV>& L, mf64x4 (&M)[2]
     return ok;
 }
 
+// Above 96 dates a wave's tiles leave few registers: loads of one tile at a
+// time are in flight (all of them at once spilled).
+template <int NT> __device__ __forceinline__ void tile_fence_wg() {
+    if constexpr (NT >= 4) __builtin_amdgcn_sched_barrier(0);
+}
+
+__device__ __forceinline__ void load_tile_wg(const GammaBuf& gam, int n, int w, int J, int col, int h, mf32x16& R,
+                                             mf32x16& I) {
+    int o = fresh_lane(gam.offset(32 * w + 4 * h, 32 * J + col));
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+        const cx<float> g = gam.at(o);
+        o += (v % 4 == 3 ? 5 : 1) * n * 8;
+        R[v] = g.re;
+        I[v] = g.im;
+    }
+}
+
 template <int NT>
 __device__ __forceinline__ void load_gamma_wg(const GammaBuf& gam, int n, int w, int col, int h, Tiles<NT>& R, Tiles<NT>& I) {
 #pragma unroll
     for (int J = 0; J < NT; ++J) {
-        int o = fresh_lane(gam.offset(32 * w + 4 * h, 32 * J + col));
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-            const cx<float> g = gam.at(o);
-            o += (v % 4 == 3 ? 5 : 1) * n * 8;
-            R[J][v] = g.re;
-            I[J][v] = g.im;
-        }
+        load_tile_wg(gam, n, w, J, col, h, R[J], I[J]);
+        tile_fence_wg<NT>();
     }
+}
+
+// Register of tile (w, w)'s diagonal in this lane, or -1.
+__device__ __forceinline__ int diagonal_wg(int col, int h) {
+    return ((col >> 2) & 1) == h ? 4 * (col >> 3) + (col & 3) : -1;
 }
 
 // One pixel on the NT waves of a workgroup.
 template <int MODE, int NT>
 __device__ __forceinline__ void solve_mfma_wg_pixel(const SolveArgs& a, LdsMfmaWg<NT, MODE != MODE_EVD>& L, int w,
-                                                    int lane, int np, const GammaBuf& gam, long long pix) {
+                                                    int np, const GammaBuf& gam, long long pix) {
     constexpr bool INV = MODE != MODE_EVD;
     constexpr int S = LdsMfmaWg<NT, INV>::S;
-    const int n = a.n, col = lane & 31, h = lane >> 5;
-    const int vd0 = ((col >> 2) & 1) == h ? 4 * (col >> 3) + (col & 3) : -1;   // diagonal entry of tile (w, w)
+    const int n = a.n;
     const bool stbas = a.method == FRINGE_METHOD_STBAS && MODE == MODE_EVD;
     float code = 0.0f;
     bool unc = false;
@@ -325,8 +345,12 @@ __device__ __forceinline__ void solve_mfma_wg_pixel(const SolveArgs& a, LdsMfmaW
     EigStateWg<NT> E;
 
     const bool act = np >= 0;
+    // What follows from the lane is computed again in each stage: held over
+    // the sweeps it spilled.
     if (act) {
+        const int lane = lane_now(), col = lane & 31, h = lane >> 5;
         if constexpr (MODE == MODE_MLE) {
+            const int vd0 = diagonal_wg(col, h);
             Tiles<NT> R, I;
             load_gamma_wg<NT>(gam, n, w, col, h, R, I);
             const float s = 1.0e-6f + kCertThrMargin * Lim<float>::eps() * (float)n;
@@ -367,6 +391,7 @@ __device__ __forceinline__ void solve_mfma_wg_pixel(const SolveArgs& a, LdsMfmaW
                             sum += v;
                             M[k][J][r] = (double)v;
                         }
+                    tile_fence_wg<NT>();
                 }
                 sum = wg_sum(L, w, turn, __all(sum < 3.0e38f) ? 0.0f : 1.0f);
                 if (sum > 0.0f) {
@@ -403,6 +428,9 @@ __device__ __forceinline__ void solve_mfma_wg_pixel(const SolveArgs& a, LdsMfmaW
 
     // ---- the eigenpair ----
     if (act && code == 0.0f && !unc) {
+        float sigma = 1.0f, sg = 1.0f, tn = 1.0f;
+        {
+        const int lane = lane_now(), col = lane & 31, h = lane >> 5;
         const float is = __builtin_amdgcn_rsqf((float)n);
 #pragma unroll
         for (int J = 0; J < NT; ++J) {   // start: the phases of the middle column
@@ -413,14 +441,11 @@ __device__ __forceinline__ void solve_mfma_wg_pixel(const SolveArgs& a, LdsMfmaW
             E.x[J] = cx<float>{g.re * s, -g.im * s};
             if (in && !(g2 > 0.0f)) E.x[J].re = is;
         }
-        float sigma = 1.0f, sg = 1.0f, tn = 1.0f;
-        const int own = 32 * w + col;
-        const float dg = inv ? (own < n ? L.T[own * (S + 1)] : 0.0f) : 1.0f;
         if (!inv) {
             sg = -1.0f;
             Tiles<NT> R, I;
             load_gamma_wg<NT>(gam, n, w, col, h, R, I);
-            const int d0 = fresh_lane(col - 4 * h - 32 * w);   // column - row of register 0 of tile 0
+            const int d0 = col - 4 * h - 32 * w;   // column - row of register 0 of tile 0
             float f2 = 0.0f;
 #pragma unroll
             for (int J = 0; J < NT; ++J)
@@ -442,22 +467,27 @@ __device__ __forceinline__ void solve_mfma_wg_pixel(const SolveArgs& a, LdsMfmaW
                     d2 = step_wg<NT>(E, y);
                 }
                 sigma = E.theta + E.theta * fmaxf(__builtin_amdgcn_sqrtf(d2), 0.02f);
-                tn = 1.0f + __builtin_amdgcn_sqrtf(fmaxf(f2 * a.inv_n - 1.0f, 0.0f) * (float)(n - 1));
+                sigma = scal(sigma);
+                tn = scal(1.0f + __builtin_amdgcn_sqrtf(fmaxf(f2 * a.inv_n - 1.0f, 0.0f) * (float)(fresh(n) - 1)));
             }
+        }
         }
         bool certified = false, checking = false, close = false;
         float lam = 0.0f, delta = 0.0f;
         if (code == 0.0f)
             for (int att = 0; att < 6; ++att) {
-                const int vd = fresh_lane(vd0), d0 = fresh_lane(col - 4 * h - 32 * w);
+                const int lane = lane_now(), col = lane & 31, h = lane >> 5;
+                const int vd = diagonal_wg(col, h), d0 = col - 4 * h - 32 * w;
                 // ---- B = +-(A - sigma I), diagonal minus 1 ----
+                const int own = 32 * w + col;
+                const float dg = inv ? (own < n ? L.T[own * (S + 1)] : 0.0f) : 1.0f;
                 const float off = own < n ? sg * (dg - sigma) - 1.0f : 0.0f;
                 Tiles<NT> R, I;
-                load_gamma_wg<NT>(gam, n, w, col, h, R, I);
                 if (inv) {
                     float f2 = 0.0f;
 #pragma unroll
-                    for (int J = 0; J < NT; ++J)
+                    for (int J = 0; J < NT; ++J) {
+                        load_tile_wg(gam, n, w, J, col, h, R[J], I[J]);
 #pragma unroll
                         for (int q = 0; q < 4; ++q) {
                             const float4 m = *(const float4*)&L.T[(32 * J + col) * S + 32 * w + 8 * q + 4 * h];
@@ -471,6 +501,8 @@ __device__ __forceinline__ void solve_mfma_wg_pixel(const SolveArgs& a, LdsMfmaW
                                 if (J == w && v == vd) R[J][v] = off;
                             }
                         }
+                        tile_fence_wg<NT>();
+                    }
                     if (att == 0) {   // |H| <= m + s sqrt(n - 1), as in solve_mfma_pixel
                         float tr = 0.0f;
 #pragma unroll
@@ -478,12 +510,13 @@ __device__ __forceinline__ void solve_mfma_wg_pixel(const SolveArgs& a, LdsMfmaW
                             if (32 * J + col < n) tr += L.T[(32 * J + col) * (S + 1)];
                         tr = uni(red32<OpAdd>(tr)) * a.inv_n;
                         const float ff = wg_sum(L, w, turn, uni(both32(red32<OpAdd>(f2)))) * a.inv_n;
-                        tn = tr + __builtin_amdgcn_sqrtf(fmaxf(ff - tr * tr, 0.0f) * (float)(n - 1));
+                        tn = scal(tr + __builtin_amdgcn_sqrtf(fmaxf(ff - tr * tr, 0.0f) * (float)(fresh(n) - 1)));
                         if (!(tn < 3.0e38f)) break;
                     }
                 } else {
 #pragma unroll
-                    for (int J = 0; J < NT; ++J)
+                    for (int J = 0; J < NT; ++J) {
+                        load_tile_wg(gam, n, w, J, col, h, R[J], I[J]);
 #pragma unroll
                         for (int v = 0; v < 16; ++v) {
                             const bool out = stbas && abs(8 * (v / 4) + v % 4 - d0 - 32 * J) > a.bw;
@@ -491,6 +524,8 @@ __device__ __forceinline__ void solve_mfma_wg_pixel(const SolveArgs& a, LdsMfmaW
                             I[J][v] = out ? 0.0f : -I[J][v];
                             if (J == w && v == vd) R[J][v] = off;
                         }
+                        tile_fence_wg<NT>();
+                    }
                 }
                 int neg, near;
                 sweep_wg<NT, INV>(L, R, I, n, w, lane, neg, near);
@@ -504,14 +539,14 @@ __device__ __forceinline__ void solve_mfma_wg_pixel(const SolveArgs& a, LdsMfmaW
                     continue;
                 }
                 iterate_wg<NT, INV>(L, R, I, w, col, h, turn, 0.0f, E);
-                const float mu = __builtin_amdgcn_rcpf(E.theta);
-                lam = sigma + sg * mu;
+                const float mu = scal(__builtin_amdgcn_rcpf(E.theta));
+                lam = scal(sigma + sg * mu);
                 if (!(fabsf(lam) < 3.0e38f)) break;
                 if (!E.done) {
                     const float q = E.q > 0.0f ? fminf(fmaxf(E.q, 1.0e-3f), 0.98f) : 0.98f;
                     const float gap = fabsf(mu) / q - mu;
                     const float e = fminf(E.dn * q / (1.0f - q), 1.0f);
-                    sigma += sg * (mu - (e * e + 0.15f) * gap);
+                    sigma = scal(sigma + sg * (mu - (e * e + 0.15f) * gap));
                     continue;
                 }
                 // ---- certification ----
@@ -519,7 +554,8 @@ __device__ __forceinline__ void solve_mfma_wg_pixel(const SolveArgs& a, LdsMfmaW
 #pragma unroll
                 for (int J = 0; J < NT; ++J)
                     if (32 * J + col < n) m2 = fminf(m2, cabs2(E.x[J]));
-                delta = (inv ? kCertScaleEmi : kCertScaleEvd) * Lim<float>::eps() * tn * __builtin_amdgcn_rsqf(uni(red32<OpMin>(m2)));
+                delta = scal((inv ? kCertScaleEmi : kCertScaleEvd) * Lim<float>::eps() *
+                             (tn * __builtin_amdgcn_rsqf(uni(red32<OpMin>(m2)))));
                 if (!(delta <= tn)) break;
                 float f = 0.0f;
 #pragma unroll
@@ -531,12 +567,11 @@ __device__ __forceinline__ void solve_mfma_wg_pixel(const SolveArgs& a, LdsMfmaW
                     }
                 if (vd >= 0 && own >= n) f -= 1.0f;   // padding: R = 0 on the diagonal
                 f = wg_sum(L, w, turn, uni(both32(red32<OpAdd>(f))));
-                const float s2 = fmaxf(f - E.theta * E.theta, 0.0f) + 4.0e-6f * f;
-                const float t = mu + delta;
+                const float s2 = scal(fmaxf(f - E.theta * E.theta, 0.0f) + 4.0e-6f * f), t = scal(mu + delta);
                 const bool side = neg == 0 ? E.theta > 0.0f : E.theta < 0.0f;
                 if (!side) break;
                 // the contraction is at most qb: the error left by the last step
-                const float qb = __builtin_amdgcn_sqrtf(s2) * fabsf(mu);
+                const float qb = scal(__builtin_amdgcn_sqrtf(s2) * fabsf(mu));
                 bool conv = qb < 0.8f;
                 if (conv && E.dn * qb > 4.0e-7f * (1.0f - qb)) {
                     iterate_wg<NT, INV>(L, R, I, w, col, h, turn, qb, E);
@@ -553,7 +588,7 @@ __device__ __forceinline__ void solve_mfma_wg_pixel(const SolveArgs& a, LdsMfmaW
                 if (E.q > 0.02f && E.dq > 4.0e-6f && fabsf(mu) * __builtin_amdgcn_rcpf(E.q) - mu < 0.7f * delta) break;
                 if (!close) {   // once more from a quarter of the distance away
                     close = true;
-                    sigma = lam - sg * 0.25f * delta;
+                    sigma = lam - sg * (0.25f * delta);
                     continue;
                 }
                 if (!conv) break;
@@ -564,6 +599,7 @@ __device__ __forceinline__ void solve_mfma_wg_pixel(const SolveArgs& a, LdsMfmaW
         unc = code == 0.0f && (unc || !certified);
     }
 
+    const int lane = lane_now(), col = lane & 31, h = lane >> 5;
     if (act && unc) {   // the FP64 re-solve writes every output of the pixel
         if (w == 0 && lane == 0) {
             const int e = atomicAdd(a.cert_count, 1);
@@ -698,17 +734,18 @@ __device__ __forceinline__ void solve_mfma_wg_pixel(const SolveArgs& a, LdsMfmaW
     }
 }
 
-// Waves per SIMD: 128 registers (four) spill in EMI at NT = 2 (three measured
-// 6 % faster on 48 dates), and EVD takes four (7 % faster than three on 64);
-// at NT = 3 three with a few spills beat two without (9 % on 96 dates).
+// Waves per SIMD, as many as leave no register spilled (a spill under a
+// partial exec mask has lost the other lanes' values).  Solve stage with one
+// fewer: 64 dates EVD 3.6 -> 4.1 ms, 96 dates EMI 21.0 -> 24.7 ms.
+constexpr int waves_wg(int mode, int nt) { return nt == 2 ? (mode == MODE_EVD ? 4 : 3) : nt == 3 && mode != MODE_MLE ? 3 : 2; }
 template <int MODE, int NT>
-__global__ __launch_bounds__(64 * NT) __attribute__((amdgpu_waves_per_eu(NT == 2 ? (MODE == MODE_EVD ? 4 : 3) : NT == 3 ? 3 : 2))) void solve_mfma_wg_kernel(SolveArgs a) {
+__global__ __launch_bounds__(64 * NT) __attribute__((amdgpu_waves_per_eu(waves_wg(MODE, NT)))) void solve_mfma_wg_kernel(SolveArgs a) {
     __shared__ LdsMfmaWg<NT, MODE != MODE_EVD> L;
-    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int slot = a.slots - 1 - (int)blockIdx.x;
     const int np = a.npix[slot];
     const cx<float>* gam = (const cx<float>*)a.gamma + (size_t)slot * a.n * a.n;
-    solve_mfma_wg_pixel<MODE, NT>(a, L, w, lane, np, GammaBuf(gam, a.n), a.first + slot);
+    solve_mfma_wg_pixel<MODE, NT>(a, L, w, np, GammaBuf(gam, a.n), a.first + slot);
 }
 
 }  // namespace fringe
