@@ -175,8 +175,8 @@ int link_check(const fringe_link_tile* t) {
     const size_t lds = (size_t)device_lds_limit();
     if (t->nbands <= 64) {
         if (link_certifies(t->nbands, t->precision) &&
-            (rows_solver_selected(t->nbands, FRINGE_PREC_FP64) ? resolve_rows_lds_bytes(t->nbands, t->Nx, t->Ny)
-                                                               : resolve_lds_bytes(t->nbands, t->Nx, t->Ny)) > lds)
+            (matrix_solver_selected(t->nbands, FRINGE_PREC_FP64) ? resolve_mfma64_lds_bytes(t->nbands, t->Nx, t->Ny)
+                                                                 : resolve_lanes_lds_bytes(t->nbands, t->Nx, t->Ny)) > lds)
             return FRINGE_ERR_UNSUPPORTED;
     } else {
         const size_t rest = (t->precision == FRINGE_PREC_FP64 ? solve_group_bytes<double>(t->nbands, false)
@@ -184,8 +184,8 @@ int link_check(const fringe_link_tile* t) {
                             solve_static_lds(t->precision);
         if (rest > lds) return FRINGE_ERR_UNSUPPORTED;
         if (link_certifies(t->nbands, t->precision)) {
-            const size_t r = rows_solver_selected(t->nbands, FRINGE_PREC_FP64)
-                                 ? resolve_rows_lds_bytes(t->nbands, t->Nx, t->Ny)
+            const size_t r = matrix_solver_selected(t->nbands, FRINGE_PREC_FP64)
+                                 ? resolve_mfma64_lds_bytes(t->nbands, t->Nx, t->Ny)
                                  : resolve_generic_lds_bytes(t->nbands, t->Nx, t->Ny);
             if (r > lds) return FRINGE_ERR_UNSUPPORTED;
         }
@@ -212,7 +212,7 @@ static int link_chunk_pixels(const fringe_link_tile* t) {
 
 struct LinkLayout {
     size_t gamma, npix, pack, cert, queue, awork, awork_stride, rwork, total;
-    int resolve_blocks;
+    int resolve_areas;
 };
 
 static LinkLayout link_layout(const fringe_link_tile* t, int chunk, size_t area_budget) {
@@ -240,11 +240,11 @@ static LinkLayout link_layout(const fringe_link_tile* t, int chunk, size_t area_
     L.rwork = b;   // the FP64 re-solve's per-workgroup areas
     if (link_certifies(n, t->precision)) {
         if (n > 64) {
-            L.resolve_blocks = resolve_generic_blocks(resolve_generic_area_bytes(n), area_budget);
-            b += (size_t)L.resolve_blocks * resolve_generic_area_bytes(n);
+            L.resolve_areas = resolve_generic_blocks(resolve_generic_area_bytes(n), area_budget);
+            b += (size_t)L.resolve_areas * resolve_generic_area_bytes(n);
         } else {
-            L.resolve_blocks = resolve_small_blocks(n, area_budget);
-            b += (size_t)L.resolve_blocks * (n <= 32 ? 2 : 1) * resolve_small_area_bytes(n);
+            L.resolve_areas = resolve_small_areas(n, area_budget);
+            b += (size_t)L.resolve_areas * resolve_small_area_bytes(n);
         }
     }
     L.total = b;
@@ -311,7 +311,7 @@ int link_run_chunked(const fringe_link_tile* t, const void* d_slc, const uint32_
     }
     if (link_certifies(P.n, P.precision)) {
         P.d_rwork = (char*)d_work + LL.rwork;
-        P.resolve_blocks = LL.resolve_blocks;
+        P.resolve_areas = LL.resolve_areas;
     }
     P.d_queue = (int*)((char*)d_work + LL.queue);
     hipStream_t s = (hipStream_t)stream;
@@ -404,8 +404,8 @@ static BatchLayout batch_layout(const fringe_link_batch_item* items, int count) 
         if (link_certifies(n, t->precision))
             max_rwork = std::max(max_rwork, n > 64 ? (size_t)resolve_generic_blocks(resolve_generic_area_bytes(n)) *
                                                          resolve_generic_area_bytes(n)
-                                                   : (size_t)resolve_small_blocks(n, kResolveAreaBudget) *
-                                                         (n <= 32 ? 2 : 1) * resolve_small_area_bytes(n));
+                                                   : (size_t)resolve_small_areas(n, kResolveAreaBudget) *
+                                                         resolve_small_area_bytes(n));
     }
     L.round = b;
     L.round_bytes = std::max(std::min(need, (size_t)2048 << 20), max_row);

@@ -72,7 +72,7 @@ struct LinkPlan {
     void* d_awork;
     size_t awork_stride;
     void* d_rwork;
-    int resolve_blocks;  // workgroups (and areas at d_rwork) of that re-solve; 0 = resolve_generic_blocks
+    int resolve_areas;  // areas at d_rwork, one per workgroup of that re-solve; 0 = the default number
     int* d_queue;       // work queue counter of a persistent solve launch
 };
 
@@ -102,17 +102,17 @@ int link_batch_launch(const BatchPlan& B, hipStream_t s);
 // group (its coherence plus the FP64 Gram's scratch), and the whole
 // workgroup's LDS including the solver's static part.
 size_t resolve_group_bytes(int n, int Nx, int Ny);
-// Re-solve up to 64 dates: one lane group's coherence area in the workspace,
-// and the workgroups that a quarter of `budget` of such areas allows
-// (16..1024; two groups per workgroup up to 32 dates).
+// Re-solve up to 64 dates: one workgroup's coherence area in the workspace,
+// and as many of them as a quarter of `budget` allows (16..1024; 32..2048 up
+// to 32 dates).
 size_t resolve_small_area_bytes(int n);
-int resolve_small_blocks(int n, size_t budget);
+int resolve_small_areas(int n, size_t budget);
 // Column block of that re-solve's FP64 Gram: each coherence entry sums the
 // same products in the same order whatever the block (bit-identical to the
 // plain path's 32); 8 keeps the accumulators, and the kernel, within the
 // plain FP64 solver's registers.
 constexpr int kResolveSmallCB = 8;
-size_t resolve_lds_bytes(int n, int Nx, int Ny);
+size_t resolve_lanes_lds_bytes(int n, int Nx, int Ny);
 // Whether a tile of this precision and date count certifies its FP32 results.
 bool link_certifies(int n, int precision);
 int device_lds_limit();
@@ -129,10 +129,16 @@ int schedule_lookup(int kind, int k0, int k1, int k2, int fallback);
 // FP32, 1.2-13 in FP64), otherwise a work matrix (0).
 constexpr int kGenericARowsDefault = 2;
 int generic_a_default(int n);
-// 33..128 dates under FRINGE_SCHED_GENERIC_A = 2 (either precision; the
-// FP64 re-solve follows the FP64 choice, whose outputs it must equal).
-bool rows_solver_selected(int n, int precision);
-size_t resolve_rows_lds_bytes(int n, int Nx, int Ny);
+// Up to 32 dates, and 33..128 under FRINGE_SCHED_GENERIC_A = 2: the
+// matrix-core solvers (the FP64 re-solve follows the FP64 choice, whose
+// outputs it must equal).
+bool matrix_solver_selected(int n, int precision);
+// LDS of the matrix-core re-solve's workgroup.
+size_t resolve_mfma64_lds_bytes(int n, int Nx, int Ny);
+// The FP64 re-solve of a tile's list, and a counter's reset.
+void resolve_tile(const LinkPlan& P, const float2* slc, const uint32_t* wts, float2* phase, float* tcorr, float2* comp,
+                  hipStream_t s);
+void clear_counter(int* p, hipStream_t s);
 // Estimator index of the solver schedules: 0 phase_link EMI, 1 evd EVD/STBAS, 2 evd MLE.
 inline int solve_mode_index(int module, int method) {
     return module == FRINGE_MODULE_PHASE_LINK ? 0 : (method == FRINGE_METHOD_MLE ? 2 : 1);

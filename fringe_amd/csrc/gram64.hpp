@@ -30,8 +30,7 @@ struct GramArgs {
 
 template <int G>
 __device__ inline int build_position_list(const uint32_t* w, bool cen, int r0, int c0, int rows,
-                                          int cols, int Nx, int Ny, int* list) {
-    const int g = threadIdx.x % G;
+                                          int cols, int Nx, int Ny, int g, int* list) {
     const int Wx = 2 * Nx + 1, Wn = (2 * Ny + 1) * Wx;
     int cnt = 0;
     for (int b0 = 0; b0 < Wn; b0 += G) {
@@ -102,7 +101,7 @@ __device__ __forceinline__ int gram_f64_pixel(const GramArgs& a, bool valid, lon
     const int r0 = (int)(pix / a.cols), c0 = (int)(pix % a.cols);
     const uint32_t* w = a.wts + pix * a.nul;
     const bool cen = valid && shp_get(w, shp_flat(0, 0, a.Nx, a.Ny));
-    const int cnt = build_position_list<G>(w, cen, r0, c0, a.rows, a.cols, a.Nx, a.Ny, list);
+    const int cnt = build_position_list<G>(w, cen, r0, c0, a.rows, a.cols, a.Nx, a.Ny, threadIdx.x % G, list);
     const bool go = cen && cnt >= a.min_nb;
     const int K = go ? cnt : 0;
     int Kw = K;

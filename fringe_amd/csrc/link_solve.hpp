@@ -74,10 +74,10 @@ void launch_solve_mfma(const SolveArgs& a, hipStream_t s);
 // at least n^2 complex doubles each, `blocks` of them; a.g64, a.list*: the
 // FP64 Gram and the list).
 void launch_solve_mfma64(const SolveArgs& a, hipStream_t s);
+void launch_gram_mfma64(const GramArgs& a, hipStream_t s);
 void launch_resolve_mfma64(const SolveArgs& a, unsigned blocks, hipStream_t s);
-// LDS of the re-solve's workgroup (static chain state plus one FP64 Gram
-// scratch per wave), for the launch checks.
-size_t resolve_mfma64_lds_bytes(int n, int Nx, int Ny);
+// The solver of a.n dates at this precision (solvers.hip), as one grid.
+void launch_solve(const SolveArgs& a, int precision, hipStream_t s);
 // Fills inv_n, inv_pairs and inv_comp.
 inline void set_solve_counts(SolveArgs& a) {
     long long pairs = (long long)a.n * (a.n - 1) / 2;
@@ -119,6 +119,10 @@ struct PersistArgs {
     int unit_end[kMaxJobs];     // prefix sums of the jobs' units
     PJob job[kMaxJobs];
 };
+
+// One persistent launch over the jobs of pa, all of date class cls (link.hip)
+// on a vector-unit solver; sched as FRINGE_SCHED_SOLVE.
+void launch_persistent_any(const PersistArgs& pa, int cls, int mode, int precision, int sched, hipStream_t s);
 
 template <typename T> struct Lim;
 template <> struct Lim<float> {

@@ -69,6 +69,27 @@ def test_workgroup_tile_edges(n, module, method):
     assert st["phase_max"] <= PHASE_TOL and st["tcorr_max"] <= TCORR_TOL and st["comp_err"] <= PHASE_TOL
 
 
+@pytest.mark.parametrize("module,method", EST)
+@pytest.mark.parametrize("n", [2, 15, 16, 17, 33, 49, 80, 81, 113, 128])
+def test_fp64_wave_edges(n, module, method):
+    """The FP64 Gram and chain, a wave per 16 dates: first and last sizes of a
+    number of waves, odd and even; a window cut at every border."""
+    if n == 2 and method == "STBAS":
+        pytest.skip("two dates have no band narrower than the matrix: refused")
+    rows, cols, Nx, Ny = 12, 16, 7, 5
+    print(f"case fp64 n={n} {module}/{method}", flush=True)
+    slc = synthetic.stack(n, rows, cols, seed=1000 + n, ramp=0.05)
+    wts = synthetic.full_mask(rows, cols, Nx, Ny)
+    bw = max(1, n // 4) if method == "STBAS" else -1
+    g, _ = _run(slc, wts, Nx, Ny, module, method, ref=n // 3, bw=bw, precision="fp64")
+    r = oracle.link(slc, wts, Nx, Ny, module=module, method=method, mini_stack_count=n // 3 + 1, bandwidth=bw,
+                    want_gap=True)
+    st = compare_link(g, r, r["gap"], stack=slc, ref_index=n // 3)
+    print(st)
+    assert st["untouched_equal"] and st["codes_equal"]
+    assert st["phase_max"] <= PHASE_TOL and st["tcorr_max"] <= TCORR_TOL and st["comp_err"] <= PHASE_TOL
+
+
 @pytest.mark.parametrize("module,method", EST[:2])
 def test_rank_one_phases(module, method):
     """One phase per date and unit-modulus noise in amplitude only: Gamma =
