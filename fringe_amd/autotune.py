@@ -11,10 +11,10 @@ stage's launches), and keeps the fastest:
 * Solver launch, per (date class, estimator, precision): one wave per unit,
   or a persistent grid of W waves per compute unit taking G units at a time
   from the work queue.
-* Above 32 dates, per (date class, precision): each row in registers (up to
-  128 dates; two or, up to 48 dates, four threads per row in FP32, four in
-  FP64), or one row per lane (up to 64 dates), or the solver's work matrix
-  in LDS (where it fits) or in global memory (above 64 dates).
+* Above 32 dates, per (date class, precision): the matrix in registers,
+  on the matrix cores (up to 128 dates), or one row per lane (up to 64
+  dates; in FP32 up to 48), or the solver's work matrix in LDS (where it
+  fits) or in global memory (above 64 dates).
 
 The chosen table (with every candidate's time) is written as JSON; the
 library installs it when it is loaded (fringe_amd._lib.load_schedules).
@@ -110,7 +110,7 @@ def tune(quick=False, log=sys.stderr):
             slc, w = slc[:, :16].contiguous(), w[:16].contiguous()
         key = (n, mode, 0 if prec == "fp64" else 1)
         # the launch schedule serves the one-row-per-lane solver and the
-        # solver with a work matrix, not the register rows
+        # solver with a work matrix, not the matrix cores
         ga_default = L.fringe_schedule_get(_lib.FRINGE_SCHED_GENERIC_A, n, key[2], 0)
         if n > 32:
             L.fringe_schedule_set(_lib.FRINGE_SCHED_GENERIC_A, n, key[2], 0, 0)

@@ -124,13 +124,13 @@ size_t resolve_generic_lds_bytes(int n, int Nx, int Ny);
 inline size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 // Value of a schedule key (fringe_schedule_set), or fallback when unset.
 int schedule_lookup(int kind, int k0, int k1, int k2, int fallback);
-// FRINGE_SCHED_GENERIC_A when unset: rows in registers (2) at 33..128 dates
-// in both precisions (the other layouts measured 2.9-9 times slower in
-// FP32, 1.2-13 in FP64), otherwise a work matrix (0).
+// FRINGE_SCHED_GENERIC_A when unset: the matrix cores (2) at 33..128 dates in
+// both precisions (the other layouts measured 4 and more times slower),
+// reported as 0 for FP32 at 49..64; otherwise a work matrix (0).
 constexpr int kGenericARowsDefault = 2;
-int generic_a_default(int n);
-// Up to 32 dates, and 33..128 under FRINGE_SCHED_GENERIC_A = 2: the
-// matrix-core solvers (the FP64 re-solve follows the FP64 choice, whose
+int generic_a_default(int n, int precision);
+// Up to 32 dates, and 33..128 under FRINGE_SCHED_GENERIC_A = 2 (in FP32 at
+// 49..64 always): the matrix-core solvers (the FP64 re-solve follows the FP64 choice, whose
 // outputs it must equal).
 bool matrix_solver_selected(int n, int precision);
 // LDS of the matrix-core re-solve's workgroup.

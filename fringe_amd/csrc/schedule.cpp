@@ -39,7 +39,9 @@ std::tuple<int, int, int, int> key_of(int kind, int k0, int k1, int k2) {
 
 }  // namespace
 
-int generic_a_default(int n) { return n > 32 && n <= 128 ? kGenericARowsDefault : 0; }
+int generic_a_default(int n, int precision) {
+    return n > 32 && n <= 128 && !(precision == 1 && n > 48 && n <= 64) ? kGenericARowsDefault : 0;
+}
 
 int schedule_lookup(int kind, int k0, int k1, int k2, int fallback) {
     std::lock_guard<std::mutex> lk(g_mu);
@@ -76,7 +78,7 @@ int fringe_schedule_set(int kind, int key0, int key1, int key2, int value) {
 
 int fringe_schedule_get(int kind, int key0, int key1, int key2) {
     if (kind != FRINGE_SCHED_GRAM_VARIANT && kind != FRINGE_SCHED_SOLVE && kind != FRINGE_SCHED_GENERIC_A) return -1;
-    if (kind == FRINGE_SCHED_GENERIC_A) return schedule_lookup(kind, key0, key1, key2, generic_a_default(key0));
+    if (kind == FRINGE_SCHED_GENERIC_A) return schedule_lookup(kind, key0, key1, key2, generic_a_default(key0, key1));
     return schedule_lookup(kind, key0, key1, key2, kind == FRINGE_SCHED_SOLVE ? 0 : FRINGE_GRAM_DEFAULT);
 }
 

@@ -167,9 +167,8 @@ long long fringe_link_resolved_pixels(const fringe_link_tile* t, const void* d_w
  * matrices of several tiles share each round's buffer, and every round's
  * Hermitian solves of one date class (<= 32, <= 64, <= 128, > 128 dates) run
  * in ONE persistent launch that drains a queue of all tiles' pixels, whatever
- * their date count and neighbour count (tiles on the register-row solvers,
- * 33..128 dates, and the mixed precisions' tiles up to 32 dates get one grid
- * launch each).  Outputs
+ * their date count and neighbour count (tiles on the matrix-core solvers, up
+ * to 128 dates by default, get one grid launch each).  Outputs
  * equal fringe_link_run's per tile
  * bit for bit.  Returns 202 for a batch that mixes modules, methods or
  * precisions. */
@@ -193,13 +192,14 @@ int fringe_link_batch_run(const fringe_link_batch_item* items, int count, void* 
  * estimator: 0 phase_link EMI, 1 evd EVD/STBAS, 2 evd MLE, precision): 0
  * launches one wave per unit of work, else (waves_per_cu << 8 | grab) runs a
  * persistent grid of waves_per_cu waves per compute unit that take `grab`
- * units at a time from a queue (up to 32 dates the mixed precisions' solver
- * always runs as a grid).  Unset keys keep the built-in defaults. */
+ * units at a time from a queue (the matrix-core solvers, which serve up to 128
+ * dates by default, always run as a grid).  Unset keys keep the built-in defaults. */
 #define FRINGE_SCHED_GRAM_VARIANT 0
 #define FRINGE_SCHED_SOLVE 1
 #define FRINGE_SCHED_GENERIC_A 2    /* (nbands class 48/64/96/128/256, precision): the solver above 32 dates
-                                       keeps each row in registers, on the matrix cores in FP32, four threads
-                                       per row in FP64 (2, up to 128 dates; the default there);
+                                       keeps the matrix in registers, on the matrix cores (2, up to 128
+                                       dates; the default there, reported as 0 for FP32 at 49..64 dates,
+                                       where 0 selects it too);
                                        otherwise one row per lane up to 64 dates (0), or its work matrix in LDS
                                        (0) or global memory (1) above 64 dates */
 #define FRINGE_GRAM_DEFAULT 0
