@@ -6,8 +6,8 @@ For every key of the schedule table it times each candidate on a resident
 synthetic tile, with the engine's own stage timers (HIP events around the
 stage's launches), and keeps the fastest:
 
-* Gram variant, per (date class, window): the staged MFMA kernel on 12, 8
-  or 4 waves (8 x 16, 4 x 16 or up to 4 x 8 pixel tiles), or the unstaged one.
+* Gram variant, per (date class, window): the staged MFMA kernel on
+  pixel tiles of up to 8 x 16, 4 x 16 or 4 x 8, or the unstaged one.
 * Solver launch, per (date class, estimator, precision): one wave per unit,
   or a persistent grid of W waves per compute unit taking G units at a time
   from the work queue.

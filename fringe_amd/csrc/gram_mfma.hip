@@ -22,7 +22,9 @@
 //               position-major packed words pk[pixel][re_0, im_0, re_1,
 //               im_1, ...] with (hi | lo << 16); one extra all-zero record at
 //               index rows*cols pads neighbour lists.
-//   gram_mfma : one wave per pixel at a time.  The wave compacts the mask
+//   gram_mfma_lds (up to 64 dates) : the records a pixel tile's windows share
+//               are staged in LDS; one wave per pixel at a time.
+//   gram_mfma : where no tile fits LDS; one wave per pixel at a time.  The wave compacts the mask
 //               into a list of pixel indices (padded to a multiple of 16) in
 //               LDS; per 16 positions lane l gathers component (l % 32) of 8
 //               positions for every 32-wide component block -- lanes 0..31
@@ -31,8 +33,7 @@
 //               block triangle of P is folded into Gamma (the transposed
 //               cross block goes through a per-wave LDS scratch) and written.
 //               Above 32 dates (gram_mfma_pairs) the wave walks the pairs of
-//               32-date blocks one at a time instead of holding every block
-//               (at 33-64 dates 9-14 % faster than gram_mfma holding both).
+//               32-date blocks one at a time instead of holding every block.
 #include <algorithm>
 
 #include "device_common.hpp"
@@ -346,7 +347,7 @@ __global__ __launch_bounds__(64 * WAVES) void gram_mfma(MfmaArgs a) {
     }
 }
 
-// 64 < n <= 128: the wave of a pixel walks the date-block pairs (I, J),
+// 64 < n <= 128, and 33..64 where nothing can be staged: the wave of a pixel walks the date-block pairs (I, J),
 // I <= J < nb = ceil(n / 32), diagonal pairs first.  Per pair it keeps the
 // four 32 x 32 real products P(re_I, re_J), P(im_I, im_J), P(re_I, im_J),
 // P(im_I, re_J) (64 accumulator registers whatever n; 12 MFMAs per 16
@@ -498,79 +499,132 @@ __global__ __launch_bounds__(64 * WAVES) void gram_mfma_pairs(MfmaArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// n <= 32: the records of the union of a workgroup's windows are staged in
-// LDS once, and the waves take their pixels' neighbour lists from there.
+// Up to 64 dates: the records of the union of a workgroup's windows are staged
+// in LDS once, and the waves take their pixels' neighbour lists from there.
 // A TH x TW pixel tile needs (TH + 2Ny) x (TW + 2Nx) positions: for 4 x 8
 // pixels and a 15 x 11 window that is 308 records for 32 pixels, against
-// 165 per pixel gathered one by one.  All four real 32 x 32 tiles
-// P(re,re), P(im,im), P(re,im), P(im,re) are accumulated, so the fold needs
-// no transpose: Re G = RR + II, Im G(i,j) = P(im_i,re_j) - P(re_i,im_j).
+// 165 per pixel gathered one by one.
+//
+// Dates are padded to NB blocks of 16, products are v_mfma_f32_16x16x32 (32
+// positions each; lane l holds date l % 16 and eight positions).  With the
+// samples' halves h + l of re (R) and im (I), a diagonal block pair needs
+//   A = Rh Rh' + Ih Ih',  X = Rh Rl' + Ih Il',  W = Ih Rh' + Ih Rl' + Il Rh':
+//   Re G = A + X + X',  Im G = W - W',
+// seven MFMAs instead of the twelve that the four real products take; the
+// transposes stay in registers.  A pair I < J takes twelve, into one
+// accumulator each for Re G and Im G, and its mirror is its transpose.
+//
+// Bound by the matrix instructions and the vector unit (operand permutes, list,
+// fold) together, and at 30 dates by Gamma's 8 n^2 bytes per pixel (2.7 TB/s).
+// Measured against 32 x 32 x 16 products of all four real Grams up to 32 dates
+// (2048 x 2048 of 30 dates 14.7 -> 11.1 ms, 640 x 640 of 20 1.40 -> 1.04, 256 x
+// 256 of 10 0.18 -> 0.06) and against the gathering kernel above (208 x 224 of
+// 48 dates 0.87 -> 0.24 ms, 131 k pixels of 64 dates in a 21 x 11 window 4.5 ->
+// 2.1).
 // Workgroups are numbered so that each XCD (which owns an L2) takes a
 // contiguous run of tiles and the halos neighbouring tiles share stay in it.
 // ---------------------------------------------------------------------------
-template <bool F16, int WAVES>
-__global__ __launch_bounds__(64 * WAVES) void gram_mfma_lds(MfmaArgs a) {
-    constexpr int NT = 64 * WAVES;
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+template <bool F16> __device__ __forceinline__ f32x4 mfma16(typename Frag<F16>::type a, typename Frag<F16>::type b, f32x4 c) {
+    if constexpr (F16) return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+    else return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
+
+// Transpose of a 16 x 16 accumulator (lane l, register v: row 4 (l / 16) + v,
+// column l % 16): the 4 x 4 blocks within each quad of lanes, then the blocks.
+template <int CTRL> __device__ __forceinline__ float quad_swap(float x) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xf, 0xf, true));
+}
+__device__ __forceinline__ f32x4 transpose16(f32x4 a, int lane) {
+    const bool o1 = lane & 1, o2 = lane & 2;
+    f32x4 s, c;   // (the swaps by every lane, then the choice)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) s[v] = quad_swap<0xB1>(a[v ^ 1]);
+#pragma unroll
+    for (int v = 0; v < 4; ++v) a[v] = o1 == ((v & 1) != 0) ? a[v] : s[v];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) s[v] = quad_swap<0x4E>(a[v ^ 2]);
+#pragma unroll
+    for (int v = 0; v < 4; ++v) c[v] = o2 == ((v & 2) != 0) ? a[v] : s[v];
+    const int from = 4 * (4 * (lane >> 4) + (lane & 3) + 4 * (lane & 12));
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        const float x = c[v];   // (a bit cast of the element itself takes element 0)
+        c[v] = __int_as_float(__builtin_amdgcn_ds_bpermute(from, __float_as_int(x)));
+    }
+    return c;
+}
+
+// The staged records, padded to 16 NB dates (zeros beyond n and outside the
+// image), eight loads of one or two dates in flight.  A group of 16 lanes
+// reads half of the 64 banks; with an even NB the date blocks of odd positions
+// change places, so that two groups on neighbouring positions read different
+// halves.
+template <typename V, int NB>
+__device__ __forceinline__ void stage_records(const MfmaArgs& a, uint2* rec, int rbase, int cbase, int WC, int NPOS) {
+    constexpr int U = sizeof(V) / 8, DP = 16 * NB / U;
+    const int n = a.n / U, NT = blockDim.x, total = (NPOS + 1) * DP;
+    const V* src = (const V*)a.pk;
+    for (int e0 = threadIdx.x; e0 < total; e0 += 8 * NT) {
+        V v[8];
+        bool in[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int e = e0 + u * NT;
+            const int pos = e / DP, d = e % DP;
+            const int rr = rbase + pos / WC, cc = cbase + pos % WC;
+            in[u] = e < total && d < n && pos < NPOS && rr >= 0 && rr < a.rows && cc >= 0 && cc < a.cols;
+            // slots without data read record 0 and are zeroed below
+            const size_t at = in[u] ? ((size_t)rr * a.cols + cc) * n + d : 0;
+            v[u] = src[at];
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int e = e0 + u * NT;
+            const int at = NB % 2 == 0 ? e ^ (((e / DP) & 1) * (16 / U)) : e;
+            if (e < total) ((V*)rec)[at] = in[u] ? v[u] : V{};
+        }
+    }
+}
+
+// Waves of the largest tile's workgroup: four and two per SIMD is what the
+// registers and LDS allow (two workgroups per CU up to 16 dates).
+constexpr int stage_waves(int nb) { return nb == 1 ? 12 : nb == 2 ? 16 : 8; }
+template <bool F16, int NB>
+__global__ __launch_bounds__(64 * stage_waves(NB)) __attribute__((amdgpu_waves_per_eu(NB <= 2 ? 4 : 2))) void
+gram_mfma_lds(MfmaArgs a) {
+    const int NT = blockDim.x, WAVES = NT >> 6;
+    constexpr int DP = 16 * NB;          // dates of a staged record
+    constexpr int PAIRS = NB * (NB - 1) / 2;
     typedef typename Frag<F16>::type frag_t;
     extern __shared__ __align__(16) char smem[];
     const int n = a.n, Nx = a.Nx, Ny = a.Ny;
     const int TH = a.TH, TW = a.TW;
     const int WR = TH + 2 * Ny, WC = TW + 2 * Nx, NPOS = WR * WC;
-    uint2* rec = (uint2*)smem;                             // [NPOS + 1][32] (re, im) words
+    uint2* rec = (uint2*)smem;                             // [NPOS + 1][DP] (re, im) words
     // wave index in a scalar register, so the pixel loop below is uniform
     // control flow (scalar branches) rather than exec-masked
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    int* list = (int*)(rec + (size_t)(NPOS + 1) * 32) + wave * (a.list_cap + 32 + 64);
-    float* dg = (float*)(list + a.list_cap);                // diagonal of Re G, 32
-    uint32_t* wbuf = (uint32_t*)(dg + 32);                  // next pixel's mask words, 64
+    int* offs = (int*)(rec + (size_t)(NPOS + 1) * DP);      // window offsets, row << 16 | column
+    int* list = offs + 32 * kStageWords + wave * (a.list_cap + DP + 64);
+    float* dg = (float*)(list + a.list_cap);                // diagonal of Re G, DP
+    uint32_t* wbuf = (uint32_t*)(dg + DP);                  // next pixel's mask words, 64
 
     // XCD-aware tile order (blocks are dealt to the 8 XCDs round-robin)
     const unsigned nb = gridDim.x * gridDim.y, bid = blockIdx.y * gridDim.x + blockIdx.x;
-    const unsigned xcd = bid % 8u, q = nb / 8u, rem = nb % 8u;
-    const unsigned logical = xcd * q + min(xcd, rem) + bid / 8u;
+    const unsigned xcd = bid % 8u, q8 = nb / 8u, rem = nb % 8u;
+    const unsigned logical = xcd * q8 + min(xcd, rem) + bid / 8u;
     const int tx = (int)(logical % gridDim.x), ty = (int)(logical / gridDim.x);
     const int R0 = a.row0 + ty * TH, C0 = tx * TW;
     const int row_end = a.row0 + a.chunk_rows;
     const int rbase = R0 - Ny, cbase = C0 - Nx;
 
-    // ---- stage the records, padded to 32 dates (zeros beyond n and outside
-    //      the image), eight loads in flight ----
-    {
-        const int total = (NPOS + 1) * 32;
-        const uint2* src = (const uint2*)a.pk;
-        for (int e0 = threadIdx.x; e0 < total; e0 += 8 * NT) {
-            uint2 v[8];
-            bool in[8];
-#pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                const int e = e0 + u * NT;
-                const int pos = e >> 5, d = e & 31;
-                const int rr = rbase + pos / WC, cc = cbase + pos % WC;
-                in[u] = e < total && d < n && pos < NPOS && rr >= 0 && rr < a.rows && cc >= 0 && cc < a.cols;
-                // slots without data read record 0 and are zeroed below
-                const size_t at = in[u] ? ((size_t)rr * a.cols + cc) * n + d : 0;
-                v[u] = src[at];
-            }
-#pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                const int e = e0 + u * NT;
-                if (e < total) rec[e] = in[u] ? v[u] : make_uint2(0u, 0u);
-            }
-        }
-    }
-    __syncthreads();
-
+    if (n & 1) stage_records<uint2, NB>(a, rec, rbase, cbase, WC, NPOS);
+    else stage_records<uint4, NB>(a, rec, rbase, cbase, WC, NPOS);   // records are 16-byte aligned
     const int Wx = 2 * Nx + 1, Wn = (2 * Ny + 1) * Wx;
-    const int m = lane & 31, hf = lane >> 5;
-    // window offsets of this lane in every 64-wide pass (pixel-independent)
-    constexpr int kPass = (kStageWords * 32 + 63) / 64;
-    int offy[kPass], offx[kPass];
-#pragma unroll
-    for (int it = 0; it < kPass; ++it) {
-        const int f = it * 64 + lane;
-        offy[it] = f / Wx;
-        offx[it] = f - offy[it] * Wx;
-    }
+    for (int f = threadIdx.x; f < Wn; f += NT) offs[f] = f / Wx * 65536 + f % Wx;
+    __syncthreads();
+    const int m = lane & 15, q = lane >> 4;
 
     // mask words of a pixel in lanes 0..nul-1 (one load).  The next pixel's
     // are requested at the top of an iteration and parked in LDS before this
@@ -592,18 +646,19 @@ __global__ __launch_bounds__(64 * WAVES) void gram_mfma_lds(MfmaArgs a) {
             wbuf[lane] = wnext;
             continue;
         }
-        const long long pix = (long long)r * a.cols + c;
         const int slot = (r - a.row0) * a.cols + c;
         const int fc = shp_flat(0, 0, Nx, Ny);
         // mask words reach the lanes through readlane (scalar registers), not
         // through an LDS-routed shuffle
         const bool cen = (__builtin_amdgcn_readlane(wword, fc >> 5) >> (fc & 31)) & 1u;
-        // ---- neighbour list (staged record indices) ----
+        // ---- neighbour list: byte offsets of staged records.  Entry k goes
+        // to the k % 4'th group of 16 lanes, whose eight entries of a step
+        // are contiguous ----
         const int lr = r - R0, lc = c - C0;                  // window origin in the stage
+        auto place = [](int k) { return (k & ~31) | ((k & 3) << 3) | ((k >> 2) & 7); };
+        auto where = [](int pos) { return NB % 2 == 0 ? pos * (DP * 8) + ((pos & 1) << 7) : pos * (DP * 8); };
         int cnt = 0;
-#pragma unroll
-        for (int it = 0; it < kPass; ++it) {
-            if (it * 64 >= Wn) break;   // uniform
+        for (int it = 0; it * 64 < Wn; ++it) {
             const int f = it * 64 + lane;
             // lanes 0..31 test word 2it, lanes 32..63 word 2it+1 (lanes past
             // the last word hold word 0 and only cover positions >= Wn)
@@ -613,7 +668,7 @@ __global__ __launch_bounds__(64 * WAVES) void gram_mfma_lds(MfmaArgs a) {
             bool take = false;
             int qpos = 0;
             if (cen && f < Wn) {
-                const int fy = offy[it], fx = offx[it];
+                const int o = offs[f], fy = o >> 16, fx = o & 0xffff;
                 const int rr = r + fy - Ny, cc = c + fx - Nx;
                 if (rr >= 0 && rr < a.rows && cc >= 0 && cc < a.cols && ((wf >> (f & 31)) & 1u)) {
                     take = true;
@@ -623,7 +678,7 @@ __global__ __launch_bounds__(64 * WAVES) void gram_mfma_lds(MfmaArgs a) {
             const uint64_t bal = __ballot(take);
             if (take) {
                 const uint64_t below = (lane == 0) ? 0ull : (bal & ((~0ull) >> (64 - lane)));
-                list[cnt + __popcll(below)] = qpos;
+                list[place(cnt + __popcll(below))] = where(qpos);
             }
             cnt += __popcll(bal);
         }
@@ -632,88 +687,131 @@ __global__ __launch_bounds__(64 * WAVES) void gram_mfma_lds(MfmaArgs a) {
             if (lane == 0) a.npix[slot] = -1;
             continue;
         }
-        const int steps = (cnt + 15) >> 4;
-        for (int e = cnt + lane; e < steps * 16; e += 64) list[e] = NPOS;
+        const int steps = (cnt + 31) >> 5;
+        for (int e = cnt + lane; e < steps * 32; e += 64) list[place(e)] = where(NPOS);
         wave_sync_lds();
 
-        f32x16 RR, II, RI, IR;
+        f32x4 A[NB], X[NB], W[NB], P[PAIRS ? PAIRS : 1], Q[PAIRS ? PAIRS : 1];
 #pragma unroll
-        for (int v = 0; v < 16; ++v) RR[v] = II[v] = RI[v] = IR[v] = 0.0f;
+        for (int b = 0; b < NB; ++b) A[b] = X[b] = W[b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int t = 0; t < PAIRS; ++t) P[t] = Q[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
         // operands of step st + 1 are loaded while step st's MFMAs run; one
         // 8-byte read gives this lane's (re, im) words of a position
-        uint2 x[8];
-        auto load_step = [&](int st, uint2 (&y)[8]) {
-            const int* lp = list + 16 * st + 8 * hf;
+        uint2 x[NB][8];
+        auto load_step = [&](int st) {
+            const int* lp = list + 32 * st + 8 * q;
 #pragma unroll
-            for (int e = 0; e < 8; ++e) y[e] = rec[(uint32_t)lp[e] * 32u + (uint32_t)m];
-        };
-        load_step(0, x);
-        for (int st = 0; st < steps; ++st) {
-            uint2 nx[8];
-            load_step(st + 1 < steps ? st + 1 : st, nx);
-            u32x4 hr, lr4, hi4, li4;
+            for (int e = 0; e < 8; ++e) {
+                const int at = lp[e] + 8 * m;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                hr[e] = __builtin_amdgcn_perm(x[2 * e + 1].x, x[2 * e].x, 0x05040100u);
-                lr4[e] = __builtin_amdgcn_perm(x[2 * e + 1].x, x[2 * e].x, 0x07060302u);
-                hi4[e] = __builtin_amdgcn_perm(x[2 * e + 1].y, x[2 * e].y, 0x05040100u);
-                li4[e] = __builtin_amdgcn_perm(x[2 * e + 1].y, x[2 * e].y, 0x07060302u);
+                for (int b = 0; b < NB; ++b)
+                    x[b][e] = *(const uint2*)((const char*)rec + (NB % 2 == 0 ? at ^ (b << 7) : at + (b << 7)));
             }
-            const frag_t fhr = __builtin_bit_cast(frag_t, hr), flr = __builtin_bit_cast(frag_t, lr4);
-            const frag_t fhi = __builtin_bit_cast(frag_t, hi4), fli = __builtin_bit_cast(frag_t, li4);
-            // interleaved so that consecutive MFMAs feed different accumulators
-            RR = Frag<F16>::mfma(fhr, fhr, RR);
-            II = Frag<F16>::mfma(fhi, fhi, II);
-            RI = Frag<F16>::mfma(fhr, fhi, RI);
-            IR = Frag<F16>::mfma(fhi, fhr, IR);
-            RR = Frag<F16>::mfma(fhr, flr, RR);
-            II = Frag<F16>::mfma(fhi, fli, II);
-            RI = Frag<F16>::mfma(fhr, fli, RI);
-            IR = Frag<F16>::mfma(fhi, flr, IR);
-            RR = Frag<F16>::mfma(flr, fhr, RR);
-            II = Frag<F16>::mfma(fli, fhi, II);
-            RI = Frag<F16>::mfma(flr, fhi, RI);
-            IR = Frag<F16>::mfma(fli, fhr, IR);
+        };
+        load_step(0);
+        for (int st = 0; st < steps; ++st) {
+            frag_t Rh[NB], Rl[NB], Ih[NB], Il[NB];
 #pragma unroll
-            for (int e = 0; e < 8; ++e) x[e] = nx[e];
+            for (int b = 0; b < NB; ++b) {
+                u32x4 hr, lr4, hi4, li4;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    hr[e] = __builtin_amdgcn_perm(x[b][2 * e + 1].x, x[b][2 * e].x, 0x05040100u);
+                    lr4[e] = __builtin_amdgcn_perm(x[b][2 * e + 1].x, x[b][2 * e].x, 0x07060302u);
+                    hi4[e] = __builtin_amdgcn_perm(x[b][2 * e + 1].y, x[b][2 * e].y, 0x05040100u);
+                    li4[e] = __builtin_amdgcn_perm(x[b][2 * e + 1].y, x[b][2 * e].y, 0x07060302u);
+                }
+                Rh[b] = __builtin_bit_cast(frag_t, hr);
+                Rl[b] = __builtin_bit_cast(frag_t, lr4);
+                Ih[b] = __builtin_bit_cast(frag_t, hi4);
+                Il[b] = __builtin_bit_cast(frag_t, li4);
+            }
+            load_step(st + 1 < steps ? st + 1 : st);
+            // interleaved so that consecutive MFMAs feed different accumulators
+#pragma unroll
+            for (int b = 0; b < NB; ++b) {
+                A[b] = mfma16<F16>(Rh[b], Rh[b], A[b]);
+                X[b] = mfma16<F16>(Rh[b], Rl[b], X[b]);
+                W[b] = mfma16<F16>(Ih[b], Rh[b], W[b]);
+            }
+#pragma unroll
+            for (int b = 0; b < NB; ++b) {
+                A[b] = mfma16<F16>(Ih[b], Ih[b], A[b]);
+                X[b] = mfma16<F16>(Ih[b], Il[b], X[b]);
+                W[b] = mfma16<F16>(Ih[b], Rl[b], W[b]);
+            }
+#pragma unroll
+            for (int b = 0; b < NB; ++b) W[b] = mfma16<F16>(Il[b], Rh[b], W[b]);
+            int t = 0;
+#pragma unroll
+            for (int b = 0; b < NB - 1; ++b) {
+                const u32x4 sign = {0x80008000u, 0x80008000u, 0x80008000u, 0x80008000u};
+                const frag_t Nh = __builtin_bit_cast(frag_t, __builtin_bit_cast(u32x4, Rh[b]) ^ sign);
+                const frag_t Nl = __builtin_bit_cast(frag_t, __builtin_bit_cast(u32x4, Rl[b]) ^ sign);
+#pragma unroll
+                for (int d = b + 1; d < NB; ++d, ++t) {   // P(im_b, re_d) - P(re_b, im_d) is Im G
+                    P[t] = mfma16<F16>(Rh[b], Rh[d], P[t]);
+                    Q[t] = mfma16<F16>(Ih[b], Rh[d], Q[t]);
+                    P[t] = mfma16<F16>(Rh[b], Rl[d], P[t]);
+                    Q[t] = mfma16<F16>(Ih[b], Rl[d], Q[t]);
+                    P[t] = mfma16<F16>(Rl[b], Rh[d], P[t]);
+                    Q[t] = mfma16<F16>(Il[b], Rh[d], Q[t]);
+                    P[t] = mfma16<F16>(Ih[b], Ih[d], P[t]);
+                    Q[t] = mfma16<F16>(Nh, Ih[d], Q[t]);
+                    P[t] = mfma16<F16>(Ih[b], Il[d], P[t]);
+                    Q[t] = mfma16<F16>(Nh, Il[d], Q[t]);
+                    P[t] = mfma16<F16>(Il[b], Ih[d], P[t]);
+                    Q[t] = mfma16<F16>(Nl, Ih[d], Q[t]);
+                }
+            }
         }
 
         wbuf[lane] = wnext;   // waits for the load here, before the stores below
 
-        // ---- fold P into Gamma ----
-        // Re G_mm sits in register 4 (m / 8) + m % 4 of the lanes whose half
-        // holds row m ((m / 4) % 2 == hf); it is picked out by selects, and
-        // every later LDS read is issued before any result is used.
-        float dv = 0.0f;
+        // ---- fold into Gamma ----
+        // Re G_mm sits in register m % 4 of the lanes of quarter m / 4; it is
+        // published as 1 / sqrt: one transcendental per lane, and the
+        // normalisation of entry (i, j) is a product
 #pragma unroll
-        for (int v = 0; v < 16; ++v) dv = (acc_row(v, lane) == m) ? RR[v] + II[v] : dv;
-        // published as 1/sqrt(Re G_mm): one transcendental per lane, and the
-        // normalisation of entry (i, m) is a product
-        if (((m >> 2) & 1) == hf) dg[m] = rsqrtf(dv);
+        for (int b = 0; b < NB; ++b) {
+            float dv = 0.0f;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) dv = (m & 3) == v ? A[b][v] + (X[b][v] + X[b][v]) : dv;
+            if (q == m >> 2) dg[16 * b + m] = rsqrtf(dv);
+        }
         wave_sync_lds();
-        float di[16];
-#pragma unroll
-        for (int v = 0; v < 16; ++v) di[v] = dg[acc_row(v, lane)];
-        const float dj = dg[m];
         float2* gout = reinterpret_cast<float2*>(a.gamma) + (size_t)slot * n * n;
+        // entries (16 I + 4 q + v, 16 J + m)
+        auto put = [&](int I, int J, const f32x4& re, const f32x4& im) {
+            const float dj = dg[16 * J + m];
+            const int col = 16 * J + m;
+            float di[4];
 #pragma unroll
-        for (int v = 0; v < 16; ++v) {
-            const int i = acc_row(v, lane);
-            const float sc = di[v] * dj;
-            const bool off = i != m;
-            const float gr = off ? (RR[v] + II[v]) * sc : 1.0f;
-            const float gi = off ? (IR[v] - RI[v]) * sc : 0.0f;   // P(im_i, re_j) - P(re_i, im_j)
-            if (i < n && m < n) gout[(size_t)i * n + m] = make_float2(gr, gi);
+            for (int v = 0; v < 4; ++v) di[v] = dg[16 * I + 4 * q + v];
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int row = 16 * I + 4 * q + v;
+                const float sc = di[v] * dj;
+                const bool off = I != J || 4 * q + v != m;
+                const float gr = off ? re[v] * sc : 1.0f;
+                const float gi = off ? im[v] * sc : 0.0f;
+                if (row < n && col < n) gout[(size_t)row * n + col] = make_float2(gr, gi);
+            }
+        };
+        int t = 0;
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            put(b, b, A[b] + (X[b] + transpose16(X[b], lane)), W[b] - transpose16(W[b], lane));
+#pragma unroll
+            for (int d = b + 1; d < NB; ++d, ++t) {
+                put(b, d, P[t], Q[t]);
+                put(d, b, transpose16(P[t], lane), -transpose16(Q[t], lane));
+            }
         }
         if (lane == 0) a.npix[slot] = cnt;
         wave_sync_lds();
     }
-}
-
-static size_t gram_lds_bytes(int Nx, int Ny, int TH, int TW, int list_cap, int waves) {
-    // records are staged padded to 32 dates
-    const size_t stage = (size_t)((TH + 2 * Ny) * (TW + 2 * Nx) + 1) * 32 * 8;
-    return stage + (size_t)waves * (list_cap + 32 + 64) * 4;
 }
 
 static int gram_list_cap(int Nx, int Ny) {
@@ -721,66 +819,49 @@ static int gram_list_cap(int Nx, int Ny) {
     return ((Wn + 15) / 16) * 16 + 16;
 }
 
-// Tile of the staged kernel.  First choice: an 8 x 16 tile for twelve
-// waves (three per SIMD), one workgroup per CU, which stages ~4.2 records
-// per pixel at a 15 x 11 window; then a 4 x 16 tile for eight waves (~6.6;
-// a 3 x 8 tile stages ~11.9).  Otherwise the largest TH x TW tile
-// (TH <= 4, TW <= 8) for four waves whose stage keeps two workgroups on a
-// CU.  Returns the stage's LDS bytes.
-// `only`: a scheduled variant (FRINGE_GRAM_STAGED12 / 8 / 4) tries that tile
-// alone; FRINGE_GRAM_DEFAULT tries them in order.
-static size_t gram_stage_tile(int Nx, int Ny, int& TH, int& TW, int& waves, int only = FRINGE_GRAM_DEFAULT) {
-    const int cap = gram_list_cap(Nx, Ny);
-    waves = 12;
-    TH = 8;
-    TW = 16;
-    if ((only == FRINGE_GRAM_DEFAULT || only == FRINGE_GRAM_STAGED12) &&
-        gram_lds_bytes(Nx, Ny, TH, TW, cap, waves) <= 156 * 1024)
-        return gram_lds_bytes(Nx, Ny, TH, TW, cap, waves);
-    waves = 8;
-    TH = 4;
-    TW = 16;
-    if ((only == FRINGE_GRAM_DEFAULT || only == FRINGE_GRAM_STAGED8) &&
-        gram_lds_bytes(Nx, Ny, TH, TW, cap, waves) <= 150 * 1024)
-        return gram_lds_bytes(Nx, Ny, TH, TW, cap, waves);
-    if (only != FRINGE_GRAM_DEFAULT && only != FRINGE_GRAM_STAGED4) return (size_t)1 << 40;
-    const size_t budget = 78 * 1024;
-    waves = 4;
-    TH = 4;
-    TW = 8;
-    while (TH > 1 && gram_lds_bytes(Nx, Ny, TH, TW, cap, waves) > budget) --TH;
-    while (TW > 1 && gram_lds_bytes(Nx, Ny, TH, TW, cap, waves) > budget) TW >>= 1;
-    if (TH * TW >= 4) return gram_lds_bytes(Nx, Ny, TH, TW, cap, waves);
-    // a stage for fewer than four pixels leaves waves idle: take the largest
-    // tile of at least four pixels that fits one workgroup per CU, or none
-    // (the unstaged kernel then gathers from L2)
-    for (TH = 4; TH >= 1; --TH)
-        for (TW = 8; TW >= 1; TW >>= 1)
-            if (TH * TW >= 4 && gram_lds_bytes(Nx, Ny, TH, TW, cap, waves) <= 156 * 1024)
-                return gram_lds_bytes(Nx, Ny, TH, TW, cap, waves);
-    return (size_t)1 << 40;
+struct StageTile {
+    int TH, TW, waves;
+};
+// Largest first.  8 x 16 pixels stage ~4.2 records per pixel at a 15 x 11
+// window, 4 x 16 ~6.6, 4 x 8 9.7, 2 x 4 27.
+constexpr StageTile kStageTiles[] = {{8, 16, 16}, {4, 16, 8}, {4, 8, 8}, {4, 4, 8}, {2, 4, 8}, {2, 2, 4}};
+
+static size_t gram_lds_bytes(int n, int Nx, int Ny, const StageTile& t) {
+    const int dp = (n + 15) / 16 * 16;
+    const size_t stage = (size_t)((t.TH + 2 * Ny) * (t.TW + 2 * Nx) + 1) * dp * 8;
+    return stage + 32 * kStageWords * 4 + (size_t)t.waves * (gram_list_cap(Nx, Ny) + dp + 64) * 4;
 }
 
-// The staged kernel takes windows of up to kStageWords mask words; larger
-// windows go to the unstaged kernel, which walks any number of words.
-// A scheduled variant (fringe_schedule_set) that does not fit the window
-// falls back to the default choice.
-static bool gram_staged(int n, int Nx, int Ny, int& TH, int& TW, int& waves, size_t& bytes) {
-    if (n > 32 || shp_words(Nx, Ny) > kStageWords) return false;
-    const int v = schedule_lookup(FRINGE_SCHED_GRAM_VARIANT, n, Nx, Ny, FRINGE_GRAM_DEFAULT);
+// Tile of the staged kernel: the largest that fits a CU's LDS and cuts the
+// grid into two workgroups per CU, or else the smallest that fits.  (64 x 64
+// pixels of 8 dates: 32 tiles of 8 x 16 took 77 us, 512 of 2 x 4 take 12.)
+// A scheduled variant (FRINGE_GRAM_STAGED12 / 8 / 4) names the largest tile
+// tried; one that does not fit the window falls back to the others.  False
+// above 64 dates, for windows of more than kStageWords mask words and where
+// nothing fits: the gathering kernels walk any number of words.
+static bool gram_staged(int n, int Nx, int Ny, long long rows, int cols, StageTile& best, size_t& bytes) {
+    if (n > 64 || shp_words(Nx, Ny) > kStageWords) return false;
+    const int v = n <= 32 ? schedule_lookup(FRINGE_SCHED_GRAM_VARIANT, n, Nx, Ny, FRINGE_GRAM_DEFAULT) : FRINGE_GRAM_DEFAULT;
     if (v == FRINGE_GRAM_UNSTAGED) return false;
-    if (v != FRINGE_GRAM_DEFAULT) {
-        bytes = gram_stage_tile(Nx, Ny, TH, TW, waves, v);
-        if (bytes <= 160 * 1024) return true;
+    const int from = v == FRINGE_GRAM_STAGED8 ? 1 : v == FRINGE_GRAM_STAGED4 ? 2 : 0;
+    bool found = false;
+    for (int k = from; k < (int)(sizeof(kStageTiles) / sizeof(kStageTiles[0])); ++k) {
+        StageTile t = kStageTiles[k];
+        t.waves = std::min(t.waves, stage_waves((n + 15) / 16));
+        const size_t b = gram_lds_bytes(n, Nx, Ny, t);
+        if (b > 160 * 1024) continue;
+        best = t;
+        bytes = b;
+        found = true;
+        if ((long long)((cols + t.TW - 1) / t.TW) * ((rows + t.TH - 1) / t.TH) >= 512) break;
     }
-    bytes = gram_stage_tile(Nx, Ny, TH, TW, waves);
-    return bytes <= 160 * 1024;
+    return found;
 }
 
 int gram_stage_rows(int n, int Nx, int Ny) {
-    int TH, TW, waves;
+    StageTile t;
     size_t bytes;
-    return gram_staged(n, Nx, Ny, TH, TW, waves, bytes) ? TH : 1;
+    return n <= 32 && gram_staged(n, Nx, Ny, 1ll << 30, 1 << 20, t, bytes) ? t.TH : 1;
 }
 
 // packed records followed by the per-date maxima (256-byte aligned)
@@ -815,6 +896,17 @@ static void launch_mfma(MfmaArgs a, hipStream_t s) {
     hipLaunchKernelGGL((gram_mfma<NBH, WAVES, F16>), grid, dim3(64 * WAVES), wbytes * WAVES, s, a);
 }
 
+template <bool F16> static void launch_staged(const MfmaArgs& a, int waves, size_t bytes, hipStream_t s) {
+    const dim3 grid((unsigned)((a.cols + a.TW - 1) / a.TW), (unsigned)((a.chunk_rows + a.TH - 1) / a.TH));
+    const dim3 blk(64 * waves);
+    switch ((a.n + 15) / 16) {   // blocks of 16 dates
+        case 1: hipLaunchKernelGGL((gram_mfma_lds<F16, 1>), grid, blk, bytes, s, a); break;
+        case 2: hipLaunchKernelGGL((gram_mfma_lds<F16, 2>), grid, blk, bytes, s, a); break;
+        case 3: hipLaunchKernelGGL((gram_mfma_lds<F16, 3>), grid, blk, bytes, s, a); break;
+        default: hipLaunchKernelGGL((gram_mfma_lds<F16, 4>), grid, blk, bytes, s, a); break;
+    }
+}
+
 int gram_mfma_launch(const LinkPlan& P, const uint32_t* pk, const uint32_t* wts, long long first,
                      int slots, hipStream_t s) {
     if (P.n > kMaxBandsMfma || first % P.cols != 0 || slots % P.cols != 0) return -1;
@@ -836,30 +928,17 @@ int gram_mfma_launch(const LinkPlan& P, const uint32_t* pk, const uint32_t* wts,
     a.npix = P.d_npix;
     a.list_cap = gram_list_cap(P.Nx, P.Ny);
     const bool f16 = (P.precision != FRINGE_PREC_MIXED_BF16);
-    if (P.n <= 32) {
-        int TH, TW, waves;
-        size_t bytes = 0;
-        if (gram_staged(P.n, P.Nx, P.Ny, TH, TW, waves, bytes)) {
-            a.TH = TH;
-            a.TW = TW;
-            const dim3 grid((unsigned)((a.cols + TW - 1) / TW), (unsigned)((a.chunk_rows + TH - 1) / TH));
-            const dim3 blk(64 * waves);
-            if (waves == 12) {
-                if (f16) hipLaunchKernelGGL((gram_mfma_lds<true, 12>), grid, blk, bytes, s, a);
-                else hipLaunchKernelGGL((gram_mfma_lds<false, 12>), grid, blk, bytes, s, a);
-            } else if (waves == 8) {
-                if (f16) hipLaunchKernelGGL((gram_mfma_lds<true, 8>), grid, blk, bytes, s, a);
-                else hipLaunchKernelGGL((gram_mfma_lds<false, 8>), grid, blk, bytes, s, a);
-            } else {
-                if (f16) hipLaunchKernelGGL((gram_mfma_lds<true, 4>), grid, blk, bytes, s, a);
-                else hipLaunchKernelGGL((gram_mfma_lds<false, 4>), grid, blk, bytes, s, a);
-            }
-        } else if (f16) {
-            launch_mfma<1, 4, true>(a, s);
-        } else {
-            launch_mfma<1, 4, false>(a, s);
-        }
-    } else {   // above 32 dates
+    StageTile t;
+    size_t bytes = 0;
+    if (gram_staged(P.n, P.Nx, P.Ny, a.chunk_rows, P.cols, t, bytes)) {
+        a.TH = t.TH;
+        a.TW = t.TW;
+        if (f16) launch_staged<true>(a, t.waves, bytes, s);
+        else launch_staged<false>(a, t.waves, bytes, s);
+    } else if (P.n <= 32) {
+        if (f16) launch_mfma<1, 4, true>(a, s);
+        else launch_mfma<1, 4, false>(a, s);
+    } else {
         const size_t wbytes = (size_t)a.list_cap * 4 + 128 * 4;
         const dim3 grid((unsigned)((a.cols + a.TW - 1) / a.TW), (unsigned)((a.chunk_rows + a.TH - 1) / a.TH));
         if (f16) hipLaunchKernelGGL((gram_mfma_pairs<4, true>), grid, dim3(256), wbytes * 4, s, a);

@@ -203,9 +203,9 @@ int fringe_link_batch_run(const fringe_link_batch_item* items, int count, void* 
                                        otherwise one row per lane up to 64 dates (0), or its work matrix in LDS
                                        (0) or global memory (1) above 64 dates */
 #define FRINGE_GRAM_DEFAULT 0
-#define FRINGE_GRAM_STAGED12 1      /* 12 waves, 8 x 16-pixel tiles staged in LDS */
-#define FRINGE_GRAM_STAGED8 2       /* 8 waves, 4 x 16 */
-#define FRINGE_GRAM_STAGED4 3       /* 4 waves, up to 4 x 8 */
+#define FRINGE_GRAM_STAGED12 1      /* pixel tiles of up to 8 x 16 staged in LDS */
+#define FRINGE_GRAM_STAGED8 2       /* up to 4 x 16 */
+#define FRINGE_GRAM_STAGED4 3       /* up to 4 x 8 */
 #define FRINGE_GRAM_UNSTAGED 4      /* one wave per pixel, records gathered from L2 */
 int fringe_schedule_set(int kind, int key0, int key1, int key2, int value);
 int fringe_schedule_get(int kind, int key0, int key1, int key2);
