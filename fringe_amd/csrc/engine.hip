@@ -592,9 +592,9 @@ int fringe_nmap_run(const fringe_nmap_tile* t, const void* d_slc, const uint8_t*
     P.alpha[0] = 1.0;
     uint8_t tab[kMaxBandsNmap + 1];
     fringe_ks_table(t->nbands, t->prob, tab);
-    std::memset(P.table.bits, 0, sizeof(P.table.bits));
-    for (int k = 0; k <= t->nbands; ++k)
-        if (tab[k]) P.table.bits[k >> 5] |= (1u << (k & 31));
+    // the p-value does not increase with k, so the similar ones are 0 .. ks_max
+    P.ks_max = -1;
+    while (P.ks_max < t->nbands && tab[P.ks_max + 1]) ++P.ks_max;
     nmap_layout(t, &P, d_work);
     P.method = t->method;
     if (t->method == 1) {

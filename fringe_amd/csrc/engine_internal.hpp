@@ -27,22 +27,17 @@ inline int resolve_generic_blocks(size_t area_bytes, size_t budget = kResolveAre
 }
 constexpr int kMaxMaskWords = 64;    // window up to 2048 positions (the reference sequential default 59 x 19 is 1121)
 
-// Decision table of the integer KS statistic, one bit per k = D*n.
-struct KsTable {
-    uint32_t bits[(kMaxBandsNmap + 1 + 31) / 32];
-};
-
 struct NmapPlan {
     int rows, cols, n, Nx, Ny, nul, row_begin, row_end;
     double alpha[kMaxBandsNmap];  // amplitudeConstant_b / amplitudeConstant_1
-    KsTable table;
+    int ks_max;        // KS2: similar iff the integer statistic k = D*n <= ks_max (-1: never)
     float* d_amp;      // [rows*cols][n] sorted amplitudes
     uint8_t* d_valid;  // [rows*cols]
     int method;        // 0 = KS2, 1 = AD2
     double ad2_sigma;  // AD2: standard deviation of A2_kN (k = 2, n + n samples)
     double ad2_max;    // AD2: similar iff the standardised statistic <= ad2_max
     double* d_ad2;     // AD2: [2n-1][n+1] per-position terms of the inner sum
-    uint32_t* d_fwd;   // forward-half mask words, [rows*cols][nul - centre/32]
+    uint32_t* d_fwd;   // forward-half mask words, [nul - centre/32][rows*cols]
     int32_t* d_fcnt;   // forward-half counts, [rows*cols]
 };
 

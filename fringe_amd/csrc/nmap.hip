@@ -7,18 +7,18 @@
 //
 // Stage 1 (nmap_prep): per pixel, amplitude |z| / alpha_b for every band,
 // validity, and an ascending sort held in registers (bitonic network).
-// Stage 2 (nmap_net for n <= 64, nmap_sweep above): per pixel, the
-// two-sample test against every valid in-image neighbour of the forward half
-// of the window (dy > 0, or dy = 0 and dx >= 0), as the reference's sweep
-// visits pairs (nmap.cpp:404-457); the bits go to a workspace.  Stage 3
+// Stage 2 (nmap_ks, nmap_walk): per pixel, the two-sample test against every
+// valid in-image neighbour of the forward half of the window (dy > 0, or dy =
+// 0 and dx >= 0), as the reference's sweep visits pairs (nmap.cpp:404-457); the
+// bits go to a workspace.  Stage 3
 // (nmap_mirror) assembles every output pixel's full mask: bit (dy, dx) of
 // the backward half is bit (-dy, -dx) of neighbour p + (dy, dx), i.e. the
-// same test of the same ordered pair, so each pair is tested once.  KS2: the statistic as an integer count k = D*n,
-// decided through a host-built table (k -> similar) instead of evaluating the
-// Kolmogorov series on the device.  AD2: the standardised Anderson-Darling
-// statistic in double, bit-identical to the host's, compared with the largest
-// statistic whose interpolated p-value still reaches the threshold (found on
-// the host, so no exp/log runs on the device).
+// same test of the same ordered pair, so each pair is tested once.  KS2: the
+// statistic as an integer count k = D*n, compared with the largest one whose
+// p-value reaches the threshold (found on the host).  AD2: the standardised
+// Anderson-Darling statistic in double, bit-identical to the host's, compared
+// with the largest statistic whose interpolated p-value still reaches the
+// threshold (found on the host, so no exp/log runs on the device).
 #include "device_common.hpp"
 #include "engine_internal.hpp"
 #include "timing.hpp"
@@ -44,15 +44,13 @@ template <int NP> __device__ inline void bitonic_sort(float (&a)[NP]) {
 #pragma unroll
         for (int j = k >> 1; j > 0; j >>= 1) {
 #pragma unroll
-            for (int i = 0; i < NP; ++i) {
-                const int l = i ^ j;
-                if (l > i) {
-                    const bool up = ((i & k) == 0);
-                    const float x = a[i], y = a[l];
-                    const float lo = fminf(x, y), hi = fmaxf(x, y);
-                    a[i] = up ? lo : hi;
-                    a[l] = up ? hi : lo;
-                }
+            for (int t = 0; t < NP / 2; ++t) {
+                const int i = ((t & ~(j - 1)) << 1) | (t & (j - 1)), l = i | j;
+                const bool up = ((i & k) == 0);
+                const float x = a[i], y = a[l];
+                const float lo = fminf(x, y), hi = fmaxf(x, y);
+                a[i] = up ? lo : hi;
+                a[l] = up ? hi : lo;
             }
         }
     }
@@ -89,60 +87,6 @@ __global__ __launch_bounds__(256) void nmap_prep(const NmapPlan P, const float2*
         if (b < n) amp_sorted[(long long)b * npx + p] = a[b];
 }
 
-// Integer KS walk over two ascending arrays of length n (element i at
-// x[i * st]), stepping exactly as KS2sample::test does
-// (KS2sample.hpp:105-138): one element on strict order, every copy of a tied
-// value on both sides on a tie, the running difference sampled after each
-// step while both sides have elements left.  Returns k = D * n.
-__device__ inline int ks_count(const float* __restrict__ a, const float* __restrict__ b, int n,
-                               long long st) {
-    int ia = 0, ib = 0, d = 0, dmax = 0;
-    float x = a[0], y = b[0];
-    for (int it = 0; it < 2 * n; ++it) {
-        if (x < y) {
-            --d;
-            ++ia;
-        } else if (x > y) {
-            ++d;
-            ++ib;
-        } else {
-            const float v = x;
-            while (ia < n && a[ia * st] == v) { --d; ++ia; }
-            while (ib < n && b[ib * st] == v) { ++d; ++ib; }
-        }
-        if (ia >= n || ib >= n) break;
-        x = a[ia * st];
-        y = b[ib * st];
-        dmax = max(dmax, abs(d));
-    }
-    return max(dmax, abs(d));
-}
-
-// Anderson-Darling inner sum of AD2unique::test (AD2unique.hpp:206-351) for
-// ascending a (first sample) and b: merge with ties taken from b first and
-// add, for every merged position j < 2n-1, the term of (j, m_j) where m_j
-// counts the a values among the first j+1.  The terms are tabulated once per
-// call (ad2_terms), so the double sum adds the same values in the same order.
-__device__ inline double ad2_inner(const float* __restrict__ a, const float* __restrict__ b, int n,
-                                   long long st, const double* __restrict__ T) {
-    int ia = 0, ib = 0, m = 0;
-    double S = 0.0;
-    float x = a[0], y = b[0];
-    for (int j = 0; j < 2 * n - 1; ++j) {
-        const bool take_a = (ia < n && ib < n) ? (x < y) : (ia < n);
-        if (take_a) {
-            ++ia;
-            ++m;
-            x = ia < n ? a[ia * st] : x;
-        } else {
-            ++ib;
-            y = ib < n ? b[ib * st] : y;
-        }
-        S = S + T[j * (n + 1) + m];
-    }
-    return S;
-}
-
 // term(j, m) = (2n m - n (j+1))^2 / ((j+1)(2n - j - 1)); every intermediate
 // is an exact integer in double, so the one rounding is the division's.
 __global__ void ad2_terms(double* __restrict__ T, int n) {
@@ -162,184 +106,261 @@ __device__ inline double ad2_standardise(double S, int n, double sigma) {
     return (A - 1) / sigma;
 }
 
-__device__ inline bool ks_similar(int k, const NmapPlan& P) {
-    const uint32_t tw = k < 32 ? P.table.bits[0] : k < 64 ? P.table.bits[1] : k < 96 ? P.table.bits[2]
-                        : k < 128 ? P.table.bits[3] : P.table.bits[4];
-    return ((tw >> (k & 31)) & 1u) != 0u;
-}
-
-// ---------------------------------------------------------------------------
-// n <= 64: merge network in registers.  Positive floats order like their bit
-// patterns, so key = bits << 1 | tag orders by value and, among equal values,
-// by tag.  The pixel's own keys stay in registers; a neighbour's keys are read
-// coalesced (date-planar layout) and the two sorted runs are merged by a
-// bitonic network (own keys ascending, neighbour's descending).
-//   KS2: tag 1 = neighbour.  d after a prefix = #neighbour - #own; the walk of
-//        KS2sample::test samples d exactly at the ends of runs of equal
-//        values (inside a run of one sample d is monotone, so the samples
-//        the walk takes there add nothing), so k = max |d| over positions
-//        whose successor has a different value.
-//   AD2: tag 1 = the test's first sample, so ties put the second sample
-//        first as AD2unique::test merges them; m_j = number of tag-1 keys in
-//        the first j+1 positions.
-// Pads (beyond n) get keys above every finite or infinite amplitude.
-// ---------------------------------------------------------------------------
-// Forward-half words of the pixels of rows [fwd_row0, row_end): the
-// output rows and the Ny rows above them whose forward tests reach into
-// them.  Pixel (r, c) keeps words centre/32 .. nul-1 of its mask at
-// F + ((r - fwd_row0) * cols + c) * nf, and its forward count (centre
-// included) at fcnt[(r - fwd_row0) * cols + c].
+// Forward-half words of the pixels of rows [fwd_row0, row_end): the output
+// rows and the Ny rows above them whose forward tests reach into them.  Word w
+// of pixel (r, c)'s mask (centre/32 .. nul-1) is in plane w - centre/32 of F, at
+// (r - fwd_row0) * cols + c, as is its forward count (centre included) in fcnt.
 __device__ inline int fwd_row0(const NmapPlan& P) { return max(0, P.row_begin - P.Ny); }
 __device__ inline int centre_flat(const NmapPlan& P) { return P.Ny * (2 * P.Nx + 1) + P.Nx; }
 
-template <int NP, bool AD2>
-__global__ __launch_bounds__(256) void nmap_net(const NmapPlan P, uint32_t* __restrict__ F,
-                                                int32_t* __restrict__ fcnt) {
+// KS2: max |F_a - F_b| n <= K for ascending a and b if and only if
+// b_{i-K} <= a_i and a_{i-K} <= b_i for every i in K .. n-1 (the count of a's
+// values up to a_i is i + 1 at least, so that of b's has to be i + 1 - K).  So
+// every date of a neighbour has a range, a_{i-K} <= b_i <= a_{i+K}, in which
+// the pixel's own values, shifted by K, put it: one subtraction and one
+// unsigned comparison a date, no merge.
+//
+// A workgroup takes up to 256 pixels of a row.  Per window row (and strip of
+// 32 columns, and chunk of CH dates) the neighbours' samples are staged in
+// LDS, pixel-major (a pitch of an odd number of quads: 16-byte reads without
+// bank conflicts), and every thread tests its window columns from there; the ranges
+// stay in registers.  Bound by the vector unit and the LDS reads (2.5 CH
+// instructions and 4 CH bytes a pair).  2048 x 2048 pixels of 30 dates, 15 x 11
+// window, against the register merge network it replaced: 16.1 -> 1.5 ms.
+template <int CH>
+__global__ __launch_bounds__(256) void nmap_ks(const NmapPlan P, int row_blocks, uint32_t* __restrict__ F,
+                                               int32_t* __restrict__ fcnt) {
+    constexpr int PITCH = CH % 8 == 4 ? CH : CH + 4, STRIP = 32;
+    __shared__ __align__(16) uint32_t L[(256 + STRIP - 1) * PITCH];
+    const uint32_t* __restrict__ keys = reinterpret_cast<const uint32_t*>(P.d_amp);
+    const uint8_t* __restrict__ valid = P.d_valid;
+    const int n = P.n, rows = P.rows, cols = P.cols, Nx = P.Nx, Ny = P.Ny, nul = P.nul, K = P.ks_max;
+    const long long npx = (long long)rows * cols;
+    const int T = blockDim.x, tid = threadIdx.x;
+    // blocks are dealt to the 8 XCDs round-robin: each takes a contiguous run
+    // of rows, whose neighbours' samples stay in its L2
+    const unsigned nb = gridDim.x, xcd = blockIdx.x % 8u;
+    const int id = (int)(xcd * (nb / 8u) + min(xcd, nb % 8u) + blockIdx.x / 8u);
+    const int h0 = fwd_row0(P), r = h0 + id / row_blocks, c0 = id % row_blocks * T, c = c0 + tid;
+    const bool here = c < cols;
+    const long long p = (long long)r * cols + (here ? c : 0);
+    const bool pv = here && valid[p] != 0;
+    const int centre = centre_flat(P), fw = centre >> 5, nf = nul - fw;
+    const long long plane = (long long)(P.row_end - h0) * cols;
+    uint32_t* out = F + (long long)(r - h0) * cols + (here ? c : 0);
+    uint32_t lo[CH], span[CH];
+    auto ranges = [&](int d0) {   // of dates d0 .. d0 + CH - 1; any valid key where there is none
+#pragma unroll
+        for (int i = 0; i < CH; ++i) {
+            const int d = d0 + i;
+            lo[i] = d < n && d >= K ? keys[(long long)(d - K) * npx + p] : 0u;
+            const uint32_t hi = d < n - K ? keys[(long long)(d + K) * npx + p] : 0x7FFFFFFFu;
+            span[i] = hi - lo[i];
+        }
+    };
+    const bool one = n <= CH;   // all dates in one chunk
+    if (K >= 0 && one) ranges(0);
+    int cnt = 0, word = 0, pos = centre & 31;
+    uint64_t cur = 0;
+    for (int dy = 0; dy <= Ny; ++dy) {
+        const int rr = r + dy;
+        for (int dx0 = dy == 0 ? 0 : -Nx; dx0 <= Nx; dx0 += STRIP) {
+            const int w = min(STRIP, Nx - dx0 + 1);
+            uint32_t fail = 0u;
+            if (rr < rows && K >= 0) {   // uniform
+                for (int d0 = 0; d0 < n; d0 += CH) {
+                    const int m = min(CH, n - d0);
+                    __syncthreads();   // the last strip's reads are over
+                    for (int e = tid; e < T + w - 1; e += T) {
+                        const int cc = c0 + dx0 + e;
+                        const bool in = cc >= 0 && cc < cols;
+                        const long long q = (long long)rr * cols + (in ? cc : 0);
+                        const bool ok = in && valid[q] != 0;
+#pragma unroll
+                        for (int i = 0; i < CH; i += 4) {
+                            uint32_t v[4];
+#pragma unroll
+                            for (int u = 0; u < 4; ++u) v[u] = i + u < m ? keys[(long long)(d0 + i + u) * npx + q] : 0u;
+                            // no range holds the key of a pixel that is not there
+                            *(uint4*)&L[e * PITCH + i] = ok ? make_uint4(v[0], v[1], v[2], v[3])
+                                                            : make_uint4(~0u, ~0u, ~0u, ~0u);
+                        }
+                    }
+                    __syncthreads();
+                    if (!one) ranges(d0);
+#pragma unroll 2
+                    for (int k = 0; k < w; ++k) {
+                        uint32_t over = 0u;   // what exceeds a range (saturating)
+#pragma unroll
+                        for (int i = 0; i < CH; i += 4) {
+                            const uint4 b = *(const uint4*)&L[(tid + k) * PITCH + i];
+                            over |= __builtin_elementwise_sub_sat(b.x - lo[i], span[i]);
+                            over |= __builtin_elementwise_sub_sat(b.y - lo[i + 1], span[i + 1]);
+                            over |= __builtin_elementwise_sub_sat(b.z - lo[i + 2], span[i + 2]);
+                            over |= __builtin_elementwise_sub_sat(b.w - lo[i + 3], span[i + 3]);
+                        }
+                        fail |= (over != 0u ? 1u : 0u) << k;
+                    }
+                }
+            } else {
+                fail = ~0u;
+            }
+            uint32_t bits = pv ? ~fail & (~0u >> (32 - w)) : 0u;
+            if (dy == 0 && dx0 == 0) bits |= pv ? 1u : 0u;   // the pixel itself
+            cnt += __popc(bits);
+            cur |= (uint64_t)bits << pos;
+            pos += w;
+            if (pos >= 32) {
+                if (here) out[word * plane] = (uint32_t)cur;
+                ++word;
+                cur >>= 32;
+                pos -= 32;
+            }
+        }
+    }
+    if (here) {
+        for (; word < nf; ++word) {
+            out[word * plane] = (uint32_t)cur;
+            cur = 0;
+        }
+        fcnt[(long long)(r - h0) * cols + c] = cnt;
+    }
+}
+
+// AD2: the merge as a walk.  The inner sum of AD2unique::test
+// (AD2unique.hpp:206-351) merges ascending a (the pixel, the test's first
+// sample) and b with ties taken from b first and adds, for every merged
+// position j < 2n-1, the term of (j, m_j) where m_j counts the a values among
+// the first j+1; the same values are added here in the same order.  The term
+// depends on |2 m - (j+1)| alone, so half of the table is kept.
+//
+// A workgroup takes 64 pixels of a row; per window row (and strip of 32
+// columns) the neighbours' samples are staged in LDS next to the pixels' own
+// and the terms, and its four waves share the window's columns, two walks at
+// a time per thread.  Bound by the walk's chain (compare, address, LDS read).
+// 203 x 317 pixels of 72 dates, 13 x 9 window, against one thread per pixel
+// walking in global memory (one wave per SIMD): 3.6 -> 0.6 ms; 512 x 512
+// pixels of 30 dates against a merge network in registers: 1.90 -> 0.72.
+constexpr int kWalkStrip = 32;
+__host__ __device__ inline int ad2_row_terms(int n, int b) { return (b < 2 * n - b ? b : 2 * n - b) / 2 + 1; }   // of position b - 1
+__host__ __device__ inline int ad2_row_offset(int n, int b) {   // sum of ad2_row_terms(n, 1 .. b - 1)
+    const int t = b <= n ? b - 1 : n, u = 2 * n - b;
+    const int head = t * t / 4 + t;
+    return b <= n ? head : head + (n - 1) * (n - 1) / 4 - u * u / 4 + (b - 1 - n);
+}
+static size_t ad2_walk_bytes(int n) {
+    return (size_t)ad2_row_offset(n, 2 * n) * 8 + (size_t)((64 + 64 + kWalkStrip - 1) * ((n + 1) | 1) + 4 * 64) * 4;
+}
+
+__global__ __launch_bounds__(256) void nmap_walk(const NmapPlan P, int row_blocks, uint32_t* __restrict__ F,
+                                                 int32_t* __restrict__ fcnt) {
+    extern __shared__ __align__(16) char smem[];
     const uint32_t* __restrict__ keys = reinterpret_cast<const uint32_t*>(P.d_amp);
     const uint8_t* __restrict__ valid = P.d_valid;
     const int n = P.n, rows = P.rows, cols = P.cols, Nx = P.Nx, Ny = P.Ny, nul = P.nul;
+    const int pitch = (n + 1) | 1;   // a run's keys, then one above every amplitude
+    const int terms = ad2_row_offset(n, 2 * n);
+    double* T = (double*)smem;
+    uint32_t* own = (uint32_t*)(T + terms);
+    uint32_t* oth = own + 64 * pitch;
+    uint32_t* part = oth + (64 + kWalkStrip - 1) * pitch;   // [4][64] bits of the waves
     const long long npx = (long long)rows * cols;
-    const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    const int h0 = fwd_row0(P);
-    if (t >= (long long)(P.row_end - h0) * cols) return;
-    const int r = h0 + (int)(t / cols);
-    const int c = (int)(t % cols);
-    const long long p = (long long)r * cols + c;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const unsigned nb = gridDim.x, xcd = blockIdx.x % 8u;   // as nmap_ks
+    const int id = (int)(xcd * (nb / 8u) + min(xcd, nb % 8u) + blockIdx.x / 8u);
+    const int h0 = fwd_row0(P), r = h0 + id / row_blocks, c0 = id % row_blocks * 64, c = c0 + lane;
+    const bool here = c < cols;
+    const long long p = (long long)r * cols + (here ? c : 0);
+    const bool pv = here && valid[p] != 0;
     const int centre = centre_flat(P), fw = centre >> 5, nf = nul - fw;
-    uint32_t* out = F + t * nf;   // word w of the mask at out[w - fw]
-    const bool pv = valid[p] != 0;
-    uint32_t A[NP];
-#pragma unroll
-    for (int i = 0; i < NP; ++i) A[i] = (pv && i < n) ? (keys[i * npx + p] << 1) : 0xFFFFFFFEu;
-    int cnt = 0, word = fw, flat = centre;
-    uint32_t cur = 0u;
+    const long long plane = (long long)(P.row_end - h0) * cols;
+    uint32_t* out = F + (long long)(r - h0) * cols + (here ? c : 0);
+    for (int j = wave; j < 2 * n - 1; j += 4) {
+        const int b = j + 1, at = ad2_row_offset(n, b);
+        for (int d = lane; d < ad2_row_terms(n, b); d += 64) T[at + d] = P.d_ad2[j * (n + 1) + (b + 2 * d + (b & 1)) / 2];
+    }
+    // keys of 64 or more consecutive pixels of row rr from column `from` on
+    auto stage = [&](uint32_t* dst, int rr, int from, int count) {
+        for (int e = lane; e < count; e += 64) {
+            const int cc = from + e;
+            const bool in = cc >= 0 && cc < cols;
+            const long long q = (long long)rr * cols + (in ? cc : 0);
+            const bool ok = in && valid[q] != 0;
+            for (int i = wave; i <= n; i += 4) dst[e * pitch + i] = ok && i < n ? keys[(long long)i * npx + q] : ~0u;
+        }
+    };
+    stage(own, r, c0, 64);
+    int cnt = 0, word = 0, pos = centre & 31;
+    uint64_t cur = 0;
     for (int dy = 0; dy <= Ny; ++dy) {
         const int rr = r + dy;
-        for (int dx = (dy == 0 ? 0 : -Nx); dx <= Nx; ++dx, ++flat) {
-            if ((flat >> 5) != word) {
-                out[word - fw] = cur;
-                cur = 0u;
-                word = flat >> 5;
-            }
-            const int cc = c + dx;
-            if (!pv || rr >= rows || cc < 0 || cc >= cols) continue;
-            const long long q = (long long)rr * cols + cc;
-            if (!valid[q]) continue;
-            bool similar = true;
-            if (q != p) {
-                // own tag: KS2 0; AD2 1 (the pixel is the test's first sample)
-                const uint32_t tp = AD2 ? 1u : 0u, tq = tp ^ 1u;
-                uint32_t S[2 * NP];
+        for (int dx0 = dy == 0 ? 0 : -Nx; dx0 <= Nx; dx0 += kWalkStrip) {
+            const int w = min(kWalkStrip, Nx - dx0 + 1);
+            if (rr < rows) stage(oth, rr, c0 + dx0, 64 + w - 1);
+            __syncthreads();
+            uint32_t bits = 0u;
+            if (rr < rows)
+                for (int k0 = wave; k0 < w; k0 += 8) {
+                    const uint32_t *pa[2], *pb[2];
+                    uint32_t x[2], y[2];
+                    int dd[2] = {0, 0};
+                    double S[2] = {0.0, 0.0};
+                    bool there[2];
 #pragma unroll
-                for (int i = 0; i < NP; ++i) {
-                    S[i] = A[i] | tp;
-                    S[2 * NP - 1 - i] = (i < n ? (keys[i * npx + q] << 1) : 0xFFFFFFFEu) | tq;
-                }
+                    for (int u = 0; u < 2; ++u) {
+                        const int k = k0 + 4 * u < w ? k0 + 4 * u : k0;   // (once more where there is no second)
+                        pa[u] = own + lane * pitch;
+                        pb[u] = oth + (lane + k) * pitch;
+                        x[u] = *pa[u];
+                        y[u] = *pb[u];
+                        there[u] = y[u] != ~0u && x[u] != ~0u;
+                        // for a neighbour that is not there, the pixel's run twice (if
+                        // that is not there either, words of other runs: not used)
+                        if (!there[u]) pb[u] = pa[u], y[u] = x[u];
+                    }
+                    const double* row = T;
+                    for (int b = 1; b < 2 * n; ++b) {
+                        const int odd = b & 1;
 #pragma unroll
-                for (int s = NP; s >= 1; s >>= 1)
-#pragma unroll
-                    for (int i = 0; i < 2 * NP; ++i)
-                        if ((i & s) == 0) {
-                            const uint32_t x = S[i], y = S[i + s];
-                            S[i] = min(x, y);
-                            S[i + s] = max(x, y);
+                        for (int u = 0; u < 2; ++u) {
+                            const bool take_a = x[u] < y[u];
+                            pa[u] += take_a ? 1 : 0;
+                            pb[u] += take_a ? 0 : 1;
+                            const uint32_t v = *(take_a ? pa[u] : pb[u]);
+                            x[u] = take_a ? v : x[u];
+                            y[u] = take_a ? y[u] : v;
+                            dd[u] += take_a ? 1 : -1;
+                            S[u] = S[u] + row[(abs(dd[u]) - odd) >> 1];
                         }
-                if constexpr (AD2) {
-                    // first sample = tag 1
-                    int m = 0;
-                    double Ssum = 0.0;
-#pragma unroll
-                    for (int j = 0; j < 2 * NP - 1; ++j) {
-                        m += (int)(S[j] & 1u);
-                        if (j < 2 * n - 1) Ssum = Ssum + P.d_ad2[j * (n + 1) + m];
+                        row += ad2_row_terms(n, b);
                     }
-                    similar = ad2_standardise(Ssum, n, P.ad2_sigma) <= P.ad2_max;
-                } else {
-                    // d_j = 2 (#tag-1 in the first j+1) - (j+1), taken where
-                    // the amplitude changes (the end of a run of ties).
-                    // Padding keys sort above every amplitude and differ from
-                    // one another only in the tag, so no end falls among them,
-                    // and at the last amplitude d = 0: j needs no bound.
-                    int nb = 0, hi = 0, lo = 0;
 #pragma unroll
-                    for (int j = 0; j < 2 * NP - 1; ++j) {
-                        nb += (int)(S[j] & 1u);
-                        const bool end = (S[j] ^ S[j + 1]) > 1u;
-                        const int x = end ? 2 * nb - (j + 1) : 0;
-                        hi = max(hi, x);
-                        lo = min(lo, x);
-                    }
-                    similar = ks_similar(max(hi, -lo), P);
+                    for (int u = 0; u < 2; ++u)
+                        if (there[u] && k0 + 4 * u < w && ad2_standardise(S[u], n, P.ad2_sigma) <= P.ad2_max)
+                            bits |= 1u << (k0 + 4 * u);
                 }
-            }
-            if (similar) {
-                cur |= (1u << (flat & 31));
-                ++cnt;
+            part[tid] = bits;
+            __syncthreads();   // the strip's reads are over, too
+            bits = pv ? part[lane] | part[64 + lane] | part[128 + lane] | part[192 + lane] : 0u;
+            if (dy == 0 && dx0 == 0) bits |= pv ? 1u : 0u;   // the pixel itself
+            cnt += __popc(bits);
+            cur |= (uint64_t)bits << pos;
+            pos += w;
+            if (pos >= 32) {
+                if (here && wave == 0) out[word * plane] = (uint32_t)cur;
+                ++word;
+                cur >>= 32;
+                pos -= 32;
             }
         }
     }
-    out[word - fw] = cur;
-    for (int w = word + 1; w < nul; ++w) out[w - fw] = 0u;
-    fcnt[t] = cnt;
-}
-
-// n > 64: one thread per output pixel walks the sorted arrays in memory.
-// The reference sweeps half the window and tests (p, q) with p first for
-// q = p + (dy, dx), dy > 0 or dy = 0 < dx (nmap.cpp:402-457); the other half
-// of a pixel's window is therefore tested with the neighbour first.
-template <bool AD2>
-__global__ __launch_bounds__(256) void nmap_sweep(const NmapPlan P, uint32_t* __restrict__ F,
-                                                  int32_t* __restrict__ fcnt) {
-    const float* __restrict__ amp_sorted = P.d_amp;
-    const uint8_t* __restrict__ valid = P.d_valid;
-    const int n = P.n, rows = P.rows, cols = P.cols, Nx = P.Nx, Ny = P.Ny, nul = P.nul;
-    const long long npx = (long long)rows * cols;
-    const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    const int h0 = fwd_row0(P);
-    if (t >= (long long)(P.row_end - h0) * cols) return;
-    const int r = h0 + (int)(t / cols);
-    const int c = (int)(t % cols);
-    const long long p = (long long)r * cols + c;
-    const int centre = centre_flat(P), fw = centre >> 5, nf = nul - fw;
-    uint32_t* out = F + t * nf;   // word w of the mask at out[w - fw]
-    const bool pv = valid[p] != 0;
-    const float* a = amp_sorted + p;
-    // Window positions are visited in bit order (flat = centre, centre + 1,
-    // ...), so the word being filled only ever advances by one; each
-    // finished word is stored once.
-    int cnt = 0, word = fw, flat = centre;
-    uint32_t cur = 0u;
-    for (int dy = 0; dy <= Ny; ++dy) {
-        const int rr = r + dy;
-        for (int dx = (dy == 0 ? 0 : -Nx); dx <= Nx; ++dx, ++flat) {
-            if ((flat >> 5) != word) {
-                out[word - fw] = cur;
-                cur = 0u;
-                word = flat >> 5;
-            }
-            const int cc = c + dx;
-            if (!pv || rr >= rows || cc < 0 || cc >= cols) continue;
-            const long long q = (long long)rr * cols + cc;
-            if (!valid[q]) continue;
-            bool similar = true;
-            if (q != p) {
-                const float* b = amp_sorted + q;
-                if constexpr (AD2) {   // the pixel is the test's first sample
-                    const double S = ad2_inner(a, b, n, npx, P.d_ad2);
-                    similar = ad2_standardise(S, n, P.ad2_sigma) <= P.ad2_max;
-                } else {
-                    similar = ks_similar(ks_count(a, b, n, npx), P);
-                }
-            }
-            if (similar) {
-                cur |= (1u << (flat & 31));
-                ++cnt;
-            }
+    if (here && wave == 0) {
+        for (; word < nf; ++word) {
+            out[word * plane] = (uint32_t)cur;
+            cur = 0;
         }
+        fcnt[(long long)(r - h0) * cols + c] = cnt;
     }
-    out[word - fw] = cur;
-    for (int w = word + 1; w < nul; ++w) out[w - fw] = 0u;
-    fcnt[t] = cnt;
 }
 
 // Full masks of the output rows.  Backward position flat (< centre) of
@@ -356,7 +377,7 @@ __global__ __launch_bounds__(256) void nmap_mirror(const NmapPlan P, const uint3
     const int h0 = fwd_row0(P);
     const int centre = centre_flat(P), fw = centre >> 5, nf = nul - fw;
     const int last = (2 * Ny + 1) * (2 * Nx + 1) - 1;
-    const long long fp = (long long)(r - h0) * cols + c;
+    const long long plane = (long long)(P.row_end - h0) * cols, fp = (long long)(r - h0) * cols + c;
     uint32_t* out = wts + ((long long)r * cols + c) * nul;
     int cnt = fcnt[fp];
     int word = 0, flat = 0;
@@ -372,7 +393,7 @@ __global__ __launch_bounds__(256) void nmap_mirror(const NmapPlan P, const uint3
             const int cc = c + dx;
             if (rr < 0 || cc < 0 || cc >= cols) continue;
             const int mf = last - flat;
-            const uint32_t qw = F[((long long)(rr - h0) * cols + cc) * nf + (mf >> 5) - fw];
+            const uint32_t qw = F[((mf >> 5) - fw) * plane + (long long)(rr - h0) * cols + cc];
             if ((qw >> (mf & 31)) & 1u) {
                 cur |= (1u << (flat & 31));
                 ++cnt;
@@ -384,9 +405,9 @@ __global__ __launch_bounds__(256) void nmap_mirror(const NmapPlan P, const uint3
         out[word] = cur;
         cur = 0u;
     }
-    const uint32_t* mine = F + fp * nf;
+    const uint32_t* mine = F + fp;
     out[fw] = cur | mine[0];
-    for (int i = 1; i < nf; ++i) out[fw + i] = mine[i];
+    for (int i = 1; i < nf; ++i) out[fw + i] = mine[i * plane];
     count[(long long)r * cols + c] = cnt;
 }
 
@@ -400,10 +421,11 @@ static void launch_prep(const NmapPlan& P, const float2* slc, const uint8_t* mas
     hipLaunchKernelGGL(nmap_prep<NP>, dim3((unsigned)blocks), dim3(threads), 0, s, P, slc, mask);
 }
 
-template <int NP>
-static void launch_net(bool ad2, dim3 g, dim3 blk, const NmapPlan& P, hipStream_t s) {
-    if (ad2) hipLaunchKernelGGL((nmap_net<NP, true>), g, blk, 0, s, P, P.d_fwd, P.d_fcnt);
-    else hipLaunchKernelGGL((nmap_net<NP, false>), g, blk, 0, s, P, P.d_fwd, P.d_fcnt);
+template <int CH> static void launch_ks(const NmapPlan& P, int fwd_rows, hipStream_t s) {
+    // the fewest workgroups of at most four waves, of the fewest waves
+    const int waves = (P.cols + 63) / 64, blocks = (waves + 3) / 4, per = (waves + blocks - 1) / blocks;
+    hipLaunchKernelGGL(nmap_ks<CH>, dim3((unsigned)blocks * (unsigned)fwd_rows), dim3(64 * per), 0, s, P, blocks, P.d_fwd,
+                       P.d_fcnt);
 }
 
 int nmap_launch(const NmapPlan& P, const float2* slc, const uint8_t* mask, uint32_t* wts,
@@ -421,20 +443,27 @@ int nmap_launch(const NmapPlan& P, const float2* slc, const uint8_t* mask, uint3
         const int threads = 256;
         // forward halves of the output rows and of the Ny rows above them
         const int h0 = P.row_begin - P.Ny > 0 ? P.row_begin - P.Ny : 0;
-        const long long nfwd = (long long)(P.row_end - h0) * P.cols;
         StageScope sc(STAGE_NMAP_KS, s);
-        if (P.method == 1) {
-            const int nt = (2 * P.n - 1) * (P.n + 1);
+        if (P.method == 0) {
+            // chunks of at most 32 dates, alike and padded to quads
+            const int chunks = (P.n + 31) / 32, quads = ((P.n + chunks - 1) / chunks + 3) / 4;
+            const int fr = P.row_end - h0;
+            switch (quads) {
+                case 1: launch_ks<4>(P, fr, s); break;
+                case 2: launch_ks<8>(P, fr, s); break;
+                case 3: launch_ks<12>(P, fr, s); break;
+                case 4: launch_ks<16>(P, fr, s); break;
+                case 5: launch_ks<20>(P, fr, s); break;
+                case 6: launch_ks<24>(P, fr, s); break;
+                case 7: launch_ks<28>(P, fr, s); break;
+                default: launch_ks<32>(P, fr, s); break;
+            }
+        } else {
+            const int nt = (2 * P.n - 1) * (P.n + 1), blocks = (P.cols + 63) / 64;
             hipLaunchKernelGGL(ad2_terms, dim3((nt + 255) / 256), dim3(256), 0, s, P.d_ad2, P.n);
+            hipLaunchKernelGGL(nmap_walk, dim3((unsigned)blocks * (unsigned)(P.row_end - h0)), dim3(256),
+                               ad2_walk_bytes(P.n), s, P, blocks, P.d_fwd, P.d_fcnt);
         }
-        const bool ad2 = P.method == 1;
-        const dim3 g((unsigned)((nfwd + threads - 1) / threads)), blk(threads);
-        if (P.n <= 8) launch_net<8>(ad2, g, blk, P, s);
-        else if (P.n <= 16) launch_net<16>(ad2, g, blk, P, s);
-        else if (P.n <= 32) launch_net<32>(ad2, g, blk, P, s);
-        else if (P.n <= 64) launch_net<64>(ad2, g, blk, P, s);
-        else if (ad2) hipLaunchKernelGGL(nmap_sweep<true>, g, blk, 0, s, P, P.d_fwd, P.d_fcnt);
-        else hipLaunchKernelGGL(nmap_sweep<false>, g, blk, 0, s, P, P.d_fwd, P.d_fcnt);
         hipLaunchKernelGGL(nmap_mirror, dim3((unsigned)((nout + threads - 1) / threads)), dim3(threads), 0, s,
                            P, (const uint32_t*)P.d_fwd, (const int32_t*)P.d_fcnt, wts, count);
     }
