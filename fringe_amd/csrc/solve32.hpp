@@ -78,11 +78,14 @@ struct OpAdd { template <typename T> __device__ static T f(T a, T b) { return a 
 struct OpMax { template <typename T> __device__ static T f(T a, T b) { return max(a, b); } };
 struct OpMin { template <typename T> __device__ static T f(T a, T b) { return min(a, b); } };
 
-template <typename Op> __device__ __forceinline__ float red32(float x) {
+template <typename Op> __device__ __forceinline__ float red16(float x) {   // (the 16-lane rows alone)
     x = Op::f(x, __uint_as_float(dpp32<0xB1>(__float_as_uint(x))));
     x = Op::f(x, __uint_as_float(dpp32<0x4E>(__float_as_uint(x))));
     x = Op::f(x, __uint_as_float(dpp32<0x141>(__float_as_uint(x))));
-    x = Op::f(x, __uint_as_float(dpp32<0x140>(__float_as_uint(x))));
+    return Op::f(x, __uint_as_float(dpp32<0x140>(__float_as_uint(x))));
+}
+template <typename Op> __device__ __forceinline__ float red32(float x) {
+    x = red16<Op>(x);
     const auto s = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
     return Op::f(__uint_as_float(s[0]), __uint_as_float(s[1]));
 }
@@ -91,11 +94,14 @@ template <int CTRL> __device__ __forceinline__ double dpp64(double v) {
     const uint32_t lo = dpp32<CTRL>((uint32_t)u), hi = dpp32<CTRL>((uint32_t)(u >> 32));
     return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
 }
-template <typename Op> __device__ __forceinline__ double red32(double x) {
+template <typename Op> __device__ __forceinline__ double red16(double x) {
     x = Op::f(x, dpp64<0xB1>(x));
     x = Op::f(x, dpp64<0x4E>(x));
     x = Op::f(x, dpp64<0x141>(x));
-    x = Op::f(x, dpp64<0x140>(x));
+    return Op::f(x, dpp64<0x140>(x));
+}
+template <typename Op> __device__ __forceinline__ double red32(double x) {
+    x = red16<Op>(x);
     const uint64_t u = __builtin_bit_cast(uint64_t, x);
     const auto lo = __builtin_amdgcn_permlane16_swap((uint32_t)u, (uint32_t)u, false, false);
     const auto hi = __builtin_amdgcn_permlane16_swap((uint32_t)(u >> 32), (uint32_t)(u >> 32), false, false);

@@ -1,19 +1,19 @@
 // solve_mfma.hip -- launcher of the matrix-core estimator chain (mixed
-// precisions, up to 128 dates): one wave per pixel up to 32 dates, one
-// workgroup of a wave per 32 dates above.
+// precisions, up to 128 dates): one wave per pixel on a 16 x 16 tile up to 16
+// dates and a 32 x 32 tile up to 32, one workgroup of a wave per 32 dates above.
 #include "solve_mfma_wg.hpp"
 
 namespace fringe {
 
-static void launch_wave(const SolveArgs& a, hipStream_t s) {
+template <int DIM> static void launch_wave(const SolveArgs& a, hipStream_t s) {
     constexpr int WPB = 4;
     const dim3 grid((unsigned)((a.slots + WPB - 1) / WPB)), block(64 * WPB);
     if (a.module == FRINGE_MODULE_PHASE_LINK)
-        hipLaunchKernelGGL((solve_mfma_kernel<MODE_EMI, WPB>), grid, block, 0, s, a);
+        hipLaunchKernelGGL((solve_mfma_kernel<MODE_EMI, DIM, WPB>), grid, block, 0, s, a);
     else if (a.method == FRINGE_METHOD_MLE)
-        hipLaunchKernelGGL((solve_mfma_kernel<MODE_MLE, WPB>), grid, block, 0, s, a);
+        hipLaunchKernelGGL((solve_mfma_kernel<MODE_MLE, DIM, WPB>), grid, block, 0, s, a);
     else
-        hipLaunchKernelGGL((solve_mfma_kernel<MODE_EVD, WPB>), grid, block, 0, s, a);
+        hipLaunchKernelGGL((solve_mfma_kernel<MODE_EVD, DIM, WPB>), grid, block, 0, s, a);
 }
 
 template <int NT> static void launch_wg(const SolveArgs& a, hipStream_t s) {
@@ -32,7 +32,8 @@ void launch_solve_mfma(const SolveArgs& args, hipStream_t s) {
     if (a.n > 96) launch_wg<4>(a, s);
     else if (a.n > 64) launch_wg<3>(a, s);
     else if (a.n > 32) launch_wg<2>(a, s);
-    else launch_wave(a, s);
+    else if (a.n > 16) launch_wave<32>(a, s);
+    else launch_wave<16>(a, s);
 }
 
 }  // namespace fringe

@@ -32,8 +32,12 @@
 // per SIMD measured the same).  At 30 dates a pixel takes 2.34 k vector
 // instructions and 135 MFMAs, against 9.2 k vector instructions in the
 // tridiagonalising two-pixel solver it replaced.  Solve stage of a 2048 x
-// 2048 tile at 30 dates (EMI): 67.5 ms before, 29.6 ms now; of a 640 x 640
+// 2048 tile at 30 dates (EMI): 67.5 ms before, 29.5 ms now; of a 640 x 640
 // tile at 20 dates (MLE): 7.4 ms before, 2.9 ms now.
+//
+// Up to 16 dates the same chain runs on one 16 x 16 tile (four registers a
+// matrix instead of sixteen, 16x16x4 MFMAs that take two pivots each): 256 x
+// 256 pixels of 10 dates (EVD) 0.21 -> 0.14 ms, 64 x 64 of 8 0.020 -> 0.015.
 #pragma once
 #include "link_solve.hpp"
 #include "solve32.hpp"
@@ -53,11 +57,24 @@ typedef double mf64x4 __attribute__((ext_vector_type(4)));
 // the tolerance, with C = 0.5 and C = 1.25.
 constexpr float kCertScaleEmi = 1.0e3f, kCertScaleEvd = 2.5e3f;
 
-struct LdsMfma32 {
-    static constexpr int S = 36;   // row stride of T: 16-byte rows of four, spread over the banks
-    float T[32 * S];   // |Gamma|^-1, row-major
-    float xr[32], xi[32];
-    cx<float> o[32];
+// Accumulator of a DIM x DIM matrix: NV registers, lane l holds column l % DIM
+// and, with h = l / DIM, rows row(v, h).
+template <int DIM> struct Acc;
+template <> struct Acc<32> {
+    typedef mf32x16 type;
+    static constexpr int NV = 16;
+    static __device__ __forceinline__ constexpr int row(int v, int h) { return 8 * (v / 4) + 4 * h + v % 4; }
+};
+template <> struct Acc<16> {
+    typedef float type __attribute__((ext_vector_type(4)));
+    static constexpr int NV = 4;
+    static __device__ __forceinline__ constexpr int row(int v, int h) { return 4 * h + v; }
+};
+
+template <int DIM> struct LdsMfma {
+    static constexpr int S = DIM + 4;   // row stride of T: 16-byte rows of four, spread over the banks
+    float T[DIM * S];   // |Gamma|^-1, row-major
+    float xr[DIM], xi[DIM];
 };
 
 __device__ __forceinline__ float lane_f32(float x, int lane) {
@@ -136,10 +153,68 @@ __device__ __forceinline__ void sweep32(mf32x16& R, mf32x16& I, int n, int lane,
         }
 }
 
-// x of the 16 rows a lane's registers hold (rows 8 a + 4 h + b), from LDS
-__device__ __forceinline__ void row_values(const LdsMfma32& L, int h, float (&xr)[16], float (&xi)[16]) {
+// The same for a matrix of 16 x 16, by pairs of pivots 8 rows apart: a swap of
+// 16-lane rows puts (re | im) of the two pivot rows into the four k of one
+// 16x16x4 MFMA.  With D the pivots' 2 x 2 block, W = D^-1 times the rows is a
+// combination of the lane's own word, the other row's and the other row's
+// other part.
+__device__ __forceinline__ void sweep32(Acc<16>::type& R, Acc<16>::type& I, int n, int lane, int& neg, int& near) {
+    neg = 0;
+    near = 0x7fffffff;
+    const uint32_t odd = (lane & 16) << 27;                          // the imaginary parts' lanes
+    const uint32_t gam = lane < 16 || lane >= 48 ? 0x80000000u : 0u;
 #pragma unroll
-    for (int a = 0; a < 4; ++a) {
+    for (int v = 0; v < 4; ++v)
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            const int p0 = v + 4 * s, p1 = p0 + 8;
+            if (p0 < fresh(n)) {
+                const float r = R[v], i = I[v];
+                const float d00 = lane_f32(r, 16 * s + p0) + 1.0f, d11 = lane_f32(r, 16 * (s + 2) + p1) + 1.0f;
+                const float x = lane_f32(r, 16 * s + p1), y = lane_f32(i, 16 * s + p1);
+                const float det = fmaf(-x, x, fmaf(-y, y, d00 * d11));
+                const float rd = __builtin_amdgcn_rcpf(det);
+                const int pa = __builtin_amdgcn_readfirstlane(__float_as_int(d00 - 1.0f));
+                const int pb = __builtin_amdgcn_readfirstlane(__float_as_int(fmaf(det, __builtin_amdgcn_rcpf(d00), -1.0f)));
+                neg += ((uint32_t)pa < 0xBF800000u ? 0 : 1) + ((uint32_t)pb < 0xBF800000u ? 0 : 1);
+                near = min(near, min(abs(pa - (int)0xBF800000), abs(pb - (int)0xBF800000)));
+                const auto bb = __builtin_amdgcn_permlane16_swap(__float_as_uint(r), __float_as_uint(i), false, false);
+                const auto cc = __builtin_amdgcn_permlane16_swap(__float_as_uint(i), __float_as_uint(r), false, false);
+                const float b = __uint_as_float(bb[s]), c = __uint_as_float(cc[s]);
+                float lo, hi;
+                swap32(b, b, lo, hi);
+                const float bo = lane < 32 ? hi : lo;   // the other pivot's row
+                swap32(c, c, lo, hi);
+                const float co = lane < 32 ? hi : lo;   // its other part
+                const float al = (lane < 32 ? d11 : d00) * -rd;
+                const float ga = __uint_as_float(__float_as_uint(y * rd) ^ gam);
+                const float a = fmaf(al, b, fmaf(x * rd, bo, ga * co));
+                const float d = __uint_as_float(__float_as_uint(a) ^ odd);
+                R = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, R, 0, 0, 0);
+                I = __builtin_amdgcn_mfma_f32_16x16x4f32(d, c, I, 0, 0, 0);
+            }
+        }
+}
+
+// Over a column's lanes, result in all of them; over the row groups of lanes.
+template <int DIM, typename Op, typename T> __device__ __forceinline__ T redC(T x) {
+    if constexpr (DIM == 32) return red32<Op>(x);
+    else return red16<Op>(x);
+}
+template <int DIM> __device__ __forceinline__ float sumH(float x) {
+    if constexpr (DIM == 16) {
+        const auto s = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+        x = __uint_as_float(s[0]) + __uint_as_float(s[1]);
+    }
+    return both32(x);
+}
+
+// x of the rows a lane's registers hold, from LDS
+template <int DIM>
+__device__ __forceinline__ void row_values(const LdsMfma<DIM>& L, int h, float (&xr)[Acc<DIM>::NV],
+                                           float (&xi)[Acc<DIM>::NV]) {
+#pragma unroll
+    for (int a = 0; a < Acc<DIM>::NV / 4; ++a) {
         const float4 p = *(const float4*)&L.xr[8 * a + 4 * h];
         const float4 q = *(const float4*)&L.xi[8 * a + 4 * h];
         xr[4 * a] = p.x; xr[4 * a + 1] = p.y; xr[4 * a + 2] = p.z; xr[4 * a + 3] = p.w;
@@ -147,26 +222,28 @@ __device__ __forceinline__ void row_values(const LdsMfma32& L, int h, float (&xr
     }
 }
 
-// y = M x for Hermitian (R, I): component c of x and y in lanes c, c + 32
-__device__ __forceinline__ cx<float> apply32(LdsMfma32& L, const mf32x16& R, const mf32x16& I, cx<float> x, int col,
-                                             int h) {
+// y = M x for Hermitian (R, I): component c of x and y in lanes c, c + DIM, ...
+template <int DIM>
+__device__ __forceinline__ cx<float> apply32(LdsMfma<DIM>& L, const typename Acc<DIM>::type& R,
+                                             const typename Acc<DIM>::type& I, cx<float> x, int col, int h) {
+    constexpr int NV = Acc<DIM>::NV;
     if (h == 0) {
         L.xr[col] = x.re;
         L.xi[col] = x.im;
     }
     wsync();
-    float xr[16], xi[16];
-    row_values(L, h, xr, xi);
+    float xr[NV], xi[NV];
+    row_values<DIM>(L, h, xr, xi);
     float re[2] = {0.0f, 0.0f}, im[2] = {0.0f, 0.0f};
 #pragma unroll
-    for (int v = 0; v < 16; ++v) {   // conj(M_rc) x_r
+    for (int v = 0; v < NV; ++v) {   // conj(M_rc) x_r
         re[v & 1] = fmaf(R[v], xr[v], re[v & 1]);
         im[v & 1] = fmaf(R[v], xi[v], im[v & 1]);
         re[v & 1] = fmaf(I[v], xi[v], re[v & 1]);
         im[v & 1] = fmaf(-I[v], xr[v], im[v & 1]);
     }
     wsync();
-    return cx<float>{both32(re[0] + re[1]), both32(im[0] + im[1])};
+    return cx<float>{sumH<DIM>(re[0] + re[1]), sumH<DIM>(im[0] + im[1])};
 }
 
 // One pixel's n x n coherence through a buffer descriptor: its bounds check
@@ -186,10 +263,12 @@ struct GammaBuf {
 };
 
 // Gamma in the accumulator layout; rows and columns >= n read as zero
-__device__ __forceinline__ void load_gamma32(const GammaBuf& gam, int n, int col, int h, mf32x16& R, mf32x16& I) {
+template <int DIM>
+__device__ __forceinline__ void load_gamma32(const GammaBuf& gam, int n, int col, int h, typename Acc<DIM>::type& R,
+                                             typename Acc<DIM>::type& I) {
     int o = fresh_lane(gam.offset(4 * h, col));   // (offsets are not worth registers from one load to the next)
 #pragma unroll
-    for (int v = 0; v < 16; ++v) {
+    for (int v = 0; v < Acc<DIM>::NV; ++v) {
         const cx<float> g = gam.at(o);
         o += (v % 4 == 3 ? 5 : 1) * n * 8;
         R[v] = g.re;
@@ -213,21 +292,22 @@ constexpr float kSlow = 0.35f;
 constexpr int kNearInside = 1600000;   // |pivot| >= 0.1
 // qb > 0: polishing instead, until the error predicted from the contraction
 // qb that the spectrum allows is below 4e-7.
-__device__ __forceinline__ void iterate32(LdsMfma32& L, const mf32x16& R, const mf32x16& I, int col, int h, float qb,
-                                          EigState& E) {
+template <int DIM>
+__device__ __forceinline__ void iterate32(LdsMfma<DIM>& L, const typename Acc<DIM>::type& R,
+                                          const typename Acc<DIM>::type& I, int col, int h, float qb, EigState& E) {
     float dp = 0.0f;
     if (!(qb > 0.0f)) E.q = E.dq = 0.0f;
     for (int k = qb > 0.0f ? 0 : -2; k < 24; ++k) {
-        const cx<float> y = csub(E.x, apply32(L, R, I, E.x, col, h));
+        const cx<float> y = csub(E.x, apply32<DIM>(L, R, I, E.x, col, h));
         if (k < 0) {
-            const float nr = k < -1 ? 1.0f : __builtin_amdgcn_rsqf(uni(red32<OpAdd>(cabs2(y))));
+            const float nr = k < -1 ? 1.0f : __builtin_amdgcn_rsqf(uni(redC<DIM, OpAdd>(cabs2(y))));
             E.x = cscale(y, nr);
             continue;
         }
-        const float th = uni(red32<OpAdd>(y.re * E.x.re + y.im * E.x.im));
+        const float th = uni(redC<DIM, OpAdd>(y.re * E.x.re + y.im * E.x.im));
         const float it = __builtin_amdgcn_rcpf(th);
         const cx<float> d = {fmaf(y.re, it, -E.x.re), fmaf(y.im, it, -E.x.im)};
-        const float d2 = uni(red32<OpAdd>(cabs2(d)));
+        const float d2 = uni(redC<DIM, OpAdd>(cabs2(d)));
         const float dn = __builtin_amdgcn_sqrtf(d2);
         const float s = __builtin_amdgcn_rsqf(1.0f + d2);
         E.x = cx<float>{(E.x.re + d.re) * s, (E.x.im + d.im) * s};
@@ -261,8 +341,8 @@ __device__ __forceinline__ void iterate32(LdsMfma32& L, const mf32x16& R, const 
 // transposed into (1, 0) through LDS in between: three MFMAs a pair, not
 // four.  Returns whether every pivot was positive; near: a pivot up to the
 // first one that is not positive lay within kCertPivotMin of 0.
-template <int K>
-__device__ __forceinline__ void sweep64_rows(mf64x4 (&M)[2][2], int n, const double (&al)[2], const double (&be)[2],
+template <int K, int NB>
+__device__ __forceinline__ void sweep64_rows(mf64x4 (&M)[NB][NB], int n, const double (&al)[2], const double (&be)[2],
                                              const double (&ga)[2], bool& ok, bool& near) {
 #pragma unroll
     for (int r = 0; r < 4; ++r)
@@ -283,19 +363,22 @@ __device__ __forceinline__ void sweep64_rows(mf64x4 (&M)[2][2], int n, const dou
             // i + 4 block + 16 k, and X and W as they lie in the tiles
             const double num = fma(ga[s / 2], d00, fma(be[s / 2], d01, al[s / 2] * d11));
             const double ca = num * fast_rcp(det);
-            double b[2], w[2];
+            double b[NB], w[NB];
 #pragma unroll
-            for (int J = 0; J < 2; ++J) {
+            for (int J = 0; J < NB; ++J) {
                 b[J] = M[K][J][r];
                 asm("" : "+v"(b[J]));   // its own registers: the tile is overwritten below
                 w[J] = __builtin_amdgcn_mfma_f64_4x4x4f64(ca, b[J], 0.0, 0, 0, 0);
             }
             M[0][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(w[0], b[0], M[0][0], 0, 0, 0);
-            M[K][1 - K] = __builtin_amdgcn_mfma_f64_16x16x4f64(w[K], b[1 - K], M[K][1 - K], 0, 0, 0);
-            M[1][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(w[1], b[1], M[1][1], 0, 0, 0);
+            if constexpr (NB == 2) {
+                M[K][1 - K] = __builtin_amdgcn_mfma_f64_16x16x4f64(w[K], b[1 - K], M[K][1 - K], 0, 0, 0);
+                M[1][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(w[1], b[1], M[1][1], 0, 0, 0);
+            }
         }
 }
-__device__ __forceinline__ bool sweep64(LdsMfma32& L, mf64x4 (&M)[2][2], int n, int lane, bool& near) {
+template <int DIM>
+__device__ __forceinline__ bool sweep64(LdsMfma<DIM>& L, mf64x4 (&M)[DIM / 16][DIM / 16], int n, int lane, bool& near) {
     bool ok = true;
     near = false;
     const int q = lane >> 4, i = lane & 3;
@@ -307,8 +390,8 @@ __device__ __forceinline__ bool sweep64(LdsMfma32& L, mf64x4 (&M)[2][2], int n, 
         ga[k] = i == s + 1 && q == s + 1 ? -1.0 : 0.0;
         be[k] = (i == s && q == s + 1) || (i == s + 1 && q == s) ? 1.0 : 0.0;
     }
-    sweep64_rows<0>(M, n, al, be, ga, ok, near);
-    if (n > 16) {
+    sweep64_rows<0, DIM / 16>(M, n, al, be, ga, ok, near);
+    if constexpr (DIM == 32) {
         double* X = (double*)L.T;   // 16 x 16, rows 17 apart
 #pragma unroll
         for (int r = 0; r < 4; ++r) X[(4 * r + q) * 17 + (lane & 15)] = M[0][1][r];
@@ -316,21 +399,22 @@ __device__ __forceinline__ bool sweep64(LdsMfma32& L, mf64x4 (&M)[2][2], int n, 
 #pragma unroll
         for (int r = 0; r < 4; ++r) M[1][0][r] = X[(lane & 15) * 17 + 4 * r + q];
         wsync();
-        sweep64_rows<1>(M, n, al, be, ga, ok, near);
+        sweep64_rows<1, 2>(M, n, al, be, ga, ok, near);
     }
     return ok;
 }
 
 // |Gamma| into the FP64 tiles (diagonal stored minus 1 = 0, also in the
 // padding); false when an entry is not finite.
-__device__ __forceinline__ bool load_abs64(const GammaBuf& gam, int n, int lane, mf64x4 (&M)[2][2]) {
+template <int NB>
+__device__ __forceinline__ bool load_abs64(const GammaBuf& gam, int n, int lane, mf64x4 (&M)[NB][NB]) {
     float sum = 0.0f;
     const int o0 = gam.offset(lane >> 4, lane & 15), o1 = gam.offset(lane >> 4, 16 + (lane & 15));
     const int dr = (lane & 15) - (lane >> 4);   // 4 r on the diagonal
 #pragma unroll
-    for (int K = 0; K < 2; ++K)
+    for (int K = 0; K < NB; ++K)
 #pragma unroll
-        for (int J = 0; J < 2; ++J)
+        for (int J = 0; J < NB; ++J)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const cx<float> g = gam.at((J ? o1 : o0) + (16 * K + 4 * r) * n * 8);
@@ -343,27 +427,34 @@ __device__ __forceinline__ bool load_abs64(const GammaBuf& gam, int n, int lane,
 }
 
 // I - M -> |Gamma|^-1 in FP32 rows in LDS (tile (0, 1) from (1, 0))
-__device__ __forceinline__ void inverse_to_lds(LdsMfma32& L, const mf64x4 (&M)[2][2], int lane) {
+template <int DIM>
+__device__ __forceinline__ void inverse_to_lds(LdsMfma<DIM>& L, const mf64x4 (&M)[DIM / 16][DIM / 16], int lane) {
+    constexpr int S = LdsMfma<DIM>::S;
     const int q = lane >> 4, c = lane & 15, dr = c - q;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
         const int row = 4 * r + q;
         const double one = dr == 4 * r ? 1.0 : 0.0;
-        L.T[row * LdsMfma32::S + c] = (float)(one - M[0][0][r]);
-        L.T[(16 + row) * LdsMfma32::S + 16 + c] = (float)(one - M[1][1][r]);
-        const float m = -(float)M[1][0][r];
-        L.T[(16 + row) * LdsMfma32::S + c] = m;
-        L.T[c * LdsMfma32::S + 16 + row] = m;
+        L.T[row * S + c] = (float)(one - M[0][0][r]);
+        if constexpr (DIM == 32) {
+            L.T[(16 + row) * S + 16 + c] = (float)(one - M[1][1][r]);
+            const float m = -(float)M[1][0][r];
+            L.T[(16 + row) * S + c] = m;
+            L.T[c * S + 16 + row] = m;
+        }
     }
 }
 
 // One pixel on the 64 lanes of a wave.
-template <int MODE>
-__device__ __forceinline__ void solve_mfma_pixel(const SolveArgs& a, LdsMfma32& L, int lane, int np,
+template <int MODE, int DIM>
+__device__ __forceinline__ void solve_mfma_pixel(const SolveArgs& a, LdsMfma<DIM>& L, int lane, int np,
                                                  const GammaBuf& gam, long long pix) {
-    const int n = a.n, col = lane & 31, h = lane >> 5;
+    typedef typename Acc<DIM>::type acc;
+    constexpr int NV = Acc<DIM>::NV, S = LdsMfma<DIM>::S;
+    const int n = a.n, col = lane & (DIM - 1), h = lane / DIM;
     const bool in = col < n;
-    const int vd0 = ((col >> 2) & 1) == h ? 4 * (col >> 3) + (col & 3) : -1;   // register of this lane's diagonal entry
+    // register of this lane's diagonal entry
+    const int vd0 = ((col >> 2) & (64 / DIM - 1)) == h ? (DIM == 32 ? 4 * (col >> 3) : 0) + (col & 3) : -1;
     const bool stbas = a.method == FRINGE_METHOD_STBAS && MODE == MODE_EVD;
     float code = 0.0f;
     bool unc = false;
@@ -376,12 +467,12 @@ __device__ __forceinline__ void solve_mfma_pixel(const SolveArgs& a, LdsMfma32& 
         if constexpr (MODE == MODE_MLE) {
             // smallest eigenvalue of Gamma at least 1e-6, by a margin
             // (Gamma has unit diagonal: its norm is at most n)
-            mf32x16 R, I;
-            load_gamma32(gam, n, col, h, R, I);
+            acc R, I;
+            load_gamma32<DIM>(gam, n, col, h, R, I);
             const float s = 1.0e-6f + kCertThrMargin * Lim<float>::eps() * (float)n;
             float sum = 0.0f;
 #pragma unroll
-            for (int v = 0; v < 16; ++v) {
+            for (int v = 0; v < NV; ++v) {
                 sum += fabsf(R[v]) + fabsf(I[v]);
                 if (v == vd0) R[v] = -s;   // 1 - s, stored minus 1
             }
@@ -396,22 +487,22 @@ __device__ __forceinline__ void solve_mfma_pixel(const SolveArgs& a, LdsMfma32& 
         }
         if constexpr (MODE != MODE_EVD) {
             if (code == 0.0f && !unc) {
-                mf64x4 M[2][2];
-                const bool fin = load_abs64(gam, n, lane, M);
+                mf64x4 M[DIM / 16][DIM / 16];
+                const bool fin = load_abs64<DIM / 16>(gam, n, lane, M);
                 if (!fin) {
                     code = -1.0f;
                 } else {
                     bool near;
-                    const bool pd = sweep64(L, M, n, lane, near);
+                    const bool pd = sweep64<DIM>(L, M, n, lane, near);
                     unc = near;
                     if (MODE == MODE_EMI) inv = pd;   // else the EVD fallback
                     else unc = unc || !pd;
-                    if (inv) inverse_to_lds(L, M, lane);
+                    if (inv) inverse_to_lds<DIM>(L, M, lane);
                     wsync();
                     if constexpr (MODE == MODE_MLE) {
                         // |Gamma| - 1e-6 I is positive definite when its
                         // smallest eigenvalue, at least 1 / trace(inverse), is
-                        const float tr = red32<OpAdd>(in ? L.T[col * LdsMfma32::S + col] : 0.0f);
+                        const float tr = redC<DIM, OpAdd>(in ? L.T[col * S + col] : 0.0f);
                         unc = unc || !(uni(tr) < 1.0e5f);
                     }
                 }
@@ -429,32 +520,32 @@ __device__ __forceinline__ void solve_mfma_pixel(const SolveArgs& a, LdsMfma32& 
         E.x = cx<float>{g.re * w, -g.im * w};
         if (in && !(g2 > 0.0f)) E.x.re = is;
         float sigma = 1.0f, sg = 1.0f, tn = 1.0f;
-        const float dg = inv ? (in ? L.T[col * LdsMfma32::S + col] : 0.0f) : 1.0f;
+        const float dg = inv ? (in ? L.T[col * S + col] : 0.0f) : 1.0f;
         if (!inv) {
             sg = -1.0f;
-            mf32x16 R, I;
-            load_gamma32(gam, n, col, h, R, I);
+            acc R, I;
+            load_gamma32<DIM>(gam, n, col, h, R, I);
             float f2 = 0.0f, sum = 0.0f;
 #pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                if (stbas && abs(8 * (v / 4) + v % 4 - fresh_lane(col - 4 * h)) > a.bw) {
+            for (int v = 0; v < NV; ++v) {
+                if (stbas && abs(Acc<DIM>::row(v, 0) - fresh_lane(col - 4 * h)) > a.bw) {
                     R[v] = 0.0f;
                     I[v] = 0.0f;
                 }
                 f2 = fmaf(R[v], R[v], fmaf(I[v], I[v], f2));
             }
             if constexpr (MODE == MODE_EVD) {
-                sum = uni(both32(red32<OpAdd>(f2)));
+                sum = uni(sumH<DIM>(redC<DIM, OpAdd>(f2)));
                 if (!(sum < 3.0e38f)) code = -6.0f;
             }
             if (code == 0.0f) {
                 float rho = 1.0f, dn = 1.0f;
                 for (int k = 0; k < 3; ++k) {
-                    const cx<float> y = apply32(L, R, I, E.x, col, h);
-                    rho = uni(red32<OpAdd>(y.re * E.x.re + y.im * E.x.im));
+                    const cx<float> y = apply32<DIM>(L, R, I, E.x, col, h);
+                    rho = uni(redC<DIM, OpAdd>(y.re * E.x.re + y.im * E.x.im));
                     const float it = __builtin_amdgcn_rcpf(rho);
                     const cx<float> d = {y.re * it - E.x.re, y.im * it - E.x.im};
-                    dn = uni(red32<OpAdd>(cabs2(d)));
+                    dn = uni(redC<DIM, OpAdd>(cabs2(d)));
                     const float s = __builtin_amdgcn_rsqf(1.0f + dn);
                     E.x = cx<float>{(E.x.re + d.re) * s, (E.x.im + d.im) * s};
                 }
@@ -471,14 +562,14 @@ __device__ __forceinline__ void solve_mfma_pixel(const SolveArgs& a, LdsMfma32& 
             for (int att = 0; att < 6; ++att) {
                 const int vd = fresh_lane(vd0);
                 // ---- B = +-(A - sigma I), diagonal minus 1 ----
-                const float off = sg * (dg - sigma) - 1.0f;
-                mf32x16 R, I;
-                load_gamma32(gam, n, col, h, R, I);
+                const float off = in ? sg * (dg - sigma) - 1.0f : 0.0f;
+                acc R, I;
+                load_gamma32<DIM>(gam, n, col, h, R, I);
                 float f2 = 0.0f;
                 if (inv) {
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        const float4 m = *(const float4*)&L.T[col * LdsMfma32::S + 8 * q + 4 * h];
+                    for (int q = 0; q < NV / 4; ++q) {
+                        const float4 m = *(const float4*)&L.T[col * S + 8 * q + 4 * h];
                         const float mm[4] = {m.x, m.y, m.z, m.w};
 #pragma unroll
                         for (int b = 0; b < 4; ++b) {
@@ -492,18 +583,18 @@ __device__ __forceinline__ void solve_mfma_pixel(const SolveArgs& a, LdsMfma32& 
                     if (att == 0) {
                         // |H| <= m + s sqrt(n - 1) with m the mean and s the
                         // deviation of the eigenvalues (Wolkowicz and Styan)
-                        const float tr = uni(red32<OpAdd>(dg)) * a.inv_n;
-                        const float ff = uni(both32(red32<OpAdd>(f2 + (vd >= 0 ? dg * dg : 0.0f)))) * a.inv_n;
+                        const float tr = uni(redC<DIM, OpAdd>(dg)) * a.inv_n;
+                        const float ff = uni(sumH<DIM>(redC<DIM, OpAdd>(f2 + (vd >= 0 ? dg * dg : 0.0f)))) * a.inv_n;
                         tn = tr + __builtin_amdgcn_sqrtf(fmaxf(ff - tr * tr, 0.0f) * (float)(n - 1));
                         if (!(tn < 3.0e38f)) break;   // H not finite: the FP64 path decides
                     }
                 } else {
 #pragma unroll
-                    for (int v = 0; v < 16; ++v) {
-                        const bool out = stbas && abs(8 * (v / 4) + v % 4 - fresh_lane(col - 4 * h)) > a.bw;
+                    for (int v = 0; v < NV; ++v) {
+                        const bool out = stbas && abs(Acc<DIM>::row(v, 0) - fresh_lane(col - 4 * h)) > a.bw;
                         R[v] = out ? 0.0f : -R[v];
                         I[v] = out ? 0.0f : -I[v];
-                        if (v == vd) R[v] = in ? off : 0.0f;
+                        if (v == vd) R[v] = off;
                     }
                 }
                 int neg;
@@ -518,7 +609,7 @@ __device__ __forceinline__ void solve_mfma_pixel(const SolveArgs& a, LdsMfma32& 
                     else sigma = sigma * 1.15f;
                     continue;
                 }
-                iterate32(L, R, I, col, h, 0.0f, E);
+                iterate32<DIM>(L, R, I, col, h, 0.0f, E);
                 const float mu = __builtin_amdgcn_rcpf(E.theta);
                 lam = sigma + sg * mu;
                 if (!(fabsf(lam) < 3.0e38f)) break;
@@ -532,19 +623,19 @@ __device__ __forceinline__ void solve_mfma_pixel(const SolveArgs& a, LdsMfma32& 
                     continue;
                 }
                 // ---- certification ----
-                const float m2 = red32<OpMin>(in ? cabs2(E.x) : 3.0e38f);
+                const float m2 = redC<DIM, OpMin>(in ? cabs2(E.x) : 3.0e38f);
                 delta = (inv ? kCertScaleEmi : kCertScaleEvd) * Lim<float>::eps() * tn * __builtin_amdgcn_rsqf(uni(m2));
                 if (!(delta <= tn)) break;
                 // Frobenius norm of the inverse: its other eigenvalues'
                 // squares sum to S2, so none of them exceeds sqrt(S2)
                 float f = 0.0f;
 #pragma unroll
-                for (int v = 0; v < 16; ++v) {
+                for (int v = 0; v < NV; ++v) {
                     const float x = v == vd ? 1.0f - R[v] : R[v];
                     f = fmaf(x, x, fmaf(I[v], I[v], f));
                 }
                 if (vd >= 0 && !in) f -= 1.0f;   // padding: R = 0 on the diagonal
-                f = uni(both32(red32<OpAdd>(f)));
+                f = uni(sumH<DIM>(redC<DIM, OpAdd>(f)));
                 const float s2 = fmaxf(f - E.theta * E.theta, 0.0f) + 4.0e-6f * f;
                 const float t = mu + delta;
                 const bool side = neg == 0 ? E.theta > 0.0f : E.theta < 0.0f;
@@ -553,7 +644,7 @@ __device__ __forceinline__ void solve_mfma_pixel(const SolveArgs& a, LdsMfma32& 
                 const float qb = __builtin_amdgcn_sqrtf(s2) * fabsf(mu);
                 bool conv = qb < 0.8f;
                 if (conv && E.dn * qb > 4.0e-7f * (1.0f - qb)) {
-                    iterate32(L, R, I, col, h, qb, E);
+                    iterate32<DIM>(L, R, I, col, h, qb, E);
                     conv = E.done;
                 }
                 // a shift inside the spectrum: small pivots would have cost accuracy
@@ -618,7 +709,7 @@ __device__ __forceinline__ void solve_mfma_pixel(const SolveArgs& a, LdsMfma32& 
         cs.re = (double)(z.x * o.re + z.y * o.im);
         cs.im = (double)(z.y * o.re - z.x * o.im);
     }
-    cs = cx<double>{red32<OpAdd>(cs.re), red32<OpAdd>(cs.im)};
+    cs = cx<double>{redC<DIM, OpAdd>(cs.re), redC<DIM, OpAdd>(cs.im)};
     // ---- temporal coherence (evd.cpp:770-786): sum over i < j (j <= i + bw
     // for STBAS) of exp(i (arg Gamma_ij - arg o_i + arg o_j)) ----
     if (h == 0) {
@@ -626,15 +717,15 @@ __device__ __forceinline__ void solve_mfma_pixel(const SolveArgs& a, LdsMfma32& 
         L.xi[col] = in ? o.im : 0.0f;
     }
     wsync();
-    float xr[16], xi[16];
-    row_values(L, h, xr, xi);
-    mf32x16 R, I;
-    load_gamma32(gam, n, col, h, R, I);
+    float xr[NV], xi[NV];
+    row_values<DIM>(L, h, xr, xi);
+    acc R, I;
+    load_gamma32<DIM>(gam, n, col, h, R, I);
     float tr = 0.0f, ti = 0.0f;
     const int rb = stbas ? col - a.bw : 0;
 #pragma unroll
-    for (int v = 0; v < 16; ++v) {
-        const int row = 8 * (v / 4) + 4 * h + v % 4;
+    for (int v = 0; v < NV; ++v) {
+        const int row = Acc<DIM>::row(v, h);
         float rs = __builtin_amdgcn_rsqf(fmaf(R[v], R[v], I[v] * I[v]));
         rs = row < col ? rs : 0.0f;
         if (stbas && row < rb) rs = 0.0f;
@@ -646,8 +737,8 @@ __device__ __forceinline__ void solve_mfma_pixel(const SolveArgs& a, LdsMfma32& 
         tr = 0.0f;
         ti = 0.0f;
 #pragma unroll
-        for (int v = 0; v < 16; ++v) {
-            const int row = 8 * (v / 4) + 4 * h + v % 4;
+        for (int v = 0; v < NV; ++v) {
+            const int row = Acc<DIM>::row(v, h);
             const float g2 = fmaf(R[v], R[v], I[v] * I[v]);
             const bool use = row < col && !(stbas && row < rb), z = !(g2 > 0.0f);
             const float rs = use ? __builtin_amdgcn_rsqf(g2) : 0.0f;
@@ -661,8 +752,8 @@ __device__ __forceinline__ void solve_mfma_pixel(const SolveArgs& a, LdsMfma32& 
         sr = 0.0f;
         si = 0.0f;
     }
-    sr = both32(red32<OpAdd>(sr));
-    si = both32(red32<OpAdd>(si));
+    sr = sumH<DIM>(redC<DIM, OpAdd>(sr));
+    si = sumH<DIM>(redC<DIM, OpAdd>(si));
     if (lane == 0) {
         // |sum| / pairs in double: rsq refined by one Newton step
         const double s2 = (double)sr * (double)sr + (double)si * (double)si;
@@ -675,15 +766,15 @@ __device__ __forceinline__ void solve_mfma_pixel(const SolveArgs& a, LdsMfma32& 
 
 // WPB waves (pixels) per workgroup; slots last-first (the coherence matrices
 // the Gram wrote last are the ones still in the last-level cache).
-template <int MODE, int WPB>
-__global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(4))) void solve_mfma_kernel(SolveArgs a) {
-    __shared__ LdsMfma32 sm[WPB];
+template <int MODE, int DIM, int WPB>
+__global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(DIM == 32 ? 4 : 6))) void solve_mfma_kernel(SolveArgs a) {
+    __shared__ LdsMfma<DIM> sm[WPB];
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int slot = a.slots - 1 - ((int)blockIdx.x * WPB + w);
     if (slot < 0) return;
     const int np = a.npix[slot];
     const cx<float>* gam = (const cx<float>*)a.gamma + (size_t)slot * a.n * a.n;
-    solve_mfma_pixel<MODE>(a, sm[w], lane, np, GammaBuf(gam, a.n), a.first + slot);
+    solve_mfma_pixel<MODE, DIM>(a, sm[w], lane, np, GammaBuf(gam, a.n), a.first + slot);
 }
 
 }  // namespace fringe
