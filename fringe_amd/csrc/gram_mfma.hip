@@ -515,12 +515,12 @@ __global__ __launch_bounds__(64 * WAVES) void gram_mfma_pairs(MfmaArgs a) {
 // accumulator each for Re G and Im G, and its mirror is its transpose.
 //
 // Bound by the matrix instructions and the vector unit (operand permutes, list,
-// fold) together, and at 30 dates by Gamma's 8 n^2 bytes per pixel (2.7 TB/s).
+// fold) together, and at 30 dates by Gamma's 8 n^2 bytes per pixel (2.9 TB/s).
 // Measured against 32 x 32 x 16 products of all four real Grams up to 32 dates
-// (2048 x 2048 of 30 dates 14.7 -> 11.1 ms, 640 x 640 of 20 1.40 -> 1.04, 256 x
+// (2048 x 2048 of 30 dates 14.7 -> 10.3 ms, 640 x 640 of 20 1.40 -> 0.97, 256 x
 // 256 of 10 0.18 -> 0.06) and against the gathering kernel above (208 x 224 of
 // 48 dates 0.87 -> 0.24 ms, 131 k pixels of 64 dates in a 21 x 11 window 4.5 ->
-// 2.1).
+// 2.0).
 // Workgroups are numbered so that each XCD (which owns an L2) takes a
 // contiguous run of tiles and the halos neighbouring tiles share stay in it.
 // ---------------------------------------------------------------------------
@@ -599,9 +599,13 @@ gram_mfma_lds(MfmaArgs a) {
     typedef typename Frag<F16>::type frag_t;
     extern __shared__ __align__(16) char smem[];
     const int n = a.n, Nx = a.Nx, Ny = a.Ny;
-    const int TH = a.TH, TW = a.TW;
+    const int TH = a.TH, tw = 31 - __builtin_clz(a.TW), TW = 1 << tw;   // TW is a power of two
     const int WR = TH + 2 * Ny, WC = TW + 2 * Nx, NPOS = WR * WC;
     uint2* rec = (uint2*)smem;                             // [NPOS + 1][DP] (re, im) words
+    // (the list holds whole addresses: the compiler adds the base to an offset
+    // at every load, although it is zero)
+    typedef const uint2 __attribute__((address_space(3))) * lds_word;
+    const int rec0 = (int)(uintptr_t)(lds_word)rec;
     // wave index in a scalar register, so the pixel loop below is uniform
     // control flow (scalar branches) rather than exec-masked
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -630,7 +634,7 @@ gram_mfma_lds(MfmaArgs a) {
     // are requested at the top of an iteration and parked in LDS before this
     // pixel's Gamma stores, so no wait for them ever waits for the stores.
     auto mask_word = [&](int pid) -> uint32_t {
-        const int r = R0 + pid / TW, c = C0 + pid % TW;
+        const int r = R0 + (pid >> tw), c = C0 + (pid & (TW - 1));
         const bool ok = pid < TH * TW && r < row_end && r < a.rows && c < a.cols;
         // always one load, of pixel 0 when there is no pixel (such a pixel is
         // skipped before its word is used)
@@ -641,7 +645,7 @@ gram_mfma_lds(MfmaArgs a) {
     for (int pid = wave; pid < TH * TW; pid += WAVES) {
         const uint32_t wword = wbuf[lane];
         const uint32_t wnext = mask_word(pid + WAVES);
-        const int r = R0 + pid / TW, c = C0 + pid % TW;
+        const int r = R0 + (pid >> tw), c = C0 + (pid & (TW - 1));
         if (r >= row_end || r >= a.rows || c >= a.cols) {   // wave-uniform
             wbuf[lane] = wnext;
             continue;
@@ -651,12 +655,12 @@ gram_mfma_lds(MfmaArgs a) {
         // mask words reach the lanes through readlane (scalar registers), not
         // through an LDS-routed shuffle
         const bool cen = (__builtin_amdgcn_readlane(wword, fc >> 5) >> (fc & 31)) & 1u;
-        // ---- neighbour list: byte offsets of staged records.  Entry k goes
+        // ---- neighbour list: LDS addresses of staged records.  Entry k goes
         // to the k % 4'th group of 16 lanes, whose eight entries of a step
         // are contiguous ----
         const int lr = r - R0, lc = c - C0;                  // window origin in the stage
         auto place = [](int k) { return (k & ~31) | ((k & 3) << 3) | ((k >> 2) & 7); };
-        auto where = [](int pos) { return NB % 2 == 0 ? pos * (DP * 8) + ((pos & 1) << 7) : pos * (DP * 8); };
+        auto where = [&](int pos) { return rec0 + (NB % 2 == 0 ? pos * (DP * 8) + ((pos & 1) << 7) : pos * (DP * 8)); };
         int cnt = 0;
         for (int it = 0; it * 64 < Wn; ++it) {
             const int f = it * 64 + lane;
@@ -700,13 +704,17 @@ gram_mfma_lds(MfmaArgs a) {
         // 8-byte read gives this lane's (re, im) words of a position
         uint2 x[NB][8];
         auto load_step = [&](int st) {
-            const int* lp = list + 32 * st + 8 * q;
+            const int4* lp = (const int4*)(list + 32 * st + 8 * q);
+            const int4 l0 = lp[0], l1 = lp[1];
+            const int at[8] = {l0.x, l0.y, l0.z, l0.w, l1.x, l1.y, l1.z, l1.w};
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
-                const int at = lp[e] + 8 * m;
+                const int o = at[e] + 8 * m;
 #pragma unroll
-                for (int b = 0; b < NB; ++b)
-                    x[b][e] = *(const uint2*)((const char*)rec + (NB % 2 == 0 ? at ^ (b << 7) : at + (b << 7)));
+                for (int b = 0; b < NB; ++b) {
+                    const lds_word w = (lds_word)(uintptr_t)(uint32_t)(NB % 2 == 0 ? o ^ (b << 7) : o + (b << 7));
+                    x[b][e] = make_uint2(w->x, w->y);
+                }
             }
         };
         load_step(0);
