@@ -610,9 +610,9 @@ gram_mfma_lds(MfmaArgs a) {
     // control flow (scalar branches) rather than exec-masked
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     int* offs = (int*)(rec + (size_t)(NPOS + 1) * DP);      // window offsets, row << 16 | column
-    int* list = offs + 32 * kStageWords + wave * (a.list_cap + DP + 64);
+    int* list = offs + a.list_cap + wave * (a.list_cap + DP + kStageWords);
     float* dg = (float*)(list + a.list_cap);                // diagonal of Re G, DP
-    uint32_t* wbuf = (uint32_t*)(dg + DP);                  // next pixel's mask words, 64
+    uint32_t* wbuf = (uint32_t*)(dg + DP);                  // next pixel's mask words
 
     // XCD-aware tile order (blocks are dealt to the 8 XCDs round-robin)
     const unsigned nb = gridDim.x * gridDim.y, bid = blockIdx.y * gridDim.x + blockIdx.x;
@@ -641,13 +641,13 @@ gram_mfma_lds(MfmaArgs a) {
         const long long px = ok ? (long long)r * a.cols + c : 0;
         return a.wts[px * a.nul + (lane < a.nul ? lane : 0)];
     };
-    wbuf[lane] = mask_word(wave);
+    if (lane < kStageWords) wbuf[lane] = mask_word(wave);
     for (int pid = wave; pid < TH * TW; pid += WAVES) {
-        const uint32_t wword = wbuf[lane];
+        const uint32_t wword = wbuf[lane & (kStageWords - 1)];
         const uint32_t wnext = mask_word(pid + WAVES);
         const int r = R0 + (pid >> tw), c = C0 + (pid & (TW - 1));
         if (r >= row_end || r >= a.rows || c >= a.cols) {   // wave-uniform
-            wbuf[lane] = wnext;
+            if (lane < kStageWords) wbuf[lane] = wnext;
             continue;
         }
         const int slot = (r - a.row0) * a.cols + c;
@@ -687,7 +687,7 @@ gram_mfma_lds(MfmaArgs a) {
             cnt += __popcll(bal);
         }
         if (!(cen && cnt >= a.min_nb)) {
-            wbuf[lane] = wnext;
+            if (lane < kStageWords) wbuf[lane] = wnext;
             if (lane == 0) a.npix[slot] = -1;
             continue;
         }
@@ -775,7 +775,7 @@ gram_mfma_lds(MfmaArgs a) {
             }
         }
 
-        wbuf[lane] = wnext;   // waits for the load here, before the stores below
+        if (lane < kStageWords) wbuf[lane] = wnext;   // waits for the load here, before the stores below
 
         // ---- fold into Gamma ----
         // Re G_mm sits in register m % 4 of the lanes of quarter m / 4; it is
@@ -837,12 +837,18 @@ constexpr StageTile kStageTiles[] = {{8, 16, 16}, {4, 16, 8}, {4, 8, 8}, {4, 4, 
 static size_t gram_lds_bytes(int n, int Nx, int Ny, const StageTile& t) {
     const int dp = (n + 15) / 16 * 16;
     const size_t stage = (size_t)((t.TH + 2 * Ny) * (t.TW + 2 * Nx) + 1) * dp * 8;
-    return stage + 32 * kStageWords * 4 + (size_t)t.waves * (gram_list_cap(Nx, Ny) + dp + 64) * 4;
+    const int cap = gram_list_cap(Nx, Ny);   // of the window offsets, too
+    return stage + (size_t)cap * 4 + (size_t)t.waves * (cap + dp + kStageWords) * 4;
 }
 
-// Tile of the staged kernel: the largest that fits a CU's LDS and cuts the
-// grid into two workgroups per CU, or else the smallest that fits.  (64 x 64
-// pixels of 8 dates: 32 tiles of 8 x 16 took 77 us, 512 of 2 x 4 take 12.)
+// Tile of the staged kernel: the one with the least estimated time on the
+// launch's pixels, in units of a CU's time for a pixel when its waves fill it
+// (0.6 us at 30 dates).  A workgroup costs its pixels, and for staging four and
+// a hundredth of its positions; those of a CU share it, and a wave's pixels,
+// one after the other, take twelve each at least; the launch takes as many
+// rounds as it fills the chip.  (64 x 64 pixels of 8
+// dates: 32 tiles of 8 x 16 took 77 us, 512 of 2 x 4 take 12; 160 x 219 of 40:
+// 560 tiles of 4 x 16 in three rounds 219 us, 2200 of 4 x 4 in nine 198.)
 // A scheduled variant (FRINGE_GRAM_STAGED12 / 8 / 4) names the largest tile
 // tried; one that does not fit the window falls back to the others.  False
 // above 64 dates, for windows of more than kStageWords mask words and where
@@ -852,16 +858,25 @@ static bool gram_staged(int n, int Nx, int Ny, long long rows, int cols, StageTi
     const int v = n <= 32 ? schedule_lookup(FRINGE_SCHED_GRAM_VARIANT, n, Nx, Ny, FRINGE_GRAM_DEFAULT) : FRINGE_GRAM_DEFAULT;
     if (v == FRINGE_GRAM_UNSTAGED) return false;
     const int from = v == FRINGE_GRAM_STAGED8 ? 1 : v == FRINGE_GRAM_STAGED4 ? 2 : 0;
+    const int blocks = (n + 15) / 16, most = blocks == 1 ? 28 : blocks == 2 ? 16 : 8;   // waves of a CU, by registers
     bool found = false;
+    double least = 0.0;
     for (int k = from; k < (int)(sizeof(kStageTiles) / sizeof(kStageTiles[0])); ++k) {
         StageTile t = kStageTiles[k];
-        t.waves = std::min(t.waves, stage_waves((n + 15) / 16));
+        t.waves = std::min(t.waves, stage_waves(blocks));
         const size_t b = gram_lds_bytes(n, Nx, Ny, t);
         if (b > 160 * 1024) continue;
+        const long long wgs = (long long)((cols + t.TW - 1) / t.TW) * ((rows + t.TH - 1) / t.TH);
+        const int fit = (int)std::min<size_t>(160 * 1024 / b, (size_t)std::max(most / t.waves, 1));
+        const int active = (int)std::min<long long>(fit, (wgs + 255) / 256), px = t.TH * t.TW;
+        const double stage = 4 + 0.01 * (t.TH + 2 * Ny) * (t.TW + 2 * Nx);
+        const double cost = (double)((wgs + 256ll * active - 1) / (256ll * active)) *
+                            std::max(active * (px + stage), 12.0 * ((px + t.waves - 1) / t.waves) + stage);
+        if (found && cost >= least) continue;
         best = t;
         bytes = b;
+        least = cost;
         found = true;
-        if ((long long)((cols + t.TW - 1) / t.TW) * ((rows + t.TH - 1) / t.TH) >= 512) break;
     }
     return found;
 }
