@@ -170,7 +170,8 @@ int link_launch(const LinkPlan& P, const float2* slc, const uint32_t* wts, float
                 float* tcorr, float2* comp, hipStream_t s);
 size_t link_gamma_bytes_per_pixel(int n, int precision);
 size_t mfma_pack_bytes(int rows, int cols, int n);
-int pack_launch(const float2* slc, int rows, int cols, int n, bool f16, uint32_t* pk, hipStream_t s);
+// (count, if given, is cleared on the way)
+int pack_launch(const float2* slc, int rows, int cols, int n, bool f16, uint32_t* pk, int* count, hipStream_t s);
 int gram_mfma_launch(const LinkPlan& P, const uint32_t* pk, const uint32_t* wts, long long first,
                      int slots, hipStream_t s);
 bool link_uses_mfma(int n, int precision);

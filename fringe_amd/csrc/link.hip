@@ -73,7 +73,7 @@ int coherence_launch(const LinkPlan& P, const float2* slc, const uint32_t* wts, 
     const int slots = (P.row_end - P.row_begin) * P.cols;
     if (slots <= 0) return 0;
     if (link_uses_mfma(P.n, P.precision)) {
-        if (pack_launch(slc, P.rows, P.cols, P.n, P.precision != FRINGE_PREC_MIXED_BF16, P.d_pack, s) != 0)
+        if (pack_launch(slc, P.rows, P.cols, P.n, P.precision != FRINGE_PREC_MIXED_BF16, P.d_pack, nullptr, s) != 0)
             return -1;
         LinkPlan Q = P;
         Q.d_gamma = gamma;
@@ -170,13 +170,12 @@ int link_launch(const LinkPlan& P, const float2* slc, const uint32_t* wts, float
     const bool mfma = link_uses_mfma(P.n, P.precision);
     const int mode = solve_mode_index(P.module, P.method);
     const int sched = schedule_lookup(FRINGE_SCHED_SOLVE, P.n, mode, fp64 ? 0 : 1, 0);
-    if (P.d_cert_count) {
-        clear_counter(P.d_cert_count, s);
-    }
     if (mfma) {
         StageScope sc(STAGE_PACK, s);
-        if (pack_launch(slc, P.rows, P.cols, P.n, P.precision != FRINGE_PREC_MIXED_BF16, P.d_pack, s) != 0)
+        if (pack_launch(slc, P.rows, P.cols, P.n, P.precision != FRINGE_PREC_MIXED_BF16, P.d_pack, P.d_cert_count, s) != 0)
             return -1;
+    } else if (P.d_cert_count) {
+        clear_counter(P.d_cert_count, s);
     }
     int rc = 0;
     for (long long done = 0; done < total; done += P.chunk) {
@@ -262,12 +261,13 @@ int link_batch_launch(const BatchPlan& B, hipStream_t s) {
     const int count = (int)B.tiles.size();
     for (int i = 0; i < count; ++i) {
         const BatchTile& T = B.tiles[i];
-        if (T.P.d_cert_count) clear_counter(T.P.d_cert_count, s);
         if (link_uses_mfma(T.P.n, T.P.precision)) {
             StageScope sc(STAGE_PACK, s);
             if (pack_launch(T.slc, T.P.rows, T.P.cols, T.P.n, T.P.precision != FRINGE_PREC_MIXED_BF16, T.P.d_pack,
-                            s) != 0)
+                            T.P.d_cert_count, s) != 0)
                 return -1;
+        } else if (T.P.d_cert_count) {
+            clear_counter(T.P.d_cert_count, s);
         }
     }
     const int mode = solve_mode_index(B.module, B.method);
