@@ -1,24 +1,24 @@
-// solve32.hpp -- register-resident per-pixel estimator for n <= 64 dates.
+// solve32.hpp -- register-resident per-pixel estimator, one row per lane, for
+// 33 to 64 dates where a schedule selects it (the matrix-core solvers are the
+// default), and the lane reductions the matrix-core solvers use.
 //
-// NR = 32 (n <= 32, FP64 only: solve_mfma.hpp serves FP32): a wave holds two
-// pixels and lane r of a 32-lane half owns row r of every matrix of its
-// pixel in registers.  NR = 64
-// (32 < n <= 64): one pixel per wave, lane r owns row r.  LDS (about 3.5 KB per pixel) is used only
-// to publish one row or one vector to the other lanes, so many waves fit on
-// a CU and the arithmetic is not serialised behind LDS round trips.
+// One pixel per wave: lane r owns row r of every matrix of its pixel in
+// registers (NR = 64 rows).  LDS (about 7 KB per pixel) is used only to
+// publish one row or one vector to the other lanes, so many waves fit on a CU
+// and the arithmetic is not serialised behind LDS round trips.
 //
 // Stages (same semantics as the generic LDS solver in link_solve.hpp):
 //   * inverse of the real |Gamma| by the symmetric sweep operator in FP64,
-//     with the matrix in 4 x 8 blocks (lane (a, b) of a half holds rows
-//     4a..4a+3, columns 8b..8b+7): per pivot a lane reads 4 multipliers and
-//     8 pivot-row entries from LDS instead of a whole row, then the blocks go
+//     with the matrix in 8 x 8 blocks (lane (a, b) holds rows 8a..8a+7,
+//     columns 8b..8b+7): per pivot a lane reads 8 multipliers and 8 pivot-row
+//     entries from LDS instead of a whole row, then the blocks go
 //     back to one row per lane a block column at a time;
 //   * H = |Gamma|^-1 o Gamma (or Gamma itself for EVD) into registers;
 //   * Householder tridiagonalisation: the owner of row j publishes it, the
 //     reflector v_j = conj(row j) * scal_j is applied, and every lane parks
 //     its own entry of v_j in the register of the column just annihilated,
 //     where the back-transformation finds it;
-//   * eigenvalue by 33-section of Sturm counts, eigenvector of T by inverse
+//   * eigenvalue by 65-section of Sturm counts, eigenvector of T by inverse
 //     iteration (every lane runs the same pivoted elimination chain on
 //     broadcast operands), back-transformation by the stored reflectors;
 //   * referenced phases, compressed SLC and temporal coherence.
@@ -138,7 +138,7 @@ template <int NR, typename T> __device__ __forceinline__ cx<T> sumR(cx<T> x) { r
 
 // ---- FP64 inverse of |Gamma| - shift*I in BR x 8 blocks -------------------
 // Lane (a, b) = (r / NCB, r % NCB) holds M[i][j] = A(BR a + i, 8b + j)
-// (BR = 4, NCB = 4 for NR = 32; BR = 8, NCB = 8 for NR = 64).
+// (BR = NCB = 8 for NR = 64).
 // Rows and columns >= n hold the identity (never swept, never mixed in).
 template <int NR, typename Tg>
 __device__ __forceinline__ bool abs_gamma_block(double (&M)[Blk<NR>::BR][8], const cx<Tg>* gam, int n, int r, bool act,
@@ -241,12 +241,7 @@ __device__ __forceinline__ void blocks_to_rows(LdsR<T, NR>& L, const double (&M)
 // ---- Householder tridiagonalisation of the rows in h ---------------------
 // Step j of the reduction, for C0 - 1 <= j <= C0 + STEP - 2: columns below
 // C0 hold only finished entries and parked reflectors, so they are skipped.
-// Columns from NC on (n <= NC <= NR) are skipped too: there h, V and W hold
-// +0 in every step, so each skipped product is a zero added to a sum that
-// is never -0 (it starts at +0, and an FMA returns -0 only from a -0
-// addend), and each skipped update leaves a +0 that nothing reads: the
-// results are the same bits as with NC = NR.
-template <typename T, int NR, int C0, int STEP, int NC = NR>
+template <typename T, int NR, int C0, int STEP>
 __device__ __forceinline__ void tri_step(LdsR<T, NR>& L, cx<T> (&h)[NR], int j, int n, int r) {
     // row j was published at the end of the previous step (or before the first)
     const cx<T> alpha = cconj(L.R[j + 1]);
@@ -278,7 +273,7 @@ __device__ __forceinline__ void tri_step(LdsR<T, NR>& L, cx<T> (&h)[NR], int j, 
     wsync();
     cx<T> p = {T(0), T(0)};
 #pragma unroll
-    for (int c = C0; c < NC; ++c) cfma(p, h[c], L.V[c]);
+    for (int c = C0; c < NR; ++c) cfma(p, h[c], L.V[c]);
     p = cmul(tau, p);
     const cx<T> s = sumR<NR>(cmulc(vr, p));
     const cx<T> a2 = cscale(cmul(tau, s), T(-0.5));
@@ -286,7 +281,7 @@ __device__ __forceinline__ void tri_step(LdsR<T, NR>& L, cx<T> (&h)[NR], int j, 
     L.W[r] = wr;
     wsync();
 #pragma unroll
-    for (int c = C0; c < NC; ++c) {
+    for (int c = C0; c < NR; ++c) {
         cfms_c(h[c], vr, L.W[c]);
         cfms_c(h[c], wr, L.V[c]);
     }
@@ -294,43 +289,40 @@ __device__ __forceinline__ void tri_step(LdsR<T, NR>& L, cx<T> (&h)[NR], int j, 
     // lane's entry of v_j there for the back-transformation (no later step
     // reads it: V and W vanish at column j from here on)
 #pragma unroll
-    for (int c = (C0 > 0 ? C0 - 1 : 0); c < (C0 + STEP - 1 < NC ? C0 + STEP - 1 : NC); ++c)
+    for (int c = (C0 > 0 ? C0 - 1 : 0); c < (C0 + STEP - 1 < NR ? C0 + STEP - 1 : NR); ++c)
         if (c == j && r > j + 1) h[c] = vr;
-    // publish row j + 1 for the next step (everyone is past reading row j;
-    // entries from NC on are never read)
+    // publish row j + 1 for the next step (everyone is past reading row j)
     if (r == j + 1) {
 #pragma unroll
-        for (int c = 0; c < NC; ++c) L.R[c] = h[c];
+        for (int c = 0; c < NR; ++c) L.R[c] = h[c];
     }
     wsync();
 }
 
 // Steps C0 - 1 .. C0 + STEP - 2 (the last block: up to n - 2), then the
-// next block of STEP columns: one loop per quad (NR = 32) or octet (NR =
-// 64) of columns left to update (separate loops keep the register
+// next block of STEP columns: one loop per octet of
+// columns left to update (separate loops keep the register
 // allocation of each variant to itself).
-template <typename T, int NR, int NC, int C0, int STEP>
+template <typename T, int NR, int C0, int STEP>
 __device__ __forceinline__ void tri_blocks(LdsR<T, NR>& L, cx<T> (&h)[NR], int& j, int n, int r) {
-    if constexpr (C0 + STEP < NC) {
-        for (; j < min(C0 + STEP - 1, n - 1); ++j) tri_step<T, NR, C0, STEP, NC>(L, h, j, n, r);
-        tri_blocks<T, NR, NC, C0 + STEP, STEP>(L, h, j, n, r);
+    if constexpr (C0 + STEP < NR) {
+        for (; j < min(C0 + STEP - 1, n - 1); ++j) tri_step<T, NR, C0, STEP>(L, h, j, n, r);
+        tri_blocks<T, NR, C0 + STEP, STEP>(L, h, j, n, r);
     } else {
-        for (; j < n - 1; ++j) tri_step<T, NR, C0, STEP, NC>(L, h, j, n, r);
+        for (; j < n - 1; ++j) tri_step<T, NR, C0, STEP>(L, h, j, n, r);
     }
 }
 
-// NC: the columns processed (n <= NC <= NR; the last block may be partial).
-template <typename T, int NR, int NC = NR>
+template <typename T, int NR>
 __device__ __forceinline__ void tridiag(LdsR<T, NR>& L, cx<T> (&h)[NR], int n, int r) {
-    static_assert(NC > 0 && NC <= NR, "columns of the lanes' rows");
     if (r == 0) {
 #pragma unroll
-        for (int c = 0; c < NC; ++c) L.R[c] = h[c];
+        for (int c = 0; c < NR; ++c) L.R[c] = h[c];
     }
     wsync();
     // columns below j+1 carry zero reflector entries
     int j = 0;
-    tri_blocks<T, NR, NC, 0, NR == 32 ? 4 : 8>(L, h, j, n, r);
+    tri_blocks<T, NR, 0, 8>(L, h, j, n, r);
     // last diagonal entry: row n - 1 is the one published last
     if (r == 0) L.D[n - 1] = L.R[n - 1].re;
     wsync();
@@ -365,7 +357,7 @@ __device__ __forceinline__ T bisect(LdsR<T, NR>& L, int n, int k, int r, T& tnor
     // (NR+1)-section shrinks the Gershgorin interval (NR+1)-fold per round:
     // 5 rounds of 33 or 4 of 65 reach ~1e-7 |T| (enough for the
     // inverse-iteration shift in FP32), 10 of 33 or 9 of 65 FP64 resolution
-    const int rounds = sizeof(T) == 4 ? (NR == 32 ? 5 : 4) : (NR == 32 ? 10 : 9);
+    const int rounds = sizeof(T) == 4 ? 4 : 9;
     for (int it = 0; it < rounds; ++it) {
         const T w33 = (hi - lo) * T(1.0 / (NR + 1));   // the same expression gives every section point
         const T sig = lo + w33 * T(r + 1);
@@ -568,7 +560,7 @@ enum { MODE_EMI = 0, MODE_EVD = 1, MODE_MLE = 2 };
 // coherence (global memory, or LDS in the FP64 re-solve), np its neighbour
 // count (-1: not linked).  CERT: the FP32 result is checked and, when it is
 // not certified, the pixel is appended to a.cert_list for the FP64 re-solve.
-template <typename T, typename Tg, int MODE, int NR, bool CERT, int NC = NR>
+template <typename T, typename Tg, int MODE, int NR, bool CERT>
 __device__ __forceinline__ void solve_reg_pixel(const SolveArgs& a, LdsR<T, NR>& L, int r, bool inslot, int np,
                                                 const cx<Tg>* gam, long long pix) {
     const int n = a.n;
@@ -584,7 +576,7 @@ __device__ __forceinline__ void solve_reg_pixel(const SolveArgs& a, LdsR<T, NR>&
 
     if constexpr (MODE == MODE_MLE) {
         const bool fin = load_rows<T, Tg, NR>(h, grow, n, r, act, -1);
-        tridiag<T, NR, NC>(L, h, n, r);
+        tridiag<T, NR>(L, h, n, r);
         const T lmin = bisect<T, NR>(L, n, 0, r, tn, pm);
         if (!fin) { code = -1.0f; failed = true; }
         else if (!(lmin >= T(1.0e-6))) { code = -2.0f; failed = true; }
@@ -601,7 +593,7 @@ __device__ __forceinline__ void solve_reg_pixel(const SolveArgs& a, LdsR<T, NR>&
         if constexpr (CERT) unc = unc || !(pmin2 >= kCertPivotMin);
         blocks_to_rows<T, NR>(L, M, m, r);
         const bool hfin = hadamard_rows<T, Tg, NR>(h, m, grow, n, r, act);
-        tridiag<T, NR, NC>(L, h, n, r);
+        tridiag<T, NR>(L, h, n, r);
         const T lam = bisect<T, NR>(L, n, 0, r, tn, pm);
         const T yr = tri_eigvec<T, NR>(L, n, r, lam, tn);
         y = back_transform<T, NR>(L, h, n, r, cx<T>{yr, T(0)});
@@ -615,7 +607,7 @@ __device__ __forceinline__ void solve_reg_pixel(const SolveArgs& a, LdsR<T, NR>&
     } else if constexpr (MODE == MODE_EVD) {
         const int band = (a.method == FRINGE_METHOD_STBAS) ? a.bw : -1;
         const bool fin = load_rows<T, Tg, NR>(h, grow, n, r, act, band);
-        tridiag<T, NR, NC>(L, h, n, r);
+        tridiag<T, NR>(L, h, n, r);
         const T lam = bisect<T, NR>(L, n, n - 1, r, tn, pm);
         const T yr = tri_eigvec<T, NR>(L, n, r, lam, tn);
         y = back_transform<T, NR>(L, h, n, r, cx<T>{yr, T(0)});
@@ -638,7 +630,7 @@ __device__ __forceinline__ void solve_reg_pixel(const SolveArgs& a, LdsR<T, NR>&
         // the EMI eigenpair, unless every pixel of the wave falls back to EVD
         // (a pixel's result never depends on whether this ran for it)
         if (__any(!run_evd)) {
-            tridiag<T, NR, NC>(L, h, n, r);
+            tridiag<T, NR>(L, h, n, r);
             const T lam = bisect<T, NR>(L, n, 0, r, tn, pm);
             const T yr = tri_eigvec<T, NR>(L, n, r, lam, tn);
             y = back_transform<T, NR>(L, h, n, r, cx<T>{yr, T(0)});
@@ -650,7 +642,7 @@ __device__ __forceinline__ void solve_reg_pixel(const SolveArgs& a, LdsR<T, NR>&
         }
         if (__any(act && fin && run_evd)) {
             load_rows<T, Tg, NR>(h, grow, n, r, act, -1);
-            tridiag<T, NR, NC>(L, h, n, r);
+            tridiag<T, NR>(L, h, n, r);
             const T le = bisect<T, NR>(L, n, n - 1, r, tn, pm);
             const T ye = tri_eigvec<T, NR>(L, n, r, le, tn);
             const cx<T> yv = back_transform<T, NR>(L, h, n, r, cx<T>{ye, T(0)});
@@ -755,12 +747,10 @@ __device__ __forceinline__ void solve_reg_pixel(const SolveArgs& a, LdsR<T, NR>&
 }
 
 // LIST = false: slot s of the round's coherence buffer is pixel first + s;
-// NR = 32 holds two pixels per wave, NR = 64 one.  The FP32 instances
-// certify their results.  LIST = true (T = Tg = double): the FP64 re-solve
+// One pixel per wave.  The FP32 instances certify their results.  LIST = true (T = Tg = double): the FP64 re-solve
 // of the listed pixels; each group computes its pixel's coherence with the
-// FP64 Gram into LDS and solves it there, looping over the list.  NC: the
-// columns the tridiagonal reductions process (n <= NC; same results).
-template <typename T, typename Tg, int MODE, int NR, bool LIST, int NC = NR>
+// FP64 Gram into LDS and solves it there, looping over the list.
+template <typename T, typename Tg, int MODE, int NR, bool LIST>
 __global__ __launch_bounds__(64) void solve_reg_kernel(SolveArgs a) {
     __shared__ LdsR<T, NR> sm[64 / NR];
     const int grp = threadIdx.x / NR, r = threadIdx.x % NR;
@@ -774,7 +764,7 @@ __global__ __launch_bounds__(64) void solve_reg_kernel(SolveArgs a) {
         const int np = inslot ? a.npix[slot] : -1;
         const cx<Tg>* gam = (const cx<Tg>*)a.gamma + (size_t)(inslot ? slot : 0) * a.n * a.n;
         const long long pix = a.first + (inslot ? slot : 0);
-        solve_reg_pixel<T, Tg, MODE, NR, sizeof(T) == 4, NC>(a, L, r, inslot, np, gam, pix);
+        solve_reg_pixel<T, Tg, MODE, NR, sizeof(T) == 4>(a, L, r, inslot, np, gam, pix);
     } else {
         static_assert(sizeof(T) == 8 && sizeof(Tg) == 8, "the re-solve runs in FP64");
         constexpr int GPW = 64 / NR;
@@ -791,14 +781,14 @@ __global__ __launch_bounds__(64) void solve_reg_kernel(SolveArgs a) {
             const int np = gram_f64_pixel<NR, 1, kResolveSmallCB>(a.g64, valid, pix, gl, gscratch);
             __threadfence();
             __syncthreads();
-            solve_reg_pixel<T, Tg, MODE, NR, false, NC>(a, L, r, valid, np, (const cx<Tg>*)gl, pix);
+            solve_reg_pixel<T, Tg, MODE, NR, false>(a, L, r, valid, np, (const cx<Tg>*)gl, pix);
             __syncthreads();
         }
     }
 }
 
-// Persistent launch up to 64 dates: each wave takes units (two pixels for
-// NR = 32, one for NR = 64) of the queued jobs until the queue is drained.
+// Persistent launch up to 64 dates: each wave takes pixels of the queued jobs
+// until the queue is drained.
 template <typename T, typename Tg, int MODE, int NR>
 __global__ __launch_bounds__(64) void solve_reg_persistent(PersistArgs pa) {
     __shared__ LdsR<T, NR> sm[64 / NR];

@@ -723,7 +723,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(waves64
 
 // The plain path's coherence: one slot per workgroup.
 template <int NW>
-__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW <= 4 ? 4 : 3))) void gram_mfma64_kernel(GramArgs a) {
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW <= 4 ? 4 : NW <= 7 ? 3 : 2))) void gram_mfma64_kernel(GramArgs a) {
     __shared__ LdsGram64<NW> L;
     extern __shared__ __align__(16) char smem[];
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
