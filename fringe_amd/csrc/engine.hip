@@ -168,27 +168,20 @@ int link_check(const fringe_link_tile* t) {
     if (link_uses_mfma(t->nbands, t->precision) && t->nbands <= 64 &&
         ((long long)t->rows * t->cols + 1) * 2 * t->nbands >= (1ll << 32))
         return FRINGE_ERR_UNSUPPORTED;
-    // LDS footprint of the generic solver used above 64 dates (one pixel per
-    // two-wave workgroup): the pixel's matrices plus the kernel's static LDS
     // LDS of the solver kernels: above 64 dates the work matrix moves to
-    // global memory when it does not fit, the rest of a pixel's group must
+    // global memory when it does not fit, the rest of a pixel's group must.
+    // The matrix-core re-solve takes 77 KB at most, whatever the window (a CU
+    // has 160)
     const size_t lds = (size_t)device_lds_limit();
+    const bool resolves = link_certifies(t->nbands, t->precision) && !matrix_solver_selected(t->nbands, FRINGE_PREC_FP64);
     if (t->nbands <= 64) {
-        if (link_certifies(t->nbands, t->precision) &&
-            (matrix_solver_selected(t->nbands, FRINGE_PREC_FP64) ? resolve_mfma64_lds_bytes(t->nbands, t->Nx, t->Ny)
-                                                                 : resolve_lanes_lds_bytes(t->nbands, t->Nx, t->Ny)) > lds)
-            return FRINGE_ERR_UNSUPPORTED;
+        if (resolves && resolve_lanes_lds_bytes(t->nbands, t->Nx, t->Ny) > lds) return FRINGE_ERR_UNSUPPORTED;
     } else {
         const size_t rest = (t->precision == FRINGE_PREC_FP64 ? solve_group_bytes<double>(t->nbands, false)
                                                               : solve_group_bytes<float>(t->nbands, false)) +
                             solve_static_lds(t->precision);
         if (rest > lds) return FRINGE_ERR_UNSUPPORTED;
-        if (link_certifies(t->nbands, t->precision)) {
-            const size_t r = matrix_solver_selected(t->nbands, FRINGE_PREC_FP64)
-                                 ? resolve_mfma64_lds_bytes(t->nbands, t->Nx, t->Ny)
-                                 : resolve_generic_lds_bytes(t->nbands, t->Nx, t->Ny);
-            if (r > lds) return FRINGE_ERR_UNSUPPORTED;
-        }
+        if (resolves && resolve_generic_lds_bytes(t->nbands, t->Nx, t->Ny) > lds) return FRINGE_ERR_UNSUPPORTED;
     }
     return 0;
 }

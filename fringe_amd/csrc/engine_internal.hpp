@@ -128,8 +128,6 @@ int generic_a_default(int n, int precision);
 // 49..64 always): the matrix-core solvers (the FP64 re-solve follows the FP64 choice, whose
 // outputs it must equal).
 bool matrix_solver_selected(int n, int precision);
-// LDS of the matrix-core re-solve's workgroup.
-size_t resolve_mfma64_lds_bytes(int n, int Nx, int Ny);
 // The FP64 re-solve of a tile's list, and a counter's reset.
 void resolve_tile(const LinkPlan& P, const float2* slc, const uint32_t* wts, float2* phase, float* tcorr, float2* comp,
                   hipStream_t s);

@@ -39,21 +39,4 @@ void launch_resolve_mfma64(const SolveArgs& args, unsigned blocks, hipStream_t s
     }
 }
 
-template <int NW> static size_t lds_of(int Nx, int Ny) {
-    return std::max(sizeof(LdsMfma64<NW>), sizeof(LdsGram64<NW>)) + scratch<NW>(Nx, Ny);
-}
-
-size_t resolve_mfma64_lds_bytes(int n, int Nx, int Ny) {
-    switch ((n + 15) / 16) {
-        case 1: return lds_of<1>(Nx, Ny);
-        case 2: return lds_of<2>(Nx, Ny);
-        case 3: return lds_of<3>(Nx, Ny);
-        case 4: return lds_of<4>(Nx, Ny);
-        case 5: return lds_of<5>(Nx, Ny);
-        case 6: return lds_of<6>(Nx, Ny);
-        case 7: return lds_of<7>(Nx, Ny);
-        default: return lds_of<8>(Nx, Ny);
-    }
-}
-
 }  // namespace fringe
