@@ -47,6 +47,9 @@ struct SolveArgs {
     // (set_solve_counts)
     float inv_n;
     double inv_pairs, inv_comp;
+    // FP32 matrix-core solver: factor on its certification scale times eps
+    // (launch_solve_mfma)
+    float cert_eps;
 };
 
 // Certification of an FP32 eigenpair.  The FP32 chain's backward error is
@@ -67,8 +70,8 @@ constexpr float kCertThrMargin = 256.0f;
 constexpr double kCertPivotMin = 1.0e-4;
 
 // FP32 solver of the mixed precisions up to 128 dates (solve_mfma.hpp,
-// solve_mfma_wg.hpp).
-void launch_solve_mfma(const SolveArgs& a, hipStream_t s);
+// solve_mfma_wg.hpp); bf16: Gamma comes from bfloat16 pairs.
+void launch_solve_mfma(const SolveArgs& a, bool bf16, hipStream_t s);
 // FP64 solver up to 128 dates (solve_mfma64.hpp): the plain path, and the
 // re-solve of a pixel list (a.awork / a.awork_stride: the workgroups' areas,
 // at least n^2 complex doubles each, `blocks` of them; a.g64, a.list*: the

@@ -54,7 +54,12 @@ typedef double mf64x4 __attribute__((ext_vector_type(4)));
 // than dates, the phase errors of certified pixels are C eps |A| / (gap
 // min|v|) with C at most 0.07 for H (the former solver: 0.61) and 0.91 for
 // Gamma (the former: 1.4): the scales keep the estimate below 5e-4 rad, half
-// the tolerance, with C = 0.5 and C = 1.25.
+// the tolerance, with C = 0.5 and C = 1.25.  They hold for Gamma from half
+// pairs (22 bits).  bfloat16 pairs carry 16 bits, and H multiplies Gamma's
+// error by up to the square of |Gamma|'s inverse: there the wider scale of
+// the vector-unit solvers (kCertScale) leaves such pixels to the FP64 path,
+// whose coherence is its own.  297 x 43 pixels of 34 dates (EMI, 77 looks):
+// error against 64 bits 2.4e-5 -> 3.9e-6, 1.05 -> 2.59 ms.
 constexpr float kCertScaleEmi = 1.0e3f, kCertScaleEvd = 2.5e3f;
 
 // Accumulator of a DIM x DIM matrix: NV registers, lane l holds column l % DIM
@@ -624,7 +629,7 @@ __device__ __forceinline__ void solve_mfma_pixel(const SolveArgs& a, LdsMfma<DIM
                 }
                 // ---- certification ----
                 const float m2 = redC<DIM, OpMin>(in ? cabs2(E.x) : 3.0e38f);
-                delta = (inv ? kCertScaleEmi : kCertScaleEvd) * Lim<float>::eps() * tn * __builtin_amdgcn_rsqf(uni(m2));
+                delta = (inv ? kCertScaleEmi : kCertScaleEvd) * a.cert_eps * tn * __builtin_amdgcn_rsqf(uni(m2));
                 if (!(delta <= tn)) break;
                 // Frobenius norm of the inverse: its other eigenvalues'
                 // squares sum to S2, so none of them exceeds sqrt(S2)

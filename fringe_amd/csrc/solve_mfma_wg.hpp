@@ -35,6 +35,7 @@ template <int NT, bool INV> struct LdsMfmaWg {
     };
     float xr[NT][32], xi[NT][32];
     double red[2][NT][2];
+    float cert_eps;                      // SolveArgs::cert_eps
 };
 
 // Sum of x (alike in the wave's lanes) over the workgroup's waves.
@@ -345,6 +346,8 @@ __device__ __forceinline__ void solve_mfma_wg_pixel(const SolveArgs& a, LdsMfmaW
     EigStateWg<NT> E;
 
     const bool act = np >= 0;
+    // read behind the sweep's barriers; held in a register it spilled
+    if (threadIdx.x == 0) L.cert_eps = a.cert_eps;
     // What follows from the lane is computed again in each stage: held over
     // the sweeps it spilled.
     if (act) {
@@ -554,7 +557,7 @@ __device__ __forceinline__ void solve_mfma_wg_pixel(const SolveArgs& a, LdsMfmaW
 #pragma unroll
                 for (int J = 0; J < NT; ++J)
                     if (32 * J + col < n) m2 = fminf(m2, cabs2(E.x[J]));
-                delta = scal((inv ? kCertScaleEmi : kCertScaleEvd) * Lim<float>::eps() *
+                delta = scal((inv ? kCertScaleEmi : kCertScaleEvd) * L.cert_eps *
                              (tn * __builtin_amdgcn_rsqf(uni(red32<OpMin>(m2)))));
                 if (!(delta <= tn)) break;
                 float f = 0.0f;

@@ -57,7 +57,7 @@ void launch_solve(const SolveArgs& a, int precision, hipStream_t s) {
     const bool fp64 = precision == FRINGE_PREC_FP64;
     if (matrix_solver_selected(a.n, precision)) {
         if (fp64) launch_solve_mfma64(a, s);
-        else launch_solve_mfma(a, s);
+        else launch_solve_mfma(a, precision == FRINGE_PREC_MIXED_BF16, s);
     } else if (a.n <= 64) {
         if (fp64) launch_lanes<double, double>(a, s);
         else launch_lanes<float, float>(a, s);

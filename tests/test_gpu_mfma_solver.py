@@ -127,3 +127,17 @@ def test_uncorrelated_dates_have_zero_coherence(module, method):
     print(st)
     assert st["untouched_equal"] and st["codes_equal"] and st["n_well"] > 0
     assert st["phase_max"] <= PHASE_TOL and st["tcorr_max"] <= TCORR_TOL and st["comp_err"] <= PHASE_TOL
+
+
+@pytest.mark.parametrize("module,method", [("phase_link", "MLE"), ("evd", "EVD")])
+@pytest.mark.parametrize("n", [28, 34])
+def test_bf16_pairs_leave_sensitive_pixels_to_fp64(n, module, method):
+    """Few looks a date: the error of bfloat16 pairs, multiplied by the
+    inverse of |Gamma|, has to stay below the phase tolerance at every pixel."""
+    rows, cols, Nx, Ny = 160, 96, (n - 1) // 6, 3
+    print(f"case bf16 n={n} {module}/{method}", flush=True)
+    slc = synthetic.stack(n, rows, cols, seed=n)
+    wts = synthetic.full_mask(rows, cols, Nx, Ny)
+    e, _ = _run(slc, wts, Nx, Ny, module, method, precision="fp64")
+    g, _ = _run(slc, wts, Nx, Ny, module, method, precision="mixed_bf16")
+    assert np.abs(np.angle(g[0] * e[0].conj())).max() <= PHASE_TOL
