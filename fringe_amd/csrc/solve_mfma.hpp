@@ -539,10 +539,8 @@ __device__ __forceinline__ void solve_mfma_pixel(const SolveArgs& a, LdsMfma<DIM
                 }
                 f2 = fmaf(R[v], R[v], fmaf(I[v], I[v], f2));
             }
-            if constexpr (MODE == MODE_EVD) {
-                sum = uni(sumH<DIM>(redC<DIM, OpAdd>(f2)));
-                if (!(sum < 3.0e38f)) code = -6.0f;
-            }
+            sum = uni(sumH<DIM>(redC<DIM, OpAdd>(f2)));
+            if (MODE == MODE_EVD && !(sum < 3.0e38f)) code = -6.0f;
             if (code == 0.0f) {
                 float rho = 1.0f, dn = 1.0f;
                 for (int k = 0; k < 3; ++k) {

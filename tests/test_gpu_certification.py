@@ -1,0 +1,54 @@
+"""Which results of the FP32 estimator chain are kept, and how far off they
+are: the certificate against eigenvalues and phases of the FP64 path, without
+the filters on eigen-gap and component size of the parity tests."""
+import numpy as np
+import pytest
+
+from conftest import gpu_available
+from helpers import to_dev
+
+pytestmark = pytest.mark.gpu
+
+if not gpu_available():
+    pytest.skip("needs a GPU", allow_module_level=True)
+
+import torch  # noqa: E402
+
+from fringe_amd import synthetic, tile  # noqa: E402
+
+EPS = 2.0 ** -24
+
+
+def _mask(rows, cols, Nx, Ny):
+    return torch.from_numpy(synthetic.full_mask(rows, cols, Nx, Ny).view(np.int32)).cuda()
+
+
+def _link(ds, w, Nx, Ny, precision, **kw):
+    n, rows, cols = ds.shape
+    r = tile.LinkRunner(tile.link_params(rows, cols, n, Nx, Ny, precision=precision, **kw))
+    out = tuple(x.cpu().numpy() for x in r.run(ds, w))
+    kept = np.ones(rows * cols, bool)
+    kept[r.resolved_pixels()] = False
+    return out, kept
+
+
+@pytest.mark.parametrize("n,Nx,Ny", [(20, 2, 1), (30, 3, 1), (30, 2, 2), (32, 2, 2)])
+def test_emi_fallback_keeps_no_close_pair(n, Nx, Ny):
+    """EMI pixels whose |Gamma| is not positive definite (fewer looks than
+    dates, coherence that decays to 0) fall back to the largest eigenvalue of
+    Gamma.  One that is kept in FP32 has no other eigenvalue within 2500 eps
+    |Gamma| / min|v| of it (eps: 2^-24; a tenth for the error of Gamma)."""
+    rows = cols = 112
+    print(f"case fallback n={n} {2 * Nx + 1}x{2 * Ny + 1}", flush=True)
+    slc = synthetic.stack(n, rows, cols, seed=5, coh=synthetic.coherence_matrix(n, ginf=0.0))
+    ds, w = to_dev(slc, torch), _mask(rows, cols, Nx, Ny)
+    gamma = tile.coherence(ds, w, Nx, Ny, precision="fp64")[0].cpu()
+    fallback = torch.linalg.eigvalsh(gamma.abs())[:, 0].numpy() < -1.0e-3
+    _, kept = _link(ds, w, Nx, Ny, "mixed", min_neighbors=2)
+    at = np.nonzero(fallback & kept)[0]
+    assert at.size > 1000
+    lam, v = torch.linalg.eigh(gamma[torch.from_numpy(at)])
+    lam, least = lam.numpy(), v[:, :, -1].abs().amin(1).numpy()
+    short = (lam[:, -1] - lam[:, -2]) * least / (2500 * EPS * lam[:, -1])
+    print(f"{at.size} kept, smallest distance {short.min():.2f} of the certificate's")
+    assert short.min() >= 0.9
