@@ -29,9 +29,7 @@ template <int NT> static void launch_wg(const SolveArgs& a, hipStream_t s) {
 void launch_solve_mfma(const SolveArgs& args, bool bf16, hipStream_t s) {
     SolveArgs a = args;
     set_solve_counts(a);
-    // bfloat16 pairs: kCertScale instead, the reason at kCertScaleEmi
-    const bool gamma = a.module == FRINGE_MODULE_EVD && a.method != FRINGE_METHOD_MLE;
-    a.cert_eps = 5.9604645e-8f * (bf16 ? kCertScale / (gamma ? kCertScaleEvd : kCertScaleEmi) : 1.0f);
+    a.cert_h = 5.9604645e-8f * (bf16 ? kCertScale : a.n <= 48 ? kCertScaleH : kCertScaleH * 48.0f / (float)a.n);
     if (a.n > 96) launch_wg<4>(a, s);
     else if (a.n > 64) launch_wg<3>(a, s);
     else if (a.n > 32) launch_wg<2>(a, s);

@@ -25,7 +25,7 @@
 // quotient after three power steps.  Slow convergence moves sigma.  Every
 // pivot's sign is counted, and the inertia, the Frobenius norm of the
 // inverse and the Rayleigh quotient certify that no other eigenvalue lies
-// within the certification distance (kCertScaleMfma).
+// within the certification distance (cert_eps).
 //
 // What bounds it: the vector unit and the FP32 / FP64 matrix instructions
 // together (their busy cycles add up to the kernel's time; 4, 5 or 6 waves
@@ -47,20 +47,27 @@ namespace fringe {
 typedef float mf32x16 __attribute__((ext_vector_type(16)));
 typedef double mf64x4 __attribute__((ext_vector_type(4)));
 
-// Certification distance of this solver, as kCertScale: no eigenvalue may lie
-// within scale eps |A| / min_t |v_t| of the selected one, with |A| bounded by
-// the eigenvalues' mean and deviation (1.2-1.6 times the norm).  Against the
-// FP64 path, on tiles of 30 to 96 dates whose windows hold few more samples
-// than dates, the phase errors of certified pixels are C eps |A| / (gap
-// min|v|) with C at most 0.07 for H (the former solver: 0.61) and 0.91 for
-// Gamma (the former: 1.4): the scales keep the estimate below 5e-4 rad, half
-// the tolerance, with C = 0.5 and C = 1.25.  They hold for Gamma from half
-// pairs (22 bits).  bfloat16 pairs carry 16 bits, and H multiplies Gamma's
-// error by up to the square of |Gamma|'s inverse: there the wider scale of
-// the vector-unit solvers (kCertScale) leaves such pixels to the FP64 path,
-// whose coherence is its own.  297 x 43 pixels of 34 dates (EMI, 77 looks):
-// error against 64 bits 2.4e-5 -> 3.9e-6, 1.05 -> 2.59 ms.
-constexpr float kCertScaleEmi = 1.0e3f, kCertScaleEvd = 2.5e3f;
+// Certification distance: no eigenvalue may lie within scale eps |A| / min_t
+// |v_t| of the selected one, |A| bounded by the eigenvalues' mean and
+// deviation (1.2-1.6 times the norm).  A certified phase is then wrong by C /
+// scale at most, where C, the error times gap min|v| / (eps |A|), was measured
+// against the FP64 path on stacks of 5 to 96 dates and 12 to 130 looks, with
+// coherences that decay to 0, to 0.2, 0.9 and 0.99, noise alone, and two
+// scatterers.  Gamma keeps kCertScale: C is 1.8 at most (the tridiagonalising
+// FP32 solver's: 6.0).  For H below |H| = 100, C is 1.0 up to 8 dates, 0.5 up to
+// 12, 0.3 up to 20, 0.17 at 30, 0.08 at 48 and 0.03 at 96, a third to a seventh
+// of that solver's, so a scale of 3e3, falling as 1 / n from 48 dates on, keeps
+// to its worst error (3.7e-4 rad at 8 dates, 8e-5 at 30, 2e-5 from 48 on).  C
+// grows with the root of |H| beyond (Gamma's own error, multiplied by the
+// inverse of |Gamma|: 0.5 at 16 dates and |H| = 1000), and so does the scale,
+// up to kCertScale.  That holds for Gamma from half pairs (22 bits): bfloat16
+// pairs carry 16, and take kCertScale throughout.  Against kCertScale for H
+// everywhere: 46.6 k pixels of 48 dates 8.0 -> 4.0 ms, 65.5 k of 96 78 -> 53.5.
+constexpr float kCertScaleH = 3.0e3f;
+__device__ __forceinline__ float cert_eps(bool inv, float cert_h, float tn) {
+    const float most = kCertScale * Lim<float>::eps();
+    return inv ? fminf(cert_h * __builtin_amdgcn_sqrtf(fmaxf(0.01f * tn, 1.0f)), most) : most;
+}
 
 // Accumulator of a DIM x DIM matrix: NV registers, lane l holds column l % DIM
 // and, with h = l / DIM, rows row(v, h).
@@ -121,7 +128,7 @@ __device__ __forceinline__ float scal(float x) {   // a value alike in all lanes
     asm volatile("" : "+v"(x));   // (else the arithmetic is moved behind the read and stays in a vector register)
     return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(x)));
 }
-__device__ __forceinline__ double lit(double x) {   // a constant, likewise
+template <typename T> __device__ __forceinline__ T lit(T x) {   // a constant, likewise
     asm volatile("" : "+s"(x));
     return x;
 }
@@ -290,8 +297,8 @@ struct EigState {
 };
 
 // Inverse iteration with B^-1 = I - M: two plain products (the start vector
-// is far off), then normalised steps until the predicted error is below 4e-7,
-// or until the contraction proves worse than kSlow (moving the shift then
+// is far off), then normalised steps until the error predicted behind one more
+// (refine32's) is below 4e-7, or until the contraction proves worse than kSlow (moving the shift then
 // costs less than going on).
 constexpr float kSlow = 0.35f;
 constexpr int kNearInside = 1600000;   // |pivot| >= 0.1
@@ -321,7 +328,7 @@ __device__ __forceinline__ void iterate32(LdsMfma<DIM>& L, const typename Acc<DI
         E.done = false;
         if (!(dn < 3.0e38f)) return;   // not finite
         if (qb > 0.0f) {
-            E.done = dn * qb < 4.0e-7f * (1.0f - qb);
+            E.done = dn * qb * qb < 4.0e-7f * (1.0f - qb);
             if (E.done) return;
             continue;
         }
@@ -330,12 +337,78 @@ __device__ __forceinline__ void iterate32(LdsMfma<DIM>& L, const typename Acc<DI
             E.q = dn * __builtin_amdgcn_rcpf(dp);
             E.dq = dn;
             const float q = fminf(E.q, 0.99f);
-            if (dn * q < 4.0e-7f * (1.0f - q)) E.done = true;
+            if (dn * q * q < 4.0e-7f * (1.0f - q)) E.done = true;
             if (k > 1 && E.q > kSlow && dn > 2.0e-5f && !E.done) return;
         }
         if (E.done) return;
         dp = dn;
     }
+}
+
+// One step of inverse iteration in residual form: with y = A x, its Rayleigh
+// quotient t and r = y - t x, x becomes x - (A - sigma I)^-1 r.  The explicit
+// inverse is wrong by eps |A| / mu (mu: the shift's distance from the
+// eigenvalue), and so is the vector that iteration with it converges to;
+// here that error multiplies r alone, and what is left is of the order of
+// eps |A| / gap, as from a backward stable solver.  A = T o Gamma (HAD) or
+// Gamma, from memory, four rows at a time.  Returns the squared change.
+template <int DIM, bool HAD>
+__device__ __forceinline__ float refine32(LdsMfma<DIM>& L, const GammaBuf& gam, const typename Acc<DIM>::type& R,
+                                         const typename Acc<DIM>::type& I, int n, int col, int h, int band, float sg,
+                                         EigState& E) {
+    if (h == 0) {
+        L.xr[col] = E.x.re;
+        L.xi[col] = E.x.im;
+    }
+    wsync();
+    float re = 0.0f, im = 0.0f;
+    int o = fresh_lane(gam.offset(4 * h, col));
+    const int d0 = fresh_lane(col - 4 * h);   // column - row of register 0
+#pragma unroll
+    for (int q = 0; q < Acc<DIM>::NV / 4; ++q) {
+        const float4 xr = *(const float4*)&L.xr[8 * q + 4 * h], xi = *(const float4*)&L.xi[8 * q + 4 * h];
+        const float pr[4] = {xr.x, xr.y, xr.z, xr.w}, pi[4] = {xi.x, xi.y, xi.z, xi.w};
+        float m[4] = {1.0f, 1.0f, 1.0f, 1.0f};
+        if constexpr (HAD) {
+            const float4 t = *(const float4*)&L.T[col * LdsMfma<DIM>::S + 8 * q + 4 * h];
+            m[0] = t.x; m[1] = t.y; m[2] = t.z; m[3] = t.w;
+        }
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+            const cx<float> g = gam.at(o);
+            o += (b == 3 ? 5 : 1) * n * 8;
+            const bool out = band > 0 && abs(8 * q + b - d0) > band;
+            const float ar = out ? 0.0f : g.re * m[b], ai = out ? 0.0f : g.im * m[b];
+            re = fmaf(ar, pr[b], re);
+            im = fmaf(ar, pi[b], im);
+            re = fmaf(ai, pi[b], re);
+            im = fmaf(-ai, pr[b], im);
+        }
+    }
+    wsync();
+    const cx<float> y = {sumH<DIM>(re), sumH<DIM>(im)};
+    const float t = uni(redC<DIM, OpAdd>(y.re * E.x.re + y.im * E.x.im));
+    const cx<float> r = {fmaf(-t, E.x.re, y.re), fmaf(-t, E.x.im, y.im)};
+    cx<float> z = csub(r, apply32<DIM>(L, R, I, r, col, h));
+    // along x the change means nothing (and is rounding, blown up by 1 / mu)
+    const float cr = uni(redC<DIM, OpAdd>(E.x.re * z.re + E.x.im * z.im));
+    const float ci = uni(redC<DIM, OpAdd>(E.x.re * z.im - E.x.im * z.re));
+    z = cx<float>{fmaf(-cr, E.x.re, fmaf(ci, E.x.im, z.re)), fmaf(-cr, E.x.im, fmaf(-ci, E.x.re, z.im))};
+    const float d2 = uni(redC<DIM, OpAdd>(cabs2(z)));
+    const float s = __builtin_amdgcn_rsqf(1.0f + d2);
+    E.x = cx<float>{fmaf(-sg, z.re, E.x.re) * s, fmaf(-sg, z.im, E.x.im) * s};
+    return d2;
+}
+// Steps (nearly always one) until one changes the vector so little that what
+// is left turns no component (of square m2 at least) by more than 4e-5 rad: a
+// step leaves the contraction qb, and the inverse's relative error (rel: |A| /
+// mu, in units of eps), of the error that it meets.  A vector that kRefines
+// steps do not settle is not certified.
+constexpr int kRefines = 4;
+__device__ __forceinline__ float refined2(float m2, float qb, float rel) {
+    const float q = qb + 8.0f * Lim<float>::eps() * rel;
+    const float k = 4.0e-5f * fmaxf(1.0f - q, 0.0f) * __builtin_amdgcn_rcpf(q);
+    return fmaxf(k * k * m2, 2.5e-13f);
 }
 
 // FP64 sweep of |Gamma| (diagonal stored minus 1, padding rows and columns
@@ -528,6 +601,10 @@ __device__ __forceinline__ void solve_mfma_pixel(const SolveArgs& a, LdsMfma<DIM
         const float dg = inv ? (in ? L.T[col * S + col] : 0.0f) : 1.0f;
         if (!inv) {
             sg = -1.0f;
+            if constexpr (MODE == MODE_EMI) {   // Gamma = T o Gamma
+                for (int e = lane; e < DIM * S; e += 64) L.T[e] = 1.0f;
+                wsync();
+            }
             acc R, I;
             load_gamma32<DIM>(gam, n, col, h, R, I);
             float f2 = 0.0f, sum = 0.0f;
@@ -627,7 +704,7 @@ __device__ __forceinline__ void solve_mfma_pixel(const SolveArgs& a, LdsMfma<DIM
                 }
                 // ---- certification ----
                 const float m2 = redC<DIM, OpMin>(in ? cabs2(E.x) : 3.0e38f);
-                delta = (inv ? kCertScaleEmi : kCertScaleEvd) * a.cert_eps * tn * __builtin_amdgcn_rsqf(uni(m2));
+                delta = cert_eps(inv, a.cert_h, tn) * tn * __builtin_amdgcn_rsqf(uni(m2));
                 if (!(delta <= tn)) break;
                 // Frobenius norm of the inverse: its other eigenvalues'
                 // squares sum to S2, so none of them exceeds sqrt(S2)
@@ -646,16 +723,21 @@ __device__ __forceinline__ void solve_mfma_pixel(const SolveArgs& a, LdsMfma<DIM
                 // the contraction is at most qb: the error left by the last step
                 const float qb = __builtin_amdgcn_sqrtf(s2) * fabsf(mu);
                 bool conv = qb < 0.8f;
-                if (conv && E.dn * qb > 4.0e-7f * (1.0f - qb)) {
+                if (conv && E.dn * qb * qb > 4.0e-7f * (1.0f - qb)) {
                     iterate32<DIM>(L, R, I, col, h, qb, E);
                     conv = E.done;
                 }
                 // a shift inside the spectrum: small pivots would have cost accuracy
                 if (neg != 0 && near < kNearInside && !close) conv = false;
-                if (conv && (t <= 0.0f || s2 * t * t < 1.0f)) {
-                    certified = true;
-                    break;
+                certified = conv && (t <= 0.0f || s2 * t * t < 1.0f);
+                if (certified || (conv && close)) {
+                    const float most = refined2(uni(m2), qb, tn * fabsf(E.theta));
+                    float d2 = 1.0f;
+                    for (int k = 0; k < kRefines && d2 > most; ++k)
+                        d2 = refine32<DIM, MODE != MODE_EVD>(L, gam, R, I, n, col, h, stbas ? a.bw : 0, sg, E);
+                    if (!(d2 <= most)) certified = conv = false;
                 }
+                if (certified) break;
                 // the next eigenvalue as the measured contraction places it is
                 // too close for any certificate: the FP64 path's pixel
                 if (E.q > 0.02f && E.dq > 4.0e-6f && fabsf(mu) * __builtin_amdgcn_rcpf(E.q) - mu < 0.7f * delta) break;

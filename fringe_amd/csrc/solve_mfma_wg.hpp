@@ -35,7 +35,6 @@ template <int NT, bool INV> struct LdsMfmaWg {
     };
     float xr[NT][32], xi[NT][32];
     double red[2][NT][2];
-    float cert_eps;                      // SolveArgs::cert_eps
 };
 
 // Sum of x (alike in the wave's lanes) over the workgroup's waves.
@@ -185,7 +184,7 @@ template <int NT, bool INV>
 __device__ __forceinline__ void iterate_wg(LdsMfmaWg<NT, INV>& L, const Tiles<NT>& R, const Tiles<NT>& I, int w,
                                            int col, int h, int& turn, float qb, EigStateWg<NT>& E) {
     float dp = 0.0f;
-    const float left = scal(4.0e-7f * (1.0f - qb));
+    const float left = scal(4.0e-7f * (1.0f - qb)), qq = scal(qb * qb);
     if (!(qb > 0.0f)) E.q = E.dq = 0.0f;
     cx<float> y[NT];
     for (int k = qb > 0.0f ? 0 : -2; k < 24; ++k) {
@@ -203,7 +202,7 @@ __device__ __forceinline__ void iterate_wg(LdsMfmaWg<NT, INV>& L, const Tiles<NT
         E.done = false;
         if (!(dn < 3.0e38f)) return;   // not finite
         if (qb > 0.0f) {
-            E.done = dn * qb < left;
+            E.done = dn * qq < left;
             if (E.done) return;
             continue;
         }
@@ -212,7 +211,7 @@ __device__ __forceinline__ void iterate_wg(LdsMfmaWg<NT, INV>& L, const Tiles<NT
             E.q = dn * __builtin_amdgcn_rcpf(dp);
             E.dq = dn;
             const float q = fminf(E.q, 0.99f);
-            if (dn * q < 4.0e-7f * (1.0f - q)) E.done = true;
+            if (dn * q * q < 4.0e-7f * (1.0f - q)) E.done = true;
             if (k > 1 && E.q > kSlow && dn > 2.0e-5f && !E.done) return;
         }
         if (E.done) return;
@@ -331,6 +330,83 @@ __device__ __forceinline__ int diagonal_wg(int col, int h) {
     return ((col >> 2) & 1) == h ? 4 * (col >> 3) + (col & 3) : -1;
 }
 
+// The step in residual form, as refine32; A = T o Gamma (INV) or Gamma.
+template <int NT, bool INV>
+__device__ __forceinline__ float refine_wg(LdsMfmaWg<NT, INV>& L, const GammaBuf& gam, const Tiles<NT>& R,
+                                          const Tiles<NT>& I, int n, int w, int band, float sg, int& turn,
+                                          EigStateWg<NT>& E) {
+    const int lane = lane_now(), col = lane & 31, h = lane >> 5;
+#pragma unroll
+    for (int J = 0; J < NT; ++J)
+        if (J == w && h == 0) {
+            L.xr[w][col] = E.x[J].re;
+            L.xi[w][col] = E.x[J].im;
+        }
+    wsync();
+    turn ^= 1;
+#pragma unroll
+    for (int J = 0; J < NT; ++J) {
+        int o = fresh_lane(gam.offset(32 * w + 4 * h, 32 * J + col));
+        const int d0 = fresh_lane(col - 4 * h - 32 * w);
+        float re = 0.0f, im = 0.0f;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const float4 xr = *(const float4*)&L.xr[w][8 * q + 4 * h], xi = *(const float4*)&L.xi[w][8 * q + 4 * h];
+            const float pr[4] = {xr.x, xr.y, xr.z, xr.w}, pi[4] = {xi.x, xi.y, xi.z, xi.w};
+            float m[4] = {1.0f, 1.0f, 1.0f, 1.0f};
+            if constexpr (INV) {
+                const float4 t = *(const float4*)&L.T[(32 * J + col) * LdsMfmaWg<NT, INV>::S + 32 * w + 8 * q + 4 * h];
+                m[0] = t.x; m[1] = t.y; m[2] = t.z; m[3] = t.w;
+            }
+#pragma unroll
+            for (int b = 0; b < 4; ++b) {
+                const cx<float> g = gam.at(o);
+                o += (b == 3 ? 5 : 1) * n * 8;
+                const bool out = !INV && band > 0 && abs(8 * q + b - d0 - 32 * J) > band;
+                const float ar = out ? 0.0f : g.re * m[b], ai = out ? 0.0f : g.im * m[b];
+                re = fmaf(ar, pr[b], re);
+                im = fmaf(ar, pi[b], im);
+                re = fmaf(ai, pi[b], re);
+                im = fmaf(-ai, pr[b], im);
+            }
+            __builtin_amdgcn_sched_barrier(0);   // four rows' loads in flight (more of them spilled)
+        }
+        const cx<float> s = {both32(re), both32(im)};
+        if (h == 0) L.part[turn][w][32 * J + col] = s;
+    }
+    __syncthreads();
+    cx<float> r[NT], z[NT];
+    float t = 0.0f;
+#pragma unroll
+    for (int J = 0; J < NT; ++J) {
+        r[J] = L.part[turn][0][32 * J + col];
+#pragma unroll
+        for (int k = 1; k < NT; ++k) r[J] = cadd(r[J], L.part[turn][k][32 * J + col]);
+        t = fmaf(r[J].re, E.x[J].re, fmaf(r[J].im, E.x[J].im, t));
+    }
+    t = uni(red32<OpAdd>(t));
+#pragma unroll
+    for (int J = 0; J < NT; ++J) r[J] = cx<float>{fmaf(-t, E.x[J].re, r[J].re), fmaf(-t, E.x[J].im, r[J].im)};
+    apply_wg<NT, INV>(L, R, I, r, z, w, col, h, turn);
+    float cr = 0.0f, ci = 0.0f;   // along x the change means nothing
+#pragma unroll
+    for (int J = 0; J < NT; ++J) {
+        z[J] = csub(r[J], z[J]);
+        cr = fmaf(E.x[J].re, z[J].re, fmaf(E.x[J].im, z[J].im, cr));
+        ci = fmaf(E.x[J].re, z[J].im, fmaf(-E.x[J].im, z[J].re, ci));
+    }
+    cr = uni(red32<OpAdd>(cr));
+    ci = uni(red32<OpAdd>(ci));
+#pragma unroll
+    for (int J = 0; J < NT; ++J)
+        z[J] = cx<float>{fmaf(-cr, E.x[J].re, fmaf(ci, E.x[J].im, z[J].re)),
+                         fmaf(-cr, E.x[J].im, fmaf(-ci, E.x[J].re, z[J].im))};
+    const float d2 = norm2_wg<NT>(z), s = __builtin_amdgcn_rsqf(1.0f + d2);
+#pragma unroll
+    for (int J = 0; J < NT; ++J) E.x[J] = cx<float>{fmaf(-sg, z[J].re, E.x[J].re) * s, fmaf(-sg, z[J].im, E.x[J].im) * s};
+    return d2;
+}
+
 // One pixel on the NT waves of a workgroup.
 template <int MODE, int NT>
 __device__ __forceinline__ void solve_mfma_wg_pixel(const SolveArgs& a, LdsMfmaWg<NT, MODE != MODE_EVD>& L, int w,
@@ -346,8 +422,6 @@ __device__ __forceinline__ void solve_mfma_wg_pixel(const SolveArgs& a, LdsMfmaW
     EigStateWg<NT> E;
 
     const bool act = np >= 0;
-    // read behind the sweep's barriers; held in a register it spilled
-    if (threadIdx.x == 0) L.cert_eps = a.cert_eps;
     // What follows from the lane is computed again in each stage: held over
     // the sweeps it spilled.
     if (act) {
@@ -446,6 +520,9 @@ __device__ __forceinline__ void solve_mfma_wg_pixel(const SolveArgs& a, LdsMfmaW
         }
         if (!inv) {
             sg = -1.0f;
+            if constexpr (INV) {   // EMI's fallback: Gamma = T o Gamma (read behind the sum's barrier)
+                for (int e = threadIdx.x; e < LdsMfmaWg<NT, INV>::N * S; e += 64 * NT) L.T[e] = 1.0f;
+            }
             Tiles<NT> R, I;
             load_gamma_wg<NT>(gam, n, w, col, h, R, I);
             const int d0 = col - 4 * h - 32 * w;   // column - row of register 0 of tile 0
@@ -530,15 +607,27 @@ __device__ __forceinline__ void solve_mfma_wg_pixel(const SolveArgs& a, LdsMfmaW
                         tile_fence_wg<NT>();
                     }
                 }
+                // the vector waits in LDS (behind the sweep's barriers) for the
+                // registers that the sweep needs
+#pragma unroll
+                for (int J = 0; J < NT; ++J)
+                    if (J == w && h == 0) {
+                        L.xr[w][col] = E.x[J].re;
+                        L.xi[w][col] = E.x[J].im;
+                    }
                 int neg, near;
                 sweep_wg<NT, INV>(L, R, I, n, w, lane, neg, near);
+#pragma unroll
+                for (int J = 0; J < NT; ++J) E.x[J] = cx<float>{L.xr[J][col], L.xi[J][col]};
                 if (checking) {
                     certified = neg <= 1 && near >= 1700;
+                    __syncthreads();   // the outputs take the vector's place
                     break;
                 }
                 if (neg > 1) {
                     if (inv) sigma = sigma > 0.5f ? 0.5f * sigma : 0.0f;
                     else sigma = sigma * 1.15f;
+                    sigma = scal(sigma);
                     continue;
                 }
                 iterate_wg<NT, INV>(L, R, I, w, col, h, turn, 0.0f, E);
@@ -553,12 +642,12 @@ __device__ __forceinline__ void solve_mfma_wg_pixel(const SolveArgs& a, LdsMfmaW
                     continue;
                 }
                 // ---- certification ----
-                float m2 = 3.0e38f;
+                float m2 = lit(3.0e38f);   // smallest component
 #pragma unroll
                 for (int J = 0; J < NT; ++J)
                     if (32 * J + col < n) m2 = fminf(m2, cabs2(E.x[J]));
-                delta = scal((inv ? kCertScaleEmi : kCertScaleEvd) * L.cert_eps *
-                             (tn * __builtin_amdgcn_rsqf(uni(red32<OpMin>(m2)))));
+                m2 = scal(red32<OpMin>(m2));
+                delta = scal(cert_eps(inv, a.cert_h, tn) * (tn * __builtin_amdgcn_rsqf(m2)));
                 if (!(delta <= tn)) break;
                 float f = 0.0f;
 #pragma unroll
@@ -576,27 +665,32 @@ __device__ __forceinline__ void solve_mfma_wg_pixel(const SolveArgs& a, LdsMfmaW
                 // the contraction is at most qb: the error left by the last step
                 const float qb = scal(__builtin_amdgcn_sqrtf(s2) * fabsf(mu));
                 bool conv = qb < 0.8f;
-                if (conv && E.dn * qb > 4.0e-7f * (1.0f - qb)) {
+                if (conv && E.dn * qb * qb > 4.0e-7f * (1.0f - qb)) {
                     iterate_wg<NT, INV>(L, R, I, w, col, h, turn, qb, E);
                     conv = E.done;
                 }
                 // a shift inside the spectrum: small pivots would have cost accuracy
                 if (neg != 0 && near < kNearInside && !close) conv = false;
-                if (conv && (t <= 0.0f || s2 * t * t < 1.0f)) {
-                    certified = true;
-                    break;
+                certified = conv && (t <= 0.0f || s2 * t * t < 1.0f);
+                if (certified || (conv && close)) {
+                    const float most = scal(refined2(m2, qb, tn * fabsf(E.theta)));
+                    float d2 = 1.0f;
+                    for (int k = 0; k < kRefines && d2 > most; ++k)
+                        d2 = scal(refine_wg<NT, INV>(L, gam, R, I, fresh(n), w, stbas ? a.bw : 0, sg, turn, E));
+                    if (!(d2 <= most)) certified = conv = false;
                 }
+                if (certified) break;
                 // the next eigenvalue as the measured contraction places it is
                 // too close for any certificate: the FP64 path's pixel
                 if (E.q > 0.02f && E.dq > 4.0e-6f && fabsf(mu) * __builtin_amdgcn_rcpf(E.q) - mu < 0.7f * delta) break;
                 if (!close) {   // once more from a quarter of the distance away
                     close = true;
-                    sigma = lam - sg * (0.25f * delta);
+                    sigma = scal(lam - sg * (0.25f * delta));
                     continue;
                 }
                 if (!conv) break;
                 checking = true;
-                sigma = lam + sg * delta;
+                sigma = scal(lam + sg * delta);
             }
         if constexpr (MODE != MODE_EMI) unc = unc || !(lam >= 1.0e-6f + kCertThrMargin * Lim<float>::eps() * tn);
         unc = code == 0.0f && (unc || !certified);

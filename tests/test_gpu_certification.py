@@ -52,3 +52,26 @@ def test_emi_fallback_keeps_no_close_pair(n, Nx, Ny):
     short = (lam[:, -1] - lam[:, -2]) * least / (2500 * EPS * lam[:, -1])
     print(f"{at.size} kept, smallest distance {short.min():.2f} of the certificate's")
     assert short.min() >= 0.9
+
+
+@pytest.mark.parametrize("n,Nx,Ny,g0,ginf", [(8, 2, 1, 0.97, 0.9), (12, 2, 1, 0.97, 0.9), (12, 2, 1, 0.998, 0.99),
+                                             (16, 2, 1, 0.97, 0.9), (20, 2, 1, 0.97, 0.9), (25, 3, 2, 0.97, 0.9),
+                                             (12, 2, 1, 0.8, 0.2), (30, 4, 2, 0.8, 0.2), (48, 5, 5, 0.8, 0.2),
+                                             (64, 7, 5, 0.8, 0.2), (96, 7, 5, 0.8, 0.2), (96, 2, 1, 0.97, 0.9)])
+@pytest.mark.parametrize("est", ["EMI", "EVD"])
+def test_kept_pixels_meet_the_estimate(n, Nx, Ny, g0, ginf, est):
+    """Every phase of a pixel kept in FP32 is within 5e-4 rad (the estimate a
+    certified result stays below) of the FP64 path's, also where |Gamma| is
+    nearly singular: high coherence, few looks."""
+    rows, cols = (96, 112) if n <= 32 else (40, 48)
+    print(f"case estimate n={n} {2 * Nx + 1}x{2 * Ny + 1} coherence {g0} to {ginf} {est}", flush=True)
+    slc = synthetic.stack(n, rows, cols, seed=40 + n, coh=synthetic.coherence_matrix(n, g0=g0, ginf=ginf))
+    ds, w = to_dev(slc, torch), _mask(rows, cols, Nx, Ny)
+    kw = dict(module="phase_link" if est == "EMI" else "evd", method="MLE" if est == "EMI" else est, min_neighbors=2)
+    want, _ = _link(ds, w, Nx, Ny, "fp64", **kw)
+    got, kept = _link(ds, w, Nx, Ny, "mixed", **kw)
+    assert kept.sum() > 20
+    err = np.abs(np.angle(got[0] * want[0].conj())).max(axis=0).reshape(-1)[kept]
+    print(f"kept {kept.sum()} of {rows * cols}: max {err.max():.1e}, rms {np.sqrt((err ** 2).mean()):.1e}")
+    assert err.max() <= 5.0e-4
+    assert np.array_equal(np.minimum(got[1], 0.0), np.minimum(want[1], 0.0))   # the same error codes
