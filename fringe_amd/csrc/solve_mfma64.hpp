@@ -18,7 +18,8 @@
 //
 // There is no other path to leave a pixel to, so the search for the extreme
 // eigenpair goes on until the inertia and the Frobenius norm of the inverse
-// show that it is the extreme one.
+// show that it is the extreme one, or 36 shifts have narrowed it down to a
+// cluster of eigenvalues, one of whose vectors is the result.
 //
 // Bound by the FP64 matrix instructions and, per pivot panel, by the chain
 // publish, barrier, read, pivot inverse.  Solve stage against the vector-unit
@@ -285,6 +286,7 @@ __device__ __forceinline__ double step_64(Eig64<NW>& E, const cx<double> (&y)[Ei
 // Inverse iteration with B^-1 = I - M (see iterate_wg; the predicted error
 // goes below 1e-11).
 constexpr double kTol64 = 1.0e-11;
+constexpr int kRounds64 = 36;
 template <int NW>
 __device__ __forceinline__ void iterate_64(LdsMfma64<NW>& L, const Tiles64<NW>& R, const Tiles64<NW>& I, int w, int lane,
                                            int& turn, double qb, int most, Eig64<NW>& E) {
@@ -487,7 +489,8 @@ __device__ __forceinline__ void solve_mfma64_pixel(const SolveArgs& a, LdsMfma64
             f2 = wg_sum64<NW>(L, w, turn, uni(sumR<64>(f2))).re;
             if (!(f2 < 1.0e300)) code = -6;
             // no eigenvalue lies above the mean, 1, plus sqrt(n - 1) deviations
-            good = 1.0 + sqrt(fmax(f2 * (1.0 / n) - 1.0, 0.0) * (double)(n - 1)) + 1.0e-9;
+            // (1e-14: what rounding can take from the squared deviation)
+            good = 1.0 + sqrt((fmax(f2 * (1.0 / n) - 1.0, 0.0) + lit(1.0e-14)) * (double)(n - 1)) + 1.0e-9;
             up = -1.0e300;
             if (code == 0) {
                 cx<double> y[NC];
@@ -501,10 +504,15 @@ __device__ __forceinline__ void solve_mfma64_pixel(const SolveArgs& a, LdsMfma64
         }
         double lam = 0.0;
         // Each round sweeps at one shift; the bracket (good, up] halves at
-        // least wherever the suggested shift leaves it, so the rounds end with
-        // the extreme eigenvalue isolated, or (a pair closer than rounding)
-        // with a vector of its eigenspace.
+        // least wherever the suggested shift leaves it, so the rounds isolate
+        // the extreme eigenvalue, unless it is nearly a multiple one.  The last
+        // rounds then take the bracket's end that no eigenvalue lies before (a
+        // little further out each), and the vector of the eigenspace that
+        // iteration from there finds.
+        bool found = false;
         for (int att = 0; att < 40 && code == 0; ++att) {
+            const bool late = att >= kRounds64;
+            if (late) sigma = good - sg * lit(1.0e-9) * (1.0 + fabs(good)) * (double)(1 << 6 * (att - kRounds64));
             // ---- B = +-(A - sigma I), diagonal stored minus 1 ----
             Tiles64<NW> R, I;
             const int lane = fresh_lane(lane_in), c16 = lane & 15, q = lane >> 4;
@@ -545,9 +553,14 @@ __device__ __forceinline__ void solve_mfma64_pixel(const SolveArgs& a, LdsMfma64
             int neg;
             double pm;
             sweep_c64<NW>(L, R, I, n, w, lane, neg, pm);
-            if (neg == 0) good = sg * (sigma - good) > 0.0 ? sigma : good;
-            else up = sg * (sigma - up) < 0.0 ? sigma : up;
             double next;   // the next shift, from the two eigenvalues next to this one
+            if (late) {
+                if (neg != 0) continue;
+            } else if (neg == 0) {
+                good = sg * (sigma - good) > 0.0 ? sigma : good;
+            } else {
+                up = sg * (sigma - up) < 0.0 ? sigma : up;
+            }
             if (neg > 1) {
                 next = 0.5 * (good + sigma);
             } else {
@@ -562,10 +575,12 @@ __device__ __forceinline__ void solve_mfma64_pixel(const SolveArgs& a, LdsMfma64
                     if (__any(bad)) fresh_start(0);
                     continue;
                 }
+                found = late;
+                if (found) break;
                 if (neg == 0 ? E.theta < 0.0 : E.theta > 0.0) {   // not the extreme one: it lies before the shift
                     fresh_start(att + 1);
                     next = 0.5 * (good + sigma);
-                } else if (!E.done && att < 36) {   // as in solve_mfma_pixel
+                } else if (!E.done) {   // as in solve_mfma_pixel
                     const double qq = E.q > 0.0 ? fmin(fmax(E.q, 1.0e-3), 0.98) : 0.98;
                     const double gap = fabs(mu) / qq - mu;
                     const double e = fmin(E.dn * qq / (1.0 - qq), 1.0);
@@ -584,9 +599,9 @@ __device__ __forceinline__ void solve_mfma64_pixel(const SolveArgs& a, LdsMfma64
                         }
                     f = wg_sum64<NW>(L, w, turn, uni(sumR<64>(f))).re;
                     const double qb = sqrt(fmax(f - E.theta * E.theta, 0.0)) * fabs(mu);
-                    if (qb < lit(0.8) || att >= 36) {
-                        if (qb < lit(0.8) && E.dn * qb > kTol64 * (1.0 - qb))
-                            iterate_64<NW>(L, R, I, w, lane, turn, qb, 60, E);
+                    found = qb < lit(0.8);
+                    if (found) {
+                        if (E.dn * qb > kTol64 * (1.0 - qb)) iterate_64<NW>(L, R, I, w, lane, turn, qb, 60, E);
                         break;
                     }
                     next = lam - sg * lit(0.1) * fabs(mu);   // closer, and before it
@@ -596,6 +611,7 @@ __device__ __forceinline__ void solve_mfma64_pixel(const SolveArgs& a, LdsMfma64
             const double in0 = sg * (next - good), in1 = sg * (up - next);
             sigma = in0 > 0.0 && in1 > 0.0 ? next : fabs(up) < 1.0e299 ? 0.5 * (good + up) : good;
         }
+        if (code == 0 && !found) code = MODE == MODE_EMI ? -1 : -6;   // (nothing but a matrix that is not finite)
         if (MODE != MODE_EMI && code == 0 && !(lam >= 1.0e-6)) code = -7;
     }
 
