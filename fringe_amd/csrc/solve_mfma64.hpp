@@ -284,12 +284,13 @@ __device__ __forceinline__ double step_64(Eig64<NW>& E, const cx<double> (&y)[Ei
 }
 
 // Inverse iteration with B^-1 = I - M (see iterate_wg; the predicted error
-// goes below 1e-11).
+// goes below 1e-11, or tol when polishing).
 constexpr double kTol64 = 1.0e-11;
 constexpr int kRounds64 = 36;
 template <int NW>
 __device__ __forceinline__ void iterate_64(LdsMfma64<NW>& L, const Tiles64<NW>& R, const Tiles64<NW>& I, int w, int lane,
-                                           int& turn, double qb, int most, Eig64<NW>& E) {
+                                           int& turn, double qb, int most, Eig64<NW>& E,
+                                           double tol = kTol64) {
     constexpr int NC = Eig64<NW>::NC;
     double dp = 0.0;
     if (!(qb > 0.0)) E.q = 0.0;
@@ -310,7 +311,7 @@ __device__ __forceinline__ void iterate_64(LdsMfma64<NW>& L, const Tiles64<NW>& 
         E.done = false;
         if (!(dn < 1.0e300)) return;   // not finite
         if (qb > 0.0) {
-            E.done = dn * qb < kTol64 * (1.0 - qb);
+            E.done = dn * qb < tol * (1.0 - qb);
             if (E.done) return;
             continue;
         }
@@ -601,7 +602,15 @@ __device__ __forceinline__ void solve_mfma64_pixel(const SolveArgs& a, LdsMfma64
                     const double qb = sqrt(fmax(f - E.theta * E.theta, 0.0)) * fabs(mu);
                     found = qb < lit(0.8);
                     if (found) {
-                        if (E.dn * qb > kTol64 * (1.0 - qb)) iterate_64<NW>(L, R, I, w, lane, turn, qb, 60, E);
+                        // no phase off by more than 1e-8 rad: a component
+                        // below 1e-3 takes more than kTol64
+                        double m2 = 1.0;
+#pragma unroll
+                        for (int t = 0; t < NC; ++t)
+                            if (lane + 64 * t < n) m2 = fmin(m2, cabs2(E.x[t]));
+                        m2 = uni(minR<64>(m2));
+                        const double tol = fmin(kTol64, fmax(lit(1.0e-8) * sqrt(m2), lit(2.0e-15)));
+                        if (E.dn * qb > tol * (1.0 - qb)) iterate_64<NW>(L, R, I, w, lane, turn, qb, 60, E, tol);
                         break;
                     }
                     next = lam - sg * lit(0.1) * fabs(mu);   // closer, and before it
