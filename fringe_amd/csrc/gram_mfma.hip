@@ -703,11 +703,23 @@ gram_mfma_lds(MfmaArgs a) {
         for (int e = cnt + lane; e < steps * 32; e += 64) list[place(e)] = where(NPOS);
         wave_sync_lds();
 
-        f32x4 A[NB], X[NB], W[NB], P[PAIRS ? PAIRS : 1], Q[PAIRS ? PAIRS : 1];
+        // A rounding of a large sum costs more than one of a small: Im Im' has
+        // a sum of its own, and so have the halves' cross products (2^-11 of
+        // the others) of the pairs.  Where the registers do not hold those,
+        // 32 positions are summed by themselves and then added.  (One sum for
+        // all: coherence error 1.01 to 1.16 times that of the four real
+        // products of 32 x 32 x 16, now 0.88 to 1.01; 160 x 219 pixels of 40
+        // dates 200 -> 201 us.)
+        constexpr bool OWN = NB <= 3, KEEP = NB == 3;
+        f32x4 A[NB], B[NB], X[NB], W[NB], P[PAIRS ? PAIRS : 1], Q[PAIRS ? PAIRS : 1];
+        f32x4 PL[KEEP && PAIRS ? PAIRS : 1], QL[KEEP && PAIRS ? PAIRS : 1];
 #pragma unroll
-        for (int b = 0; b < NB; ++b) A[b] = X[b] = W[b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int b = 0; b < NB; ++b) A[b] = B[b] = X[b] = W[b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-        for (int t = 0; t < PAIRS; ++t) P[t] = Q[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int t = 0; t < PAIRS; ++t) {
+            P[t] = Q[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            if constexpr (KEEP) PL[t] = QL[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        }
         // operands of step st + 1 are loaded while step st's MFMAs run; one
         // 8-byte read gives this lane's (re, im) words of a position
         uint2 x[NB][8];
@@ -747,18 +759,22 @@ gram_mfma_lds(MfmaArgs a) {
             // interleaved so that consecutive MFMAs feed different accumulators
 #pragma unroll
             for (int b = 0; b < NB; ++b) {
-                A[b] = mfma16<F16>(Rh[b], Rh[b], A[b]);
+                B[b] = OWN ? B[b] : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                (OWN ? A[b] : B[b]) = mfma16<F16>(Rh[b], Rh[b], OWN ? A[b] : B[b]);
                 X[b] = mfma16<F16>(Rh[b], Rl[b], X[b]);
                 W[b] = mfma16<F16>(Ih[b], Rh[b], W[b]);
             }
 #pragma unroll
             for (int b = 0; b < NB; ++b) {
-                A[b] = mfma16<F16>(Ih[b], Ih[b], A[b]);
+                B[b] = mfma16<F16>(Ih[b], Ih[b], B[b]);
                 X[b] = mfma16<F16>(Ih[b], Il[b], X[b]);
                 W[b] = mfma16<F16>(Ih[b], Rl[b], W[b]);
             }
 #pragma unroll
-            for (int b = 0; b < NB; ++b) W[b] = mfma16<F16>(Il[b], Rh[b], W[b]);
+            for (int b = 0; b < NB; ++b) {
+                W[b] = mfma16<F16>(Il[b], Rh[b], W[b]);
+                if constexpr (!OWN) A[b] += B[b];
+            }
             int t = 0;
 #pragma unroll
             for (int b = 0; b < NB - 1; ++b) {
@@ -767,18 +783,29 @@ gram_mfma_lds(MfmaArgs a) {
                 const frag_t Nl = __builtin_bit_cast(frag_t, __builtin_bit_cast(u32x4, Rl[b]) ^ sign);
 #pragma unroll
                 for (int d = b + 1; d < NB; ++d, ++t) {   // P(im_b, re_d) - P(re_b, im_d) is Im G
-                    P[t] = mfma16<F16>(Rh[b], Rh[d], P[t]);
-                    Q[t] = mfma16<F16>(Ih[b], Rh[d], Q[t]);
-                    P[t] = mfma16<F16>(Rh[b], Rl[d], P[t]);
-                    Q[t] = mfma16<F16>(Ih[b], Rl[d], Q[t]);
-                    P[t] = mfma16<F16>(Rl[b], Rh[d], P[t]);
-                    Q[t] = mfma16<F16>(Il[b], Rh[d], Q[t]);
-                    P[t] = mfma16<F16>(Ih[b], Ih[d], P[t]);
-                    Q[t] = mfma16<F16>(Nh, Ih[d], Q[t]);
-                    P[t] = mfma16<F16>(Ih[b], Il[d], P[t]);
-                    Q[t] = mfma16<F16>(Nh, Il[d], Q[t]);
-                    P[t] = mfma16<F16>(Il[b], Ih[d], P[t]);
-                    Q[t] = mfma16<F16>(Nl, Ih[d], Q[t]);
+                    f32x4 p = f32x4{0.0f, 0.0f, 0.0f, 0.0f}, q = p, pl = p, ql = p;
+                    if constexpr (KEEP) p = P[t], q = Q[t], pl = PL[t], ql = QL[t];
+                    p = mfma16<F16>(Rh[b], Rh[d], p);
+                    q = mfma16<F16>(Ih[b], Rh[d], q);
+                    pl = mfma16<F16>(Rh[b], Rl[d], pl);
+                    ql = mfma16<F16>(Ih[b], Rl[d], ql);
+                    p = mfma16<F16>(Ih[b], Ih[d], p);
+                    q = mfma16<F16>(Nh, Ih[d], q);
+                    pl = mfma16<F16>(Rl[b], Rh[d], pl);
+                    ql = mfma16<F16>(Il[b], Rh[d], ql);
+                    pl = mfma16<F16>(Ih[b], Il[d], pl);
+                    ql = mfma16<F16>(Nh, Il[d], ql);
+                    pl = mfma16<F16>(Il[b], Ih[d], pl);
+                    ql = mfma16<F16>(Nl, Ih[d], ql);
+                    if constexpr (KEEP) {
+                        P[t] = p;
+                        Q[t] = q;
+                        PL[t] = pl;
+                        QL[t] = ql;
+                    } else {
+                        P[t] += p + pl;
+                        Q[t] += q + ql;
+                    }
                 }
             }
         }
@@ -786,6 +813,10 @@ gram_mfma_lds(MfmaArgs a) {
         if (lane < kStageWords) wbuf[lane] = wnext;   // waits for the load here, before the stores below
 
         // ---- fold into Gamma ----
+        if constexpr (OWN) {
+#pragma unroll
+            for (int b = 0; b < NB; ++b) A[b] += B[b];
+        }
         // Re G_mm sits in register m % 4 of the lanes of quarter m / 4; it is
         // published as 1 / sqrt: one transcendental per lane, and the
         // normalisation of entry (i, j) is a product
@@ -821,6 +852,10 @@ gram_mfma_lds(MfmaArgs a) {
             put(b, b, A[b] + (X[b] + transpose16(X[b], lane)), W[b] - transpose16(W[b], lane));
 #pragma unroll
             for (int d = b + 1; d < NB; ++d, ++t) {
+                if constexpr (KEEP) {
+                    P[t] += PL[t];
+                    Q[t] += QL[t];
+                }
                 put(b, d, P[t], Q[t]);
                 put(d, b, transpose16(P[t], lane), -transpose16(Q[t], lane));
             }
