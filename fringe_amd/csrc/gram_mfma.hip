@@ -909,6 +909,7 @@ static bool gram_staged(int n, int Nx, int Ny, long long rows, int cols, StageTi
         t.waves = std::min(t.waves, stage_waves(blocks));
         const size_t b = gram_lds_bytes(n, Nx, Ny, t);
         if (b > 160 * 1024) continue;
+        if ((long long)((cols + t.TW - 1) / t.TW) * 64 * t.waves >= 1ll << 32) continue;   // threads of a launch's x
         const long long wgs = (long long)((cols + t.TW - 1) / t.TW) * ((rows + t.TH - 1) / t.TH);
         const int fit = (int)std::min<size_t>(160 * 1024 / b, (size_t)std::max(most / t.waves, 1));
         const int active = (int)std::min<long long>(fit, (wgs + 255) / 256), px = t.TH * t.TW;

@@ -93,6 +93,22 @@ inline void set_solve_counts(SolveArgs& a) {
     a.inv_comp = 1.0 / (double)(a.n - a.ref);
 }
 
+// A launch holds less than 2^32 threads, `threads` of them for a slot: launch
+// for parts of a's slots (SolveArgs or GramArgs), whose coherence matrices have
+// elements of `elem` bytes.
+template <typename Args, typename Launch>
+inline void slots_in_parts(const Args& a, int threads, size_t elem, Launch launch) {
+    const long long most = ((1ll << 32) - 1) / threads - 4;   // (the last workgroup may hold three slots more)
+    for (long long s = 0; s < a.slots; s += most) {
+        Args p = a;
+        p.slots = (int)(a.slots - s < most ? a.slots - s : most);
+        p.first += s;
+        p.npix += s;
+        p.gamma = (decltype(p.gamma))((const char*)a.gamma + (size_t)s * a.n * a.n * elem);
+        launch(p);
+    }
+}
+
 // ---- persistent solve launch over a queue of jobs -------------------------
 // A job is one round segment of one tile: slots [0, slots) of its coherence
 // buffer are pixels first + s of that tile.  One launch drains the work

@@ -19,6 +19,8 @@
 // Anderson-Darling statistic in double, bit-identical to the host's, compared
 // with the largest statistic whose interpolated p-value still reaches the
 // threshold (found on the host, so no exp/log runs on the device).
+#include <algorithm>
+
 #include "device_common.hpp"
 #include "engine_internal.hpp"
 #include "timing.hpp"
@@ -128,7 +130,7 @@ __device__ inline int centre_flat(const NmapPlan& P) { return P.Ny * (2 * P.Nx +
 // instructions and 4 CH bytes a pair).  2048 x 2048 pixels of 30 dates, 15 x 11
 // window, against the register merge network it replaced: 16.1 -> 1.5 ms.
 template <int CH>
-__global__ __launch_bounds__(256) void nmap_ks(const NmapPlan P, int row_blocks, uint32_t* __restrict__ F,
+__global__ __launch_bounds__(256) void nmap_ks(const NmapPlan P, int row_blocks, int wg0, uint32_t* __restrict__ F,
                                                int32_t* __restrict__ fcnt) {
     constexpr int PITCH = CH % 8 == 4 ? CH : CH + 4, STRIP = 32;
     __shared__ __align__(16) uint32_t L[(256 + STRIP - 1) * PITCH];
@@ -140,7 +142,7 @@ __global__ __launch_bounds__(256) void nmap_ks(const NmapPlan P, int row_blocks,
     // blocks are dealt to the 8 XCDs round-robin: each takes a contiguous run
     // of rows, whose neighbours' samples stay in its L2
     const unsigned nb = gridDim.x, xcd = blockIdx.x % 8u;
-    const int id = (int)(xcd * (nb / 8u) + min(xcd, nb % 8u) + blockIdx.x / 8u);
+    const int id = wg0 + (int)(xcd * (nb / 8u) + min(xcd, nb % 8u) + blockIdx.x / 8u);
     const int h0 = fwd_row0(P), r = h0 + id / row_blocks, c0 = id % row_blocks * T, c = c0 + tid;
     const bool here = c < cols;
     const long long p = (long long)r * cols + (here ? c : 0);
@@ -252,7 +254,7 @@ static size_t ad2_walk_bytes(int n) {
     return (size_t)ad2_row_offset(n, 2 * n) * 8 + (size_t)((64 + 64 + kWalkStrip - 1) * ((n + 1) | 1) + 4 * 64) * 4;
 }
 
-__global__ __launch_bounds__(256) void nmap_walk(const NmapPlan P, int row_blocks, uint32_t* __restrict__ F,
+__global__ __launch_bounds__(256) void nmap_walk(const NmapPlan P, int row_blocks, int wg0, uint32_t* __restrict__ F,
                                                  int32_t* __restrict__ fcnt) {
     extern __shared__ __align__(16) char smem[];
     const uint32_t* __restrict__ keys = reinterpret_cast<const uint32_t*>(P.d_amp);
@@ -267,7 +269,7 @@ __global__ __launch_bounds__(256) void nmap_walk(const NmapPlan P, int row_block
     const long long npx = (long long)rows * cols;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const unsigned nb = gridDim.x, xcd = blockIdx.x % 8u;   // as nmap_ks
-    const int id = (int)(xcd * (nb / 8u) + min(xcd, nb % 8u) + blockIdx.x / 8u);
+    const int id = wg0 + (int)(xcd * (nb / 8u) + min(xcd, nb % 8u) + blockIdx.x / 8u);
     const int h0 = fwd_row0(P), r = h0 + id / row_blocks, c0 = id % row_blocks * 64, c = c0 + lane;
     const bool here = c < cols;
     const long long p = (long long)r * cols + (here ? c : 0);
@@ -421,11 +423,26 @@ static void launch_prep(const NmapPlan& P, const float2* slc, const uint8_t* mas
     hipLaunchKernelGGL(nmap_prep<NP>, dim3((unsigned)blocks), dim3(threads), 0, s, P, slc, mask);
 }
 
-template <int CH> static void launch_ks(const NmapPlan& P, int fwd_rows, hipStream_t s) {
+// A launch holds less than 2^32 threads: launch(first, count) for parts of
+// `wgs` workgroups.
+template <typename L> static void in_parts(long long wgs, int threads, L launch) {
+    const long long most = ((1ll << 32) - 1) / threads;
+    for (long long w = 0; w < wgs; w += most) launch((int)w, dim3((unsigned)std::min(wgs - w, most)));
+}
+
+template <int CH> static void launch_ks(const NmapPlan& P, long long fwd_rows, hipStream_t s) {
     // the fewest workgroups of at most four waves, of the fewest waves
     const int waves = (P.cols + 63) / 64, blocks = (waves + 3) / 4, per = (waves + blocks - 1) / blocks;
-    hipLaunchKernelGGL(nmap_ks<CH>, dim3((unsigned)blocks * (unsigned)fwd_rows), dim3(64 * per), 0, s, P, blocks, P.d_fwd,
-                       P.d_fcnt);
+    in_parts(fwd_rows * blocks, 64 * per, [&](int wg0, dim3 grid) {
+        hipLaunchKernelGGL(nmap_ks<CH>, grid, dim3(64 * per), 0, s, P, blocks, wg0, P.d_fwd, P.d_fcnt);
+    });
+}
+
+static void launch_walk(const NmapPlan& P, long long fwd_rows, hipStream_t s) {
+    const int blocks = (P.cols + 63) / 64;
+    in_parts(fwd_rows * blocks, 256, [&](int wg0, dim3 grid) {
+        hipLaunchKernelGGL(nmap_walk, grid, dim3(256), ad2_walk_bytes(P.n), s, P, blocks, wg0, P.d_fwd, P.d_fcnt);
+    });
 }
 
 int nmap_launch(const NmapPlan& P, const float2* slc, const uint8_t* mask, uint32_t* wts,
@@ -459,10 +476,9 @@ int nmap_launch(const NmapPlan& P, const float2* slc, const uint8_t* mask, uint3
                 default: launch_ks<32>(P, fr, s); break;
             }
         } else {
-            const int nt = (2 * P.n - 1) * (P.n + 1), blocks = (P.cols + 63) / 64;
+            const int nt = (2 * P.n - 1) * (P.n + 1);
             hipLaunchKernelGGL(ad2_terms, dim3((nt + 255) / 256), dim3(256), 0, s, P.d_ad2, P.n);
-            hipLaunchKernelGGL(nmap_walk, dim3((unsigned)blocks * (unsigned)(P.row_end - h0)), dim3(256),
-                               ad2_walk_bytes(P.n), s, P, blocks, P.d_fwd, P.d_fcnt);
+            launch_walk(P, P.row_end - h0, s);
         }
         hipLaunchKernelGGL(nmap_mirror, dim3((unsigned)((nout + threads - 1) / threads)), dim3(threads), 0, s,
                            P, (const uint32_t*)P.d_fwd, (const int32_t*)P.d_fcnt, wts, count);

@@ -5,25 +5,29 @@
 
 namespace fringe {
 
-template <int DIM> static void launch_wave(const SolveArgs& a, hipStream_t s) {
+template <int DIM> static void launch_wave(const SolveArgs& args, hipStream_t s) {
     constexpr int WPB = 4;
-    const dim3 grid((unsigned)((a.slots + WPB - 1) / WPB)), block(64 * WPB);
-    if (a.module == FRINGE_MODULE_PHASE_LINK)
-        hipLaunchKernelGGL((solve_mfma_kernel<MODE_EMI, DIM, WPB>), grid, block, 0, s, a);
-    else if (a.method == FRINGE_METHOD_MLE)
-        hipLaunchKernelGGL((solve_mfma_kernel<MODE_MLE, DIM, WPB>), grid, block, 0, s, a);
-    else
-        hipLaunchKernelGGL((solve_mfma_kernel<MODE_EVD, DIM, WPB>), grid, block, 0, s, a);
+    slots_in_parts(args, 64, sizeof(cx<float>), [&](const SolveArgs& a) {
+        const dim3 grid((unsigned)((a.slots + WPB - 1) / WPB)), block(64 * WPB);
+        if (a.module == FRINGE_MODULE_PHASE_LINK)
+            hipLaunchKernelGGL((solve_mfma_kernel<MODE_EMI, DIM, WPB>), grid, block, 0, s, a);
+        else if (a.method == FRINGE_METHOD_MLE)
+            hipLaunchKernelGGL((solve_mfma_kernel<MODE_MLE, DIM, WPB>), grid, block, 0, s, a);
+        else
+            hipLaunchKernelGGL((solve_mfma_kernel<MODE_EVD, DIM, WPB>), grid, block, 0, s, a);
+    });
 }
 
-template <int NT> static void launch_wg(const SolveArgs& a, hipStream_t s) {
-    const dim3 grid((unsigned)a.slots), block(64 * NT);
-    if (a.module == FRINGE_MODULE_PHASE_LINK)
-        hipLaunchKernelGGL((solve_mfma_wg_kernel<MODE_EMI, NT>), grid, block, 0, s, a);
-    else if (a.method == FRINGE_METHOD_MLE)
-        hipLaunchKernelGGL((solve_mfma_wg_kernel<MODE_MLE, NT>), grid, block, 0, s, a);
-    else
-        hipLaunchKernelGGL((solve_mfma_wg_kernel<MODE_EVD, NT>), grid, block, 0, s, a);
+template <int NT> static void launch_wg(const SolveArgs& args, hipStream_t s) {
+    slots_in_parts(args, 64 * NT, sizeof(cx<float>), [&](const SolveArgs& a) {
+        const dim3 grid((unsigned)a.slots), block(64 * NT);
+        if (a.module == FRINGE_MODULE_PHASE_LINK)
+            hipLaunchKernelGGL((solve_mfma_wg_kernel<MODE_EMI, NT>), grid, block, 0, s, a);
+        else if (a.method == FRINGE_METHOD_MLE)
+            hipLaunchKernelGGL((solve_mfma_wg_kernel<MODE_MLE, NT>), grid, block, 0, s, a);
+        else
+            hipLaunchKernelGGL((solve_mfma_wg_kernel<MODE_EVD, NT>), grid, block, 0, s, a);
+    });
 }
 
 void launch_solve_mfma(const SolveArgs& args, bool bf16, hipStream_t s) {

@@ -4,14 +4,16 @@
 
 namespace fringe {
 
-template <int NW> static void launch(const SolveArgs& a, hipStream_t s) {
-    const dim3 grid((unsigned)a.slots), block(64 * NW);
-    if (a.module == FRINGE_MODULE_PHASE_LINK)
-        hipLaunchKernelGGL((solve_mfma64_kernel<MODE_EMI, NW>), grid, block, (keep64_bytes<MODE_EMI, NW>()), s, a);
-    else if (a.method == FRINGE_METHOD_MLE)
-        hipLaunchKernelGGL((solve_mfma64_kernel<MODE_MLE, NW>), grid, block, (keep64_bytes<MODE_MLE, NW>()), s, a);
-    else
-        hipLaunchKernelGGL((solve_mfma64_kernel<MODE_EVD, NW>), grid, block, (keep64_bytes<MODE_EVD, NW>()), s, a);
+template <int NW> static void launch(const SolveArgs& args, hipStream_t s) {
+    slots_in_parts(args, 64 * NW, sizeof(cx<double>), [&](const SolveArgs& a) {
+        const dim3 grid((unsigned)a.slots), block(64 * NW);
+        if (a.module == FRINGE_MODULE_PHASE_LINK)
+            hipLaunchKernelGGL((solve_mfma64_kernel<MODE_EMI, NW>), grid, block, (keep64_bytes<MODE_EMI, NW>()), s, a);
+        else if (a.method == FRINGE_METHOD_MLE)
+            hipLaunchKernelGGL((solve_mfma64_kernel<MODE_MLE, NW>), grid, block, (keep64_bytes<MODE_MLE, NW>()), s, a);
+        else
+            hipLaunchKernelGGL((solve_mfma64_kernel<MODE_EVD, NW>), grid, block, (keep64_bytes<MODE_EVD, NW>()), s, a);
+    });
 }
 
 void launch_solve_mfma64(const SolveArgs& args, hipStream_t s) {
@@ -29,8 +31,11 @@ void launch_solve_mfma64(const SolveArgs& args, hipStream_t s) {
     }
 }
 
-template <int NW> static void launch_gram(const GramArgs& a, hipStream_t s) {
-    hipLaunchKernelGGL((gram_mfma64_kernel<NW>), dim3((unsigned)a.slots), dim3(64 * NW), gram_list_bytes(a.Nx, a.Ny), s, a);
+template <int NW> static void launch_gram(const GramArgs& args, hipStream_t s) {
+    slots_in_parts(args, 64 * NW, sizeof(cx<double>), [&](const GramArgs& a) {
+        hipLaunchKernelGGL((gram_mfma64_kernel<NW>), dim3((unsigned)a.slots), dim3(64 * NW), gram_list_bytes(a.Nx, a.Ny), s,
+                           a);
+    });
 }
 
 void launch_gram_mfma64(const GramArgs& a, hipStream_t s) {
