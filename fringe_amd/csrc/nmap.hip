@@ -129,7 +129,12 @@ __device__ inline int centre_flat(const NmapPlan& P) { return P.Ny * (2 * P.Nx +
 // stay in registers.  Bound by the vector unit and the LDS reads (2.5 CH
 // instructions and 4 CH bytes a pair).  2048 x 2048 pixels of 30 dates, 15 x 11
 // window, against the register merge network it replaced: 16.1 -> 1.5 ms.
-template <int CH>
+//
+// Narrow images (NARROW, up to 32 columns) are taken as whole rows, as many as
+// 256 threads hold: with a workgroup a row most lanes idle.  Maps of 30 dates,
+// 15 x 11 window: 40000 x 1 pixels 2.39 -> 0.08 ms, 8000 x 8 0.56 -> 0.11, 5000 x
+// 16 0.39 -> 0.13; from 33 columns on half of the lanes work either way.
+template <int CH, bool NARROW>
 __global__ __launch_bounds__(256) void nmap_ks(const NmapPlan P, int row_blocks, int wg0, uint32_t* __restrict__ F,
                                                int32_t* __restrict__ fcnt) {
     constexpr int PITCH = CH % 8 == 4 ? CH : CH + 4, STRIP = 32;
@@ -143,13 +148,15 @@ __global__ __launch_bounds__(256) void nmap_ks(const NmapPlan P, int row_blocks,
     // of rows, whose neighbours' samples stay in its L2
     const unsigned nb = gridDim.x, xcd = blockIdx.x % 8u;
     const int id = wg0 + (int)(xcd * (nb / 8u) + min(xcd, nb % 8u) + blockIdx.x / 8u);
-    const int h0 = fwd_row0(P), r = h0 + id / row_blocks, c0 = id % row_blocks * T, c = c0 + tid;
-    const bool here = c < cols;
-    const long long p = (long long)r * cols + (here ? c : 0);
+    const int h0 = fwd_row0(P), at = NARROW ? tid / cols : 0;   // row in the workgroup
+    const int r0 = h0 + (NARROW ? id * (T / cols) : id / row_blocks), r = r0 + at;
+    const int c0 = NARROW ? 0 : id % row_blocks * T, c = NARROW ? tid - at * cols : c0 + tid;
+    const bool here = NARROW ? at < T / cols && r < P.row_end : c < cols;
+    const long long p = here ? (long long)r * cols + c : (long long)r0 * cols;
     const bool pv = here && valid[p] != 0;
     const int centre = centre_flat(P), fw = centre >> 5, nf = nul - fw;
     const long long plane = (long long)(P.row_end - h0) * cols;
-    uint32_t* out = F + (long long)(r - h0) * cols + (here ? c : 0);
+    uint32_t* out = F + (p - (long long)h0 * cols);
     uint32_t lo[CH], span[CH];
     auto ranges = [&](int d0) {   // of dates d0 .. d0 + CH - 1; any valid key where there is none
 #pragma unroll
@@ -165,18 +172,19 @@ __global__ __launch_bounds__(256) void nmap_ks(const NmapPlan P, int row_blocks,
     int cnt = 0, word = 0, pos = centre & 31;
     uint64_t cur = 0;
     for (int dy = 0; dy <= Ny; ++dy) {
-        const int rr = r + dy;
         for (int dx0 = dy == 0 ? 0 : -Nx; dx0 <= Nx; dx0 += STRIP) {
             const int w = min(STRIP, Nx - dx0 + 1);
-            uint32_t fail = 0u;
-            if (rr < rows && K >= 0) {   // uniform
+            // positions that some column has (the others are outside the image)
+            const int k0 = NARROW ? max(0, 1 - cols - dx0) : 0, k1 = NARROW ? min(w, cols - dx0) : w;
+            uint32_t fail = NARROW ? ~0u : 0u;
+            if (r0 + dy < rows && K >= 0) {   // uniform
                 for (int d0 = 0; d0 < n; d0 += CH) {
                     const int m = min(CH, n - d0);
                     __syncthreads();   // the last strip's reads are over
-                    for (int e = tid; e < T + w - 1; e += T) {
-                        const int cc = c0 + dx0 + e;
-                        const bool in = cc >= 0 && cc < cols;
-                        const long long q = (long long)rr * cols + (in ? cc : 0);
+                    for (int e = tid; e < (NARROW ? T / cols * cols : T + w - 1); e += T) {
+                        const int er = NARROW ? e / cols : 0, cc = NARROW ? e - er * cols : c0 + dx0 + e, rr = r0 + er + dy;
+                        const bool in = cc >= 0 && cc < cols && (!NARROW || rr < rows);
+                        const long long q = in ? (long long)rr * cols + cc : 0;
                         const bool ok = in && valid[q] != 0;
 #pragma unroll
                         for (int i = 0; i < CH; i += 4) {
@@ -191,16 +199,19 @@ __global__ __launch_bounds__(256) void nmap_ks(const NmapPlan P, int row_blocks,
                     __syncthreads();
                     if (!one) ranges(d0);
 #pragma unroll 2
-                    for (int k = 0; k < w; ++k) {
-                        uint32_t over = 0u;   // what exceeds a range (saturating)
+                    for (int k = k0; k < k1; ++k) {
+                        const bool in = !NARROW || (c + dx0 + k >= 0 && c + dx0 + k < cols);
+                        const int e = NARROW ? (in ? tid + dx0 + k : 0) : tid + k;
+                        uint32_t over = in ? 0u : 1u;   // what exceeds a range (saturating)
 #pragma unroll
                         for (int i = 0; i < CH; i += 4) {
-                            const uint4 b = *(const uint4*)&L[(tid + k) * PITCH + i];
+                            const uint4 b = *(const uint4*)&L[e * PITCH + i];
                             over |= __builtin_elementwise_sub_sat(b.x - lo[i], span[i]);
                             over |= __builtin_elementwise_sub_sat(b.y - lo[i + 1], span[i + 1]);
                             over |= __builtin_elementwise_sub_sat(b.z - lo[i + 2], span[i + 2]);
                             over |= __builtin_elementwise_sub_sat(b.w - lo[i + 3], span[i + 3]);
                         }
+                        if (NARROW && d0 == 0) fail &= ~(1u << k);
                         fail |= (over != 0u ? 1u : 0u) << k;
                     }
                 }
@@ -225,7 +236,7 @@ __global__ __launch_bounds__(256) void nmap_ks(const NmapPlan P, int row_blocks,
             out[word * plane] = (uint32_t)cur;
             cur = 0;
         }
-        fcnt[(long long)(r - h0) * cols + c] = cnt;
+        fcnt[p - (long long)h0 * cols] = cnt;
     }
 }
 
@@ -254,6 +265,9 @@ static size_t ad2_walk_bytes(int n) {
     return (size_t)ad2_row_offset(n, 2 * n) * 8 + (size_t)((64 + 64 + kWalkStrip - 1) * ((n + 1) | 1) + 4 * 64) * 4;
 }
 
+// Narrow images as in nmap_ks: maps of 30 dates, 40000 x 1 pixels 6.87 -> 0.12
+// ms, 8000 x 8 1.56 -> 0.30, 5000 x 16 1.02 -> 0.35.
+template <bool NARROW>
 __global__ __launch_bounds__(256) void nmap_walk(const NmapPlan P, int row_blocks, int wg0, uint32_t* __restrict__ F,
                                                  int32_t* __restrict__ fcnt) {
     extern __shared__ __align__(16) char smem[];
@@ -270,39 +284,42 @@ __global__ __launch_bounds__(256) void nmap_walk(const NmapPlan P, int row_block
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const unsigned nb = gridDim.x, xcd = blockIdx.x % 8u;   // as nmap_ks
     const int id = wg0 + (int)(xcd * (nb / 8u) + min(xcd, nb % 8u) + blockIdx.x / 8u);
-    const int h0 = fwd_row0(P), r = h0 + id / row_blocks, c0 = id % row_blocks * 64, c = c0 + lane;
-    const bool here = c < cols;
-    const long long p = (long long)r * cols + (here ? c : 0);
+    const int h0 = fwd_row0(P), at = NARROW ? lane / cols : 0;   // row in the workgroup
+    const int r0 = h0 + (NARROW ? id * (64 / cols) : id / row_blocks), r = r0 + at;
+    const int c0 = NARROW ? 0 : id % row_blocks * 64, c = NARROW ? lane - at * cols : c0 + lane;
+    const bool here = NARROW ? at < 64 / cols && r < P.row_end : c < cols;
+    const long long p = here ? (long long)r * cols + c : (long long)r0 * cols;
     const bool pv = here && valid[p] != 0;
     const int centre = centre_flat(P), fw = centre >> 5, nf = nul - fw;
     const long long plane = (long long)(P.row_end - h0) * cols;
-    uint32_t* out = F + (long long)(r - h0) * cols + (here ? c : 0);
+    uint32_t* out = F + (p - (long long)h0 * cols);
     for (int j = wave; j < 2 * n - 1; j += 4) {
         const int b = j + 1, at = ad2_row_offset(n, b);
         for (int d = lane; d < ad2_row_terms(n, b); d += 64) T[at + d] = P.d_ad2[j * (n + 1) + (b + 2 * d + (b & 1)) / 2];
     }
-    // keys of 64 or more consecutive pixels of row rr from column `from` on
-    auto stage = [&](uint32_t* dst, int rr, int from, int count) {
+    // keys of 64 or more consecutive pixels of row `row` from column `from` on,
+    // or of the rows from it on
+    auto stage = [&](uint32_t* dst, int row, int from, int count) {
         for (int e = lane; e < count; e += 64) {
-            const int cc = from + e;
-            const bool in = cc >= 0 && cc < cols;
-            const long long q = (long long)rr * cols + (in ? cc : 0);
+            const int er = NARROW ? e / cols : 0, rr = row + er, cc = NARROW ? e - er * cols : from + e;
+            const bool in = cc >= 0 && cc < cols && (!NARROW || (er < 64 / cols && rr < rows));
+            const long long q = in ? (long long)rr * cols + cc : 0;
             const bool ok = in && valid[q] != 0;
             for (int i = wave; i <= n; i += 4) dst[e * pitch + i] = ok && i < n ? keys[(long long)i * npx + q] : ~0u;
         }
     };
-    stage(own, r, c0, 64);
+    stage(own, r0, c0, 64);
     int cnt = 0, word = 0, pos = centre & 31;
     uint64_t cur = 0;
     for (int dy = 0; dy <= Ny; ++dy) {
-        const int rr = r + dy;
         for (int dx0 = dy == 0 ? 0 : -Nx; dx0 <= Nx; dx0 += kWalkStrip) {
             const int w = min(kWalkStrip, Nx - dx0 + 1);
-            if (rr < rows) stage(oth, rr, c0 + dx0, 64 + w - 1);
+            if (r0 + dy < rows) stage(oth, r0 + dy, c0 + dx0, NARROW ? 64 : 64 + w - 1);
             __syncthreads();
             uint32_t bits = 0u;
-            if (rr < rows)
-                for (int k0 = wave; k0 < w; k0 += 8) {
+            if (r0 + dy < rows)
+                // (positions that some column has)
+                for (int k0 = wave + (NARROW ? max(0, 1 - cols - dx0) : 0); k0 < (NARROW ? min(w, cols - dx0) : w); k0 += 8) {
                     const uint32_t *pa[2], *pb[2];
                     uint32_t x[2], y[2];
                     int dd[2] = {0, 0};
@@ -311,11 +328,12 @@ __global__ __launch_bounds__(256) void nmap_walk(const NmapPlan P, int row_block
 #pragma unroll
                     for (int u = 0; u < 2; ++u) {
                         const int k = k0 + 4 * u < w ? k0 + 4 * u : k0;   // (once more where there is no second)
+                        const bool in = !NARROW || (c + dx0 + k >= 0 && c + dx0 + k < cols);
                         pa[u] = own + lane * pitch;
-                        pb[u] = oth + (lane + k) * pitch;
+                        pb[u] = oth + (NARROW ? (in ? lane + dx0 + k : lane) : lane + k) * pitch;
                         x[u] = *pa[u];
                         y[u] = *pb[u];
-                        there[u] = y[u] != ~0u && x[u] != ~0u;
+                        there[u] = in && y[u] != ~0u && x[u] != ~0u;
                         // for a neighbour that is not there, the pixel's run twice (if
                         // that is not there either, words of other runs: not used)
                         if (!there[u]) pb[u] = pa[u], y[u] = x[u];
@@ -361,7 +379,7 @@ __global__ __launch_bounds__(256) void nmap_walk(const NmapPlan P, int row_block
             out[word * plane] = (uint32_t)cur;
             cur = 0;
         }
-        fcnt[(long long)(r - h0) * cols + c] = cnt;
+        fcnt[p - (long long)h0 * cols] = cnt;
     }
 }
 
@@ -423,6 +441,8 @@ static void launch_prep(const NmapPlan& P, const float2* slc, const uint8_t* mas
     hipLaunchKernelGGL(nmap_prep<NP>, dim3((unsigned)blocks), dim3(threads), 0, s, P, slc, mask);
 }
 
+// Images up to kNarrow columns are mapped row after row.
+constexpr int kNarrow = 32;
 // A launch holds less than 2^32 threads: launch(first, count) for parts of
 // `wgs` workgroups.
 template <typename L> static void in_parts(long long wgs, int threads, L launch) {
@@ -431,17 +451,32 @@ template <typename L> static void in_parts(long long wgs, int threads, L launch)
 }
 
 template <int CH> static void launch_ks(const NmapPlan& P, long long fwd_rows, hipStream_t s) {
+    if (P.cols <= kNarrow) {
+        const int per = 256 / P.cols;
+        in_parts((fwd_rows + per - 1) / per, 256, [&](int wg0, dim3 grid) {
+            hipLaunchKernelGGL((nmap_ks<CH, true>), grid, dim3(256), 0, s, P, 1, wg0, P.d_fwd, P.d_fcnt);
+        });
+        return;
+    }
     // the fewest workgroups of at most four waves, of the fewest waves
     const int waves = (P.cols + 63) / 64, blocks = (waves + 3) / 4, per = (waves + blocks - 1) / blocks;
     in_parts(fwd_rows * blocks, 64 * per, [&](int wg0, dim3 grid) {
-        hipLaunchKernelGGL(nmap_ks<CH>, grid, dim3(64 * per), 0, s, P, blocks, wg0, P.d_fwd, P.d_fcnt);
+        hipLaunchKernelGGL((nmap_ks<CH, false>), grid, dim3(64 * per), 0, s, P, blocks, wg0, P.d_fwd, P.d_fcnt);
     });
 }
 
 static void launch_walk(const NmapPlan& P, long long fwd_rows, hipStream_t s) {
+    const size_t lds = ad2_walk_bytes(P.n);
+    if (P.cols <= kNarrow) {
+        const int per = 64 / P.cols;
+        in_parts((fwd_rows + per - 1) / per, 256, [&](int wg0, dim3 grid) {
+            hipLaunchKernelGGL(nmap_walk<true>, grid, dim3(256), lds, s, P, 1, wg0, P.d_fwd, P.d_fcnt);
+        });
+        return;
+    }
     const int blocks = (P.cols + 63) / 64;
     in_parts(fwd_rows * blocks, 256, [&](int wg0, dim3 grid) {
-        hipLaunchKernelGGL(nmap_walk, grid, dim3(256), ad2_walk_bytes(P.n), s, P, blocks, wg0, P.d_fwd, P.d_fcnt);
+        hipLaunchKernelGGL(nmap_walk<false>, grid, dim3(256), lds, s, P, blocks, wg0, P.d_fwd, P.d_fcnt);
     });
 }
 
