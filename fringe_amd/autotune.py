@@ -10,7 +10,8 @@ stage's launches), and keeps the fastest:
   pixel tiles of up to 8 x 16, 4 x 16 or 4 x 8, or the unstaged one.
 * Solver launch, per (date class, estimator, precision): one wave per unit,
   or a persistent grid of W waves per compute unit taking G units at a time
-  from the work queue.
+  from the work queue.  It serves the vector-unit solvers, so no key is tuned
+  where the matrix cores run whatever the schedule (matrix_cores_only).
 * Above 32 dates, per (date class, precision): the matrix in registers,
   on the matrix cores (up to 128 dates), or one row per lane (up to 64
   dates; in FP32 up to 48), or the solver's work matrix in LDS (where it
@@ -33,6 +34,18 @@ if ROOT not in sys.path:
     sys.path.insert(0, ROOT)
 
 MODES = {0: ("phase_link", "MLE"), 1: ("evd", "EVD"), 2: ("evd", "MLE")}
+
+# "staged12" allows the tiles that the default does
+GRAM_CANDIDATES = ("default", "staged8", "staged4", "unstaged")
+SOLVE_CASES = ((48, 0, "mixed"), (48, 1, "mixed"), (96, 0, "mixed"))
+LAYOUT_CASES = ((48, "mixed"), (48, "fp64"), (64, "fp64"), (72, "mixed"), (96, "mixed"), (72, "fp64"), (96, "fp64"),
+                (128, "mixed"), (128, "fp64"))
+
+
+def matrix_cores_only(n, precision):
+    """Whether a link of n dates runs on the matrix cores under every schedule:
+    its candidates are one kernel, and the fastest of them is noise."""
+    return n <= 32 or (precision != "fp64" and 48 < n <= 64)
 
 
 def _time_stage(L, run, stage, reps):
@@ -83,8 +96,8 @@ def tune(quick=False, log=sys.stderr):
         slc, w = data(n, Nx, Ny)
         p = tile.link_params(rows, cols, n, Nx, Ny, min_neighbors=5, precision="mixed")
         times = {}
-        for name, v in _lib.GRAM_VARIANTS.items():
-            L.fringe_schedule_set(_lib.FRINGE_SCHED_GRAM_VARIANT, n, Nx, Ny, v)
+        for name in GRAM_CANDIDATES:
+            L.fringe_schedule_set(_lib.FRINGE_SCHED_GRAM_VARIANT, n, Nx, Ny, _lib.GRAM_VARIANTS[name])
             r = tile.LinkRunner(p, device=dev)
             times[name] = _time_stage(L, lambda: r.run(slc, w), "gram", reps)
             del r
@@ -96,13 +109,9 @@ def tune(quick=False, log=sys.stderr):
     # ---- solver launches ---------------------------------------------------
     cands = [("grid", 0, 0)] + [("persistent", wv, g) for wv in ((8, 16) if quick else (8, 12, 16, 24))
                                 for g in ((1, 4) if quick else (1, 2, 4, 8))]
-    cases = [(30, 0, "mixed"), (30, 0, "fp64"), (20, 2, "mixed"), (30, 1, "mixed"),
-             (48, 0, "mixed"), (64, 1, "mixed"), (96, 0, "mixed")]
-    if quick:
-        cases = cases[:3]
-    for n, mode, prec in cases:
+    for n, mode, prec in SOLVE_CASES[:1] if quick else SOLVE_CASES:
         module, method = MODES[mode]
-        Nx, Ny = (10, 5) if n == 64 else (7, 5)
+        Nx, Ny = 7, 5
         slc, w = data(n, Nx, Ny, fill=None if n <= 64 else 0.9)
         p = tile.link_params(rows if n <= 64 else 16, cols, n, Nx, Ny, module=module, method=method,
                              min_neighbors=5, precision=prec)
@@ -112,8 +121,7 @@ def tune(quick=False, log=sys.stderr):
         # the launch schedule serves the one-row-per-lane solver and the
         # solver with a work matrix, not the matrix cores
         ga_default = L.fringe_schedule_get(_lib.FRINGE_SCHED_GENERIC_A, n, key[2], 0)
-        if n > 32:
-            L.fringe_schedule_set(_lib.FRINGE_SCHED_GENERIC_A, n, key[2], 0, 0)
+        L.fringe_schedule_set(_lib.FRINGE_SCHED_GENERIC_A, n, key[2], 0, 0)
         times = {}
         for launch, wv, g in cands:
             L.fringe_schedule_set(_lib.FRINGE_SCHED_SOLVE, *key, 0 if launch == "grid" else (wv << 8) | g)
@@ -121,8 +129,7 @@ def tune(quick=False, log=sys.stderr):
             times[f"{launch}:{wv}:{g}"] = _time_stage(L, lambda: r.run(slc, w), "solve", reps)
             del r
         L.fringe_schedule_set(_lib.FRINGE_SCHED_SOLVE, *key, 0)
-        if n > 32:
-            L.fringe_schedule_set(_lib.FRINGE_SCHED_GENERIC_A, n, key[2], 0, ga_default)
+        L.fringe_schedule_set(_lib.FRINGE_SCHED_GENERIC_A, n, key[2], 0, ga_default)
         best = min(times, key=times.get)
         launch, wv, g = best.split(":")
         solve.append({"n": n, "mode": mode, "precision": key[2], "estimator": f"{module}/{method}",
@@ -132,8 +139,7 @@ def tune(quick=False, log=sys.stderr):
     # ---- above 32 dates: rows in registers, or one row per lane (up to 64
     # dates), or a work matrix in LDS or global memory (above) --------------
     generic_a = []
-    for n, prec in ((48, "mixed"), (64, "mixed"), (48, "fp64"), (64, "fp64"), (72, "mixed"), (96, "mixed"),
-                    (72, "fp64"), (96, "fp64"), (128, "mixed"), (128, "fp64")):
+    for n, prec in LAYOUT_CASES:
         if quick and n != 96:
             continue
         prow = 16 if n > 64 else 256
