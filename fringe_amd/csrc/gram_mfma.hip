@@ -7,8 +7,9 @@
 //     Re G_ij = P(re_i, re_j) + P(im_i, im_j)
 //     Im G_ij = P(im_i, re_j) - P(re_i, im_j)
 // Each sample is split once into a 16-bit hi + lo pair (hi = h(x), lo =
-// h(x - hi)) and P is accumulated in FP32 by v_mfma_f32_32x32x16_{f16,bf16}
-// over hi*hi + hi*lo + lo*hi.
+// h(x - hi)) and P is accumulated in FP32 over hi*hi + hi*lo + lo*hi, by
+// v_mfma_f32_16x16x32_{f16,bf16} in the staged kernel and by 32x32x16 in the
+// gathering ones.
 //   * fp16 (default): every date is first scaled by an exact power of two so
 //     that its largest |Re|, |Im| over the tile lies in [2^14, 2^15); the pair
 //     then carries ~22 significant bits.  The coherence
@@ -24,12 +25,13 @@
 //               index rows*cols pads neighbour lists.
 //   gram_mfma_lds (up to 64 dates) : the records a pixel tile's windows share
 //               are staged in LDS; one wave per pixel at a time.
-//   gram_mfma : where no tile fits LDS; one wave per pixel at a time.  The wave compacts the mask
-//               into a list of pixel indices (padded to a multiple of 16) in
-//               LDS; per 16 positions lane l gathers component (l % 32) of 8
-//               positions for every 32-wide component block -- lanes 0..31
-//               read one contiguous 128-byte record slice, lanes 32..63
-//               another -- and issues 3 MFMAs per block pair.  The upper
+//   gram_mfma : where no tile fits LDS; one wave per pixel at a time.  The
+//               wave compacts the mask into a list of pixel indices (padded
+//               to a multiple of 16) in LDS; per 16 positions lane l gathers
+//               component (l % 32) of 8 positions for every 32-wide component
+//               block -- lanes 0..31 read one contiguous 128-byte record
+//               slice, lanes 32..63 another -- and issues 3 MFMAs per block
+//               pair.  The upper
 //               block triangle of P is folded into Gamma (the transposed
 //               cross block goes through a per-wave LDS scratch) and written.
 //               Above 32 dates (gram_mfma_pairs) the wave walks the pairs of
@@ -523,12 +525,12 @@ __global__ __launch_bounds__(64 * WAVES) void gram_mfma_pairs(MfmaArgs a) {
 // accumulator each for Re G and Im G, and its mirror is its transpose.
 //
 // Bound by the matrix instructions and the vector unit (operand permutes, list,
-// fold) together, and at 30 dates by Gamma's 8 n^2 bytes per pixel (2.9 TB/s).
+// fold) together, and at 30 dates by Gamma's 8 n^2 bytes per pixel (2.8 TB/s).
 // Measured against 32 x 32 x 16 products of all four real Grams up to 32 dates
-// (2048 x 2048 of 30 dates 14.7 -> 10.3 ms, 640 x 640 of 20 1.40 -> 0.97, 256 x
+// (2048 x 2048 of 30 dates 14.7 -> 10.9 ms, 640 x 640 of 20 1.40 -> 1.03, 256 x
 // 256 of 10 0.18 -> 0.06) and against the gathering kernel above (208 x 224 of
 // 48 dates 0.87 -> 0.24 ms, 131 k pixels of 64 dates in a 21 x 11 window 4.5 ->
-// 2.0).
+// 2.3).
 // Workgroups are numbered so that each XCD (which owns an L2) takes a
 // contiguous run of tiles and the halos neighbouring tiles share stay in it.
 // ---------------------------------------------------------------------------
@@ -891,7 +893,13 @@ static size_t gram_lds_bytes(int n, int Nx, int Ny, const StageTile& t) {
 // one after the other, take twelve each at least; the launch takes as many
 // rounds as it fills the chip.  (64 x 64 pixels of 8
 // dates: 32 tiles of 8 x 16 took 77 us, 512 of 2 x 4 take 12; 160 x 219 of 40:
-// 560 tiles of 4 x 16 in three rounds 219 us, 2200 of 4 x 4 in nine 198.)
+// 560 tiles of 4 x 16 in three rounds 219 us, 2200 of 4 x 4 in nine 198.)  The
+// four constants are fitted to the measured times of about twenty sizes, not
+// derived.  Where they lead, over 6, 12, 16, 24 and 30 dates, windows of 5 x 5
+// to 21 x 11 and 48 x 48 to 1024 x 1024 pixels (120 in all): the median is
+// 0.4 % over the best of this choice, 4 x 16 at most and 4 x 8 at most; the
+// worst 17 %, at a 21 x 11 window up to 16 dates, where 4 x 16 is faster (1024
+// x 1024 of 6: 1.22 and 1.04 ms); next 11 %, 131 x 300 of 12 (41 and 37 us).
 // A scheduled variant (FRINGE_GRAM_STAGED12 / 8 / 4) names the largest tile
 // tried; one that does not fit the window falls back to the others.  False
 // above 64 dates, for windows of more than kStageWords mask words and where
@@ -945,8 +953,9 @@ int pack_launch(const float2* slc, int rows, int cols, int n, bool f16, uint32_t
     if (f16) {
         // one workgroup per date needs no cleared words, and a launch less
         // outweighs its fewer loads in flight: calls back to back of 64 x 64
-        // pixels of 8 dates 38 -> 31 us, 128 x 128 of 30 212 -> 197, 256 x 256
-        // of 10 209.5 -> 208.2
+        // pixels of 8 dates 38 -> 31 us, 128 x 128 of 30 212 -> 197, 140 x 140
+        // of 8 87.6 -> 83.2; at 256 x 256 (of 10, 209.5 and 208.2) the two are
+        // level, so the line lies there
         if (npx <= 65536) {
             hipLaunchKernelGGL(date_absmax<1024>, dim3(1, n), dim3(1024), 0, s, slc, npx, dmax);
         } else {

@@ -55,16 +55,17 @@ struct SolveArgs {
 // Certification of an FP32 eigenpair.  The FP32 chain's backward error is
 // C eps32 |H| for a small C, so the selected unit eigenvector v moves by
 // about C eps32 |H| / gap, and the phase of its smallest component by that
-// over |v_t|.  Against the FP64 oracle, pixels with small gaps and small
-// components showed C between 0.3 and 2.4 (|H| taken as the spectral spread;
-// |T| below bounds it from above).  A result counts as certified when the
-// estimate with C = 5 stays below 5e-4 rad, half the phase tolerance: no
-// eigenvalue of T may lie within 1e4 eps32 |T| / min|v_t| of the selected
-// one.  Decisions against the reference's 1e-6 eigenvalue thresholds are
-// certified 256 eps32 |T| away from them, and the positive definiteness of
-// |Gamma| when no sweep pivot up to the first non-positive one lies within
-// 1e-4 of zero (|Gamma| has unit diagonal, so its pivots lie in (0, 1] when
-// it is definite).
+// over |v_t|.  Against 64 bits, the tridiagonalising solver's C was between
+// 0.3 and 2.4 on pixels with small gaps and small components (|H| taken as
+// the spectral spread; |T| below bounds it from above), 6.0 at most on wider
+// data.  A result counts as certified when no eigenvalue of T lies within 1e4
+// eps32 |T| / min|v_t| of the selected one, which leaves C / 1e4 rad (5e-4,
+// half the phase tolerance, at C = 5).  The matrix-core solvers take
+// cert_eps of solve_mfma.hpp, from their own C.  Decisions against the
+// reference's 1e-6 eigenvalue thresholds are certified 256 eps32 |T| away
+// from them, and the positive definiteness of |Gamma| when no sweep pivot up
+// to the first non-positive one lies within 1e-4 of zero (|Gamma| has unit
+// diagonal, so its pivots lie in (0, 1] when it is definite).
 constexpr float kCertScale = 1.0e4f;
 constexpr float kCertThrMargin = 256.0f;
 constexpr double kCertPivotMin = 1.0e-4;
@@ -113,9 +114,8 @@ inline void slots_in_parts(const Args& a, int threads, size_t elem, Launch launc
 // A job is one round segment of one tile: slots [0, slots) of its coherence
 // buffer are pixels first + s of that tile.  One launch drains the work
 // units of up to kMaxJobs jobs, of different date counts and tiles, from an
-// atomic counter (a unit is one wave's share: two slots for n <= 32, one
-// slot otherwise); units are taken last-first, the matrices the Gram wrote
-// last being the ones still cached.
+// atomic counter (a unit is one slot); units are taken last-first, the
+// matrices the Gram wrote last being the ones still cached.
 constexpr int kMaxJobs = 16;
 struct PJob {
     const void* gamma;

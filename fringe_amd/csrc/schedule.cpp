@@ -1,19 +1,20 @@
 // schedule.cpp -- launch schedules picked by the autotuner
 // (fringe_amd/autotune.py), kept per key in a process-wide table.
 //
-//   Gram variant, keyed by (date class, Nx, Ny): which MFMA Gram kernel and
-//   tile the mixed path launches (the staged kernel on 12 waves with 8 x 16
-//   pixel tiles, on 8 waves with 4 x 16, on 4 waves with at most 4 x 8, or
-//   the unstaged kernel that gathers from L2).
+//   Gram variant, keyed by (date class, Nx, Ny), up to 32 dates: the largest
+//   pixel tile that the staged MFMA kernel of the mixed path tries (8 x 16,
+//   the default's too; 4 x 16; 4 x 8), or the unstaged kernel that gathers
+//   from L2.  A workgroup has up to 16, 12 or 8 waves by its blocks of 16
+//   dates (1, 2, more).  Above 32 dates the default is taken.
 //   Solver launch, keyed by (date class, estimator, precision): a grid with
 //   one wave per unit, or a persistent grid of `waves per CU` x CUs waves
-//   that take `grab` units at a time from a queue.
+//   that take `grab` units at a time from a queue.  The matrix-core solvers
+//   launch as a grid whatever it says.
 //   Solver layout above 32 dates, keyed by (date class 48 / 64 / 96 / 128 /
-//   256, precision): the solver that keeps each row in registers, on the
-//   matrix cores in FP32, four threads per row in FP64 (2, up to 128 dates);
-//   otherwise,
-//   up to 64 dates, the solver with one row per lane (0), and above 64 dates
-//   a work matrix in LDS where it fits (0) or in global memory (1).
+//   256, precision): the matrix cores (2, up to 128 dates, and the default
+//   there; 0 is the same for FP32 at 49..64 dates); otherwise, up to 64
+//   dates, the vector-unit solver with one row per lane (0), and above 64
+//   dates a work matrix in LDS where it fits (0) or in global memory (1).
 //
 // Unset keys use the built-in defaults (the heuristics the table replaces).
 #include <map>

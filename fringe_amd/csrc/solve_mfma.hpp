@@ -28,16 +28,16 @@
 // within the certification distance (cert_eps).
 //
 // What bounds it: the vector unit and the FP32 / FP64 matrix instructions
-// together (their busy cycles add up to the kernel's time; 4, 5 or 6 waves
-// per SIMD measured the same).  At 30 dates a pixel takes 2.34 k vector
+// together (65 and 42 % of the kernel's cycles at 30 dates; 4, 5 or 6 waves
+// per SIMD measured the same).  There a pixel takes 2.55 k vector
 // instructions and 135 MFMAs, against 9.2 k vector instructions in the
 // tridiagonalising two-pixel solver it replaced.  Solve stage of a 2048 x
-// 2048 tile at 30 dates (EMI): 67.5 ms before, 29.5 ms now; of a 640 x 640
-// tile at 20 dates (MLE): 7.4 ms before, 2.9 ms now.
+// 2048 tile at 30 dates (EMI): 67.5 ms before, 31.6 ms now (29.5 without
+// refine32); of a 640 x 640 tile at 20 dates (MLE): 7.4 ms before, 3.1 ms now.
 //
 // Up to 16 dates the same chain runs on one 16 x 16 tile (four registers a
 // matrix instead of sixteen, 16x16x4 MFMAs that take two pivots each): 256 x
-// 256 pixels of 10 dates (EVD) 0.21 -> 0.14 ms, 64 x 64 of 8 0.020 -> 0.015.
+// 256 pixels of 10 dates (EVD) 0.21 -> 0.16 ms, 64 x 64 of 8 0.020 -> 0.017.
 #pragma once
 #include "link_solve.hpp"
 #include "solve32.hpp"
@@ -298,8 +298,8 @@ struct EigState {
 
 // Inverse iteration with B^-1 = I - M: two plain products (the start vector
 // is far off), then normalised steps until the error predicted behind one more
-// (refine32's) is below 4e-7, or until the contraction proves worse than kSlow (moving the shift then
-// costs less than going on).
+// (refine32's) is below 4e-7, or until the contraction proves worse than kSlow
+// (moving the shift then costs less than going on).
 constexpr float kSlow = 0.35f;
 constexpr int kNearInside = 1600000;   // |pivot| >= 0.1
 // qb > 0: polishing instead, until the error predicted from the contraction

@@ -12,9 +12,11 @@
 // Bound by the matrix instructions and the vector unit together (65-95 % of
 // the kernel's cycles; the rest is the latency of a pivot's chain).  Solve
 // stage against the register-row and one-row-per-lane solvers it replaced:
-// 48 dates (208 x 224, EMI) 4.8 -> 2.7 ms, 64 dates (131 k pixels, EVD) 15.1
-// -> 3.6 ms, 96 dates (256 x 256, EMI) 37.4 -> 21.0 ms, with the pixels left
-// to the FP64 re-solve down from 10.9 k, 0 and 38.5 k to 1.1 k, 0 and 14.7 k.
+// 48 dates (208 x 224, EMI) 4.8 -> 2.8 ms, 64 dates (131 k pixels, EVD) 15.1
+// -> 4.1 ms, 96 dates (256 x 256, EMI) 37.4 -> 22.1 ms, with the pixels left
+// to the FP64 re-solve down from 10.9 k, 0 and 38.5 k to 4.4 k, 0 and 23.0 k.
+// (Without refine_wg 2.6, 3.6 and 21.0 ms, and errors of kept pixels beyond
+// the certificate's estimate.)
 #pragma once
 #include "solve_mfma.hpp"
 
@@ -831,9 +833,10 @@ __device__ __forceinline__ void solve_mfma_wg_pixel(const SolveArgs& a, LdsMfmaW
     }
 }
 
-// Waves per SIMD, as many as leave no register spilled (a spill under a
-// partial exec mask has lost the other lanes' values).  Solve stage with one
-// fewer: 64 dates EVD 3.6 -> 4.1 ms, 96 dates EMI 21.0 -> 24.7 ms.
+// Waves per SIMD, as many as leave no vector register spilled (the build
+// fails on one: a value alike in all lanes, stored to scratch with lanes
+// switched off, came back without theirs).  Solve stage with one wave fewer,
+// before refine_wg: 64 dates EVD 3.6 -> 4.1 ms, 96 dates EMI 21.0 -> 24.7 ms.
 constexpr int waves_wg(int mode, int nt) { return nt == 2 ? (mode == MODE_EVD ? 4 : 3) : nt == 3 && mode != MODE_MLE ? 3 : 2; }
 template <int MODE, int NT>
 __global__ __launch_bounds__(64 * NT) __attribute__((amdgpu_waves_per_eu(waves_wg(MODE, NT)))) void solve_mfma_wg_kernel(SolveArgs a) {

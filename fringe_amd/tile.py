@@ -100,8 +100,9 @@ class LinkRunner:
 class BatchRunner:
     """Outputs + workspace for fringe_link_batch_run over a list of
     (slc, wts, params) tiles of different date counts and windows (one
-    module, method and precision); the solves of each date class run in one
-    persistent launch per round."""
+    module, method and precision).  Tiles on the matrix-core solvers, up to
+    128 dates by default, get a grid launch each; the others of a round share
+    one persistent launch per date class."""
 
     def __init__(self, tiles, device="cuda"):
         L = _lib.lib()

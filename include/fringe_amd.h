@@ -158,19 +158,18 @@ int fringe_link_run_noalloc(const fringe_link_tile* t, const void* d_slc, const 
  * diagnostic of the mixed-precision path.  Returns -1 on bad arguments. */
 long long fringe_link_resolved_pixels(const fringe_link_tile* t, const void* d_work, size_t work_bytes);
 
-/* ---- batched tiles: one persistent solve launch over mixed date counts ---
+/* ---- batched tiles of mixed date counts ----------------------------------
  * No counterpart in the reference, whose pixel loops run one stack at a time
  * (evd.cpp:512-514; sequential.py:193-240 links mini-stacks one after the
  * other).  fringe_link_batch_run links `count` independent tiles (their own
  * nbands, window, size, min_neighbors, ref_index, bandwidth; one module,
  * method and precision for the whole batch) on one stream: the coherence
- * matrices of several tiles share each round's buffer, and every round's
- * Hermitian solves of one date class (<= 32, <= 64, <= 128, > 128 dates) run
- * in ONE persistent launch that drains a queue of all tiles' pixels, whatever
- * their date count and neighbour count (tiles on the matrix-core solvers, up
- * to 128 dates by default, get one grid launch each).  Outputs
- * equal fringe_link_run's per tile
- * bit for bit.  Returns 202 for a batch that mixes modules, methods or
+ * matrices of several tiles share each round's buffer.  Tiles on the
+ * matrix-core solvers, which is up to 128 dates by default, get one grid
+ * launch each; a round's other solves of one date class (<= 32, <= 64,
+ * <= 128, > 128 dates) run in one persistent launch that drains a queue of
+ * all tiles' pixels, whatever their date count and neighbour count.  Outputs
+ * equal fringe_link_run's per tile bit for bit.  Returns 202 for a batch that mixes modules, methods or
  * precisions. */
 typedef struct fringe_link_batch_item {
     fringe_link_tile tile;
@@ -187,8 +186,8 @@ int fringe_link_batch_run(const fringe_link_batch_item* items, int count, void* 
 /* ---- launch schedules (set by fringe_amd/autotune.py's table) ------------
  * No counterpart in the reference.  FRINGE_SCHED_GRAM_VARIANT, keyed by
  * (nbands, Nx, Ny) (nbands taken by class: <= 32, <= 64): the mixed path's
- * Gram kernel, FRINGE_GRAM_*; a variant that does not fit the window falls
- * back to the default choice.  FRINGE_SCHED_SOLVE, keyed by (nbands class,
+ * Gram kernel, FRINGE_GRAM_*, up to 32 dates (above, the default is taken); a
+ * variant that does not fit the window falls back to the default choice.  FRINGE_SCHED_SOLVE, keyed by (nbands class,
  * estimator: 0 phase_link EMI, 1 evd EVD/STBAS, 2 evd MLE, precision): 0
  * launches one wave per unit of work, else (waves_per_cu << 8 | grab) runs a
  * persistent grid of waves_per_cu waves per compute unit that take `grab`
@@ -203,7 +202,7 @@ int fringe_link_batch_run(const fringe_link_batch_item* items, int count, void* 
                                        otherwise one row per lane up to 64 dates (0), or its work matrix in LDS
                                        (0) or global memory (1) above 64 dates */
 #define FRINGE_GRAM_DEFAULT 0
-#define FRINGE_GRAM_STAGED12 1      /* pixel tiles of up to 8 x 16 staged in LDS */
+#define FRINGE_GRAM_STAGED12 1      /* pixel tiles of up to 8 x 16 staged in LDS, as the default up to 32 dates */
 #define FRINGE_GRAM_STAGED8 2       /* up to 4 x 16 */
 #define FRINGE_GRAM_STAGED4 3       /* up to 4 x 8 */
 #define FRINGE_GRAM_UNSTAGED 4      /* one wave per pixel, records gathered from L2 */
