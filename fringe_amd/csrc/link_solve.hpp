@@ -47,9 +47,9 @@ struct SolveArgs {
     // (set_solve_counts)
     float inv_n;
     double inv_pairs, inv_comp;
-    // FP32 matrix-core solver: eps times the certification scale for H
-    // (launch_solve_mfma)
-    float cert_h;
+    // FP32 matrix-core solver: eps times the certification scales for H and
+    // for Gamma (launch_solve_mfma)
+    float cert_h, cert_g;
 };
 
 // Certification of an FP32 eigenpair.  The FP32 chain's backward error is

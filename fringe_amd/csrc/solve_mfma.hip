@@ -33,7 +33,9 @@ template <int NT> static void launch_wg(const SolveArgs& args, hipStream_t s) {
 void launch_solve_mfma(const SolveArgs& args, bool bf16, hipStream_t s) {
     SolveArgs a = args;
     set_solve_counts(a);
-    a.cert_h = 5.9604645e-8f * (bf16 ? kCertScale : a.n <= 48 ? kCertScaleH : kCertScaleH * 48.0f / (float)a.n);
+    const float n = (float)a.n;
+    a.cert_h = 5.9604645e-8f * (bf16 ? kCertScale : fminf(kCertScaleH, kCertScaleH * 48.0f / n));
+    a.cert_g = 5.9604645e-8f * (bf16 ? kCertScale : fminf(kCertScale, fmaxf(kCertScaleG, kCertScale * 8.0f / n)));
     if (a.n > 96) launch_wg<4>(a, s);
     else if (a.n > 64) launch_wg<3>(a, s);
     else if (a.n > 32) launch_wg<2>(a, s);

@@ -51,22 +51,33 @@ typedef double mf64x4 __attribute__((ext_vector_type(4)));
 // |v_t| of the selected one, |A| bounded by the eigenvalues' mean and
 // deviation (1.2-1.6 times the norm).  A certified phase is then wrong by C /
 // scale at most, where C, the error times gap min|v| / (eps |A|), was measured
-// against the FP64 path on stacks of 5 to 96 dates and 12 to 130 looks, with
+// against the FP64 path on stacks of 5 to 128 dates and 12 to 130 looks, with
 // coherences that decay to 0, to 0.2, 0.9 and 0.99, noise alone, and two
-// scatterers.  Gamma keeps kCertScale: C is 1.8 at most (the tridiagonalising
-// FP32 solver's: 6.0).  For H below |H| = 100, C is 1.0 up to 8 dates, 0.5 up to
-// 12, 0.3 up to 20, 0.17 at 30, 0.08 at 48 and 0.03 at 96, a third to a seventh
-// of that solver's, so a scale of 3e3, falling as 1 / n from 48 dates on, keeps
-// to its worst error (3.7e-4 rad at 8 dates, 8e-5 at 30, 2e-5 from 48 on).  C
-// grows with the root of |H| beyond (Gamma's own error, multiplied by the
-// inverse of |Gamma|: 0.5 at 16 dates and |H| = 1000), and so does the scale,
-// up to kCertScale.  That holds for Gamma from half pairs (22 bits): bfloat16
-// pairs carry 16, and take kCertScale throughout.  Against kCertScale for H
-// everywhere: 46.6 k pixels of 48 dates 8.0 -> 4.0 ms, 65.5 k of 96 78 -> 53.5.
-constexpr float kCertScaleH = 3.0e3f;
-__device__ __forceinline__ float cert_eps(bool inv, float cert_h, float tn) {
+// scatterers.
+//
+// Gamma: C is 1.8 at 5 dates, 1.25 at 8, 1.13 at 12, 0.8 at 16 and 20, 0.54 at
+// 30, 0.41 at 40, 0.3 at 64 and 0.22 at 96 and more (the tridiagonalising FP32
+// solver's, at 1e4: 2.4 to 6.0).  So kCertScale up to 8 dates falls as 1 / n to
+// kCertScaleG at 32: errors of 2.1e-4 rad at most, and less than that solver's
+// at every n.  kCertScale throughout, with the bound on |A|, left more pixels
+// to FP64 than that solver did (48 k pixels of 128 dates, EVD: 14.8 k, that
+// solver 9.1 k, now 3.1 k; solver and re-solve 40.0 -> 22.3 ms).
+//
+// H below |H| = 100: C is 1.0 up to 8 dates, 0.5 up to 12, 0.3 up to 20, 0.17
+// at 30, 0.08 at 48 and 0.03 at 96, a third to a seventh of that solver's, so a
+// scale of 3e3, falling as 1 / n from 48 dates on, keeps to its worst error
+// (3.7e-4 rad at 8 dates, 8e-5 at 30, 2e-5 from 48 on).  C grows with the root
+// of |H| beyond (Gamma's own error, multiplied by the inverse of |Gamma|: 0.5
+// at 16 dates and |H| = 1000), and so does the scale, up to kCertScale.
+// Against kCertScale for H everywhere: 46.6 k pixels of 48 dates 8.0 -> 4.0
+// ms, 65.5 k of 96 78 -> 53.5.
+//
+// Both hold for Gamma from half pairs (22 bits): bfloat16 pairs carry 16, and
+// take kCertScale throughout.
+constexpr float kCertScaleH = 3.0e3f, kCertScaleG = 2.5e3f;
+__device__ __forceinline__ float cert_eps(bool inv, float cert_h, float cert_g, float tn) {
     const float most = kCertScale * Lim<float>::eps();
-    return inv ? fminf(cert_h * __builtin_amdgcn_sqrtf(fmaxf(0.01f * tn, 1.0f)), most) : most;
+    return inv ? fminf(cert_h * __builtin_amdgcn_sqrtf(fmaxf(0.01f * tn, 1.0f)), most) : cert_g;
 }
 
 // Accumulator of a DIM x DIM matrix: NV registers, lane l holds column l % DIM
@@ -704,7 +715,7 @@ __device__ __forceinline__ void solve_mfma_pixel(const SolveArgs& a, LdsMfma<DIM
                 }
                 // ---- certification ----
                 const float m2 = redC<DIM, OpMin>(in ? cabs2(E.x) : 3.0e38f);
-                delta = cert_eps(inv, a.cert_h, tn) * tn * __builtin_amdgcn_rsqf(uni(m2));
+                delta = cert_eps(inv, a.cert_h, a.cert_g, tn) * tn * __builtin_amdgcn_rsqf(uni(m2));
                 if (!(delta <= tn)) break;
                 // Frobenius norm of the inverse: its other eigenvalues'
                 // squares sum to S2, so none of them exceeds sqrt(S2)

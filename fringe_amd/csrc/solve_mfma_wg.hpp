@@ -649,7 +649,7 @@ __device__ __forceinline__ void solve_mfma_wg_pixel(const SolveArgs& a, LdsMfmaW
                 for (int J = 0; J < NT; ++J)
                     if (32 * J + col < n) m2 = fminf(m2, cabs2(E.x[J]));
                 m2 = scal(red32<OpMin>(m2));
-                delta = scal(cert_eps(inv, a.cert_h, tn) * (tn * __builtin_amdgcn_rsqf(m2)));
+                delta = scal(cert_eps(inv, a.cert_h, a.cert_g, tn) * (tn * __builtin_amdgcn_rsqf(m2)));
                 if (!(delta <= tn)) break;
                 float f = 0.0f;
 #pragma unroll

@@ -75,3 +75,30 @@ def test_kept_pixels_meet_the_estimate(n, Nx, Ny, g0, ginf, est):
     print(f"kept {kept.sum()} of {rows * cols}: max {err.max():.1e}, rms {np.sqrt((err ** 2).mean()):.1e}")
     assert err.max() <= 5.0e-4
     assert np.array_equal(np.minimum(got[1], 0.0), np.minimum(want[1], 0.0))   # the same error codes
+
+
+@pytest.mark.parametrize("n", [64, 96, 128])
+def test_gamma_certificate_lies_at_its_scale(n):
+    """EVD pixels (from 32 dates on: no eigenvalue within 2500 eps |A| /
+    min|v|, |A| bounded by the eigenvalues' mean and deviation) whose 64-bit
+    distance is below 0.8 of that go to FP64, and most of those between 1.25
+    and 3 times it, which a scale of 1e4 refuses to the last one, stay in
+    FP32, within the estimate of 5e-4 rad."""
+    rows, cols, Nx, Ny = 40, 48, 7, 5
+    print(f"case scale n={n}", flush=True)
+    slc = synthetic.stack(n, rows, cols, seed=70 + n, coh=synthetic.coherence_matrix(n, ginf=0.0))
+    ds, w = to_dev(slc, torch), _mask(rows, cols, Nx, Ny)
+    kw = dict(module="evd", method="EVD", min_neighbors=2)
+    want, _ = _link(ds, w, Nx, Ny, "fp64", **kw)
+    got, kept = _link(ds, w, Nx, Ny, "mixed", **kw)
+    lam, v = torch.linalg.eigh(tile.coherence(ds, w, Nx, Ny, precision="fp64")[0].cpu())
+    lam, least = lam.numpy(), v[:, :, -1].abs().amin(1).numpy()
+    bound = 1.0 + np.sqrt(np.maximum((lam ** 2).mean(1) - 1.0, 0.0) * (n - 1))
+    ratio = (lam[:, -1] - lam[:, -2]) * least / (2500 * EPS * bound)
+    beyond = (ratio > 1.25) & (ratio < 3.0)
+    err = np.abs(np.angle(got[0] * want[0].conj())).max(axis=0).reshape(-1)[kept]
+    print(f"{(beyond & kept).sum()} of {beyond.sum()} kept, {kept.sum()} in all: max {err.max():.1e}")
+    assert beyond.sum() > 200
+    assert 2 * (beyond & kept).sum() > beyond.sum()
+    assert not (kept & (ratio < 0.8)).any()
+    assert err.max() <= 5.0e-4
