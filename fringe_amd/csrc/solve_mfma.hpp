@@ -32,7 +32,7 @@
 // per SIMD measured the same).  There a pixel takes 2.55 k vector
 // instructions and 135 MFMAs, against 9.2 k vector instructions in the
 // tridiagonalising two-pixel solver it replaced.  Solve stage of a 2048 x
-// 2048 tile at 30 dates (EMI): 67.5 ms before, 31.6 ms now (29.5 without
+// 2048 tile at 30 dates (EMI): 67.5 ms before, 31.2 ms now (29.5 before
 // refine32); of a 640 x 640 tile at 20 dates (MLE): 7.4 ms before, 3.1 ms now.
 //
 // Up to 16 dates the same chain runs on one 16 x 16 tile (four registers a
@@ -69,8 +69,8 @@ typedef double mf64x4 __attribute__((ext_vector_type(4)));
 // (3.7e-4 rad at 8 dates, 8e-5 at 30, 2e-5 from 48 on).  C grows with the root
 // of |H| beyond (Gamma's own error, multiplied by the inverse of |Gamma|: 0.5
 // at 16 dates and |H| = 1000), and so does the scale, up to kCertScale.
-// Against kCertScale for H everywhere: 46.6 k pixels of 48 dates 8.0 -> 4.0
-// ms, 65.5 k of 96 78 -> 53.5.
+// Against kCertScale for H everywhere: 46.6 k pixels of 48 dates 8.0 -> 3.9
+// ms, 65.5 k of 96 78 -> 54 (51 with Gamma's).
 //
 // Both hold for Gamma from half pairs (22 bits): bfloat16 pairs carry 16, and
 // take kCertScale throughout.

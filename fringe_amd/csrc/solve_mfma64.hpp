@@ -25,8 +25,8 @@
 // publish, barrier, read, pivot inverse.  Solve stage against the vector-unit
 // solvers it replaced: 301 x 409 pixels of 27 dates (EMI) 4.1 -> 2.5 ms; the
 // re-solve with its Gram, a pixel: of 1.1 k pixels of 48 dates 0.74 -> 0.26
-// us (0.19 of 4.4 k), of 14.7 k pixels of 96 dates 2.8 -> 1.24 us (1.20 of
-// 23.0 k).
+// us (0.19 of 4.4 k), of 14.7 k pixels of 96 dates 2.8 -> 1.24 us (1.29 of
+// 19.5 k).
 #pragma once
 #include "gram_mfma64.hpp"
 

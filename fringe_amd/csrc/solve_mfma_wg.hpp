@@ -13,9 +13,9 @@
 // the kernel's cycles; the rest is the latency of a pivot's chain).  Solve
 // stage against the register-row and one-row-per-lane solvers it replaced:
 // 48 dates (208 x 224, EMI) 4.8 -> 2.8 ms, 64 dates (131 k pixels, EVD) 15.1
-// -> 4.1 ms, 96 dates (256 x 256, EMI) 37.4 -> 22.1 ms, with the pixels left
-// to the FP64 re-solve down from 10.9 k, 0 and 38.5 k to 4.4 k, 0 and 23.0 k.
-// (Without refine_wg 2.6, 3.6 and 21.0 ms, and errors of kept pixels beyond
+// -> 3.9 ms, 96 dates (256 x 256, EMI) 37.4 -> 21.1 ms, with the pixels left
+// to the FP64 re-solve down from 10.9 k, 0 and 38.5 k to 4.4 k, 0 and 19.5 k.
+// (Before refine_wg 2.6, 3.6 and 21.0 ms, and errors of kept pixels beyond
 // the certificate's estimate.)
 #pragma once
 #include "solve_mfma.hpp"

@@ -31,7 +31,7 @@ bool matrix_solver_selected(int n, int precision) {
     if (n > kMaxBandsMfma) return false;
     const int pk = precision == FRINGE_PREC_FP64 ? 0 : 1;
     // FP32 at 49..64 dates: 0 is the default's value, and the matrix cores too
-    // (one row per lane took 15.1 ms for 131 k pixels of 64 dates, they 4.1)
+    // (one row per lane took 15.1 ms for 131 k pixels of 64 dates, they 3.9)
     if (pk == 1 && n > 48 && n <= 64) return true;
     return schedule_lookup(FRINGE_SCHED_GENERIC_A, n, pk, 0, generic_a_default(n, pk)) == 2;
 }
